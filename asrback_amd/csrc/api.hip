@@ -63,14 +63,23 @@ int decode_splits(const asrattn_decode_params& p) {
   if (p.num_splits > 0) return p.num_splits;
   // One workgroup per (sequence, kv head) once there are enough of them to
   // spread over the 256 CUs (192 and more: Whisper-small's 16 x 12, Qwen3's
-  // 64 x 8); fewer get their keys split, at least 256 keys per split (128
-  // pairs, Gemma 4's 32 rows x 4 kv heads: two splits measured 7% faster
-  // than one).
+  // 64 x 8); fewer get their keys split over at most one workgroup per CU (a
+  // 257th costs a second round: 96 pairs over 1500 keys 10.0 us with two
+  // splits, 12.5 with three, 11.5 with one).
   const long long pairs = (long long)p.batch * p.heads_kv;
   if (pairs >= 192) return 1;
-  long long s = (256 + pairs - 1) / pairs;
-  const long long by_len = (p.max_len_k + 255) / 256;
+  long long s = 256 / (pairs < 1 ? 1 : pairs);
+  // At least 256 keys of head_dim 64 per split, 128 of 128, and so on (Qwen3's
+  // 1024 slots with 480 in use, 8 pairs: 6.4 us with eight splits, 7.4 with
+  // four; Whisper-tiny's 256-key bucket: 4.4 unsplit, 5.7 with two).
+  const int span = asrattn::decode_span(p);
+  const long long least = 16384 / p.head_dim;
+  const long long by_len = (span + least - 1) / least;
   if (s > by_len) s = by_len;
+  // The fold reads eight splits a round trip: past sixteen splits, longer
+  // ones (1024 keys).
+  const long long most = span / 1024 > 16 ? span / 1024 : 16;
+  if (s > most) s = most;
   if (s > 64) s = 64;
   if (s < 1) s = 1;
   return (int)s;
@@ -94,21 +103,22 @@ int check_decode(const asrattn_decode_params* p) {
   return ASRATTN_OK;
 }
 
-// Workspace layout: partial outputs, then (max, sum) pairs, each section
-// 256-byte aligned.
+// Workspace layout: partial outputs, then (max, sum) pairs and the arrival
+// words behind them, each section 256-byte aligned.
 struct DecodeWorkspace {
-  size_t partials, stats, total;
+  size_t partials, stats, arrive, total;
 };
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 DecodeWorkspace decode_workspace(const asrattn_decode_params& p, int splits) {
-  DecodeWorkspace w{0, 0, 0};
+  DecodeWorkspace w{0, 0, 0, 0};
   if (splits == 1) return w;
   const size_t rows = (size_t)p.batch * p.heads_q * splits;
   w.partials = 0;
   w.stats = align256(rows * (size_t)p.head_dim * sizeof(float));
-  w.total = w.stats + align256(rows * 2 * sizeof(float));
+  w.arrive = w.stats + rows * 2 * sizeof(float);
+  w.total = w.stats + align256(rows * 2 * sizeof(float) + (size_t)p.batch * p.heads_kv * sizeof(unsigned long long));
   return w;
 }
 
@@ -300,6 +310,7 @@ int run_decode(const asrattn_decode_params* params, const asrattn_append_params*
   const DecodeWorkspace w = decode_workspace(p, s);
   float* ws_o = nullptr;
   float* ws_ml = nullptr;
+  unsigned long long* ws_arrive = nullptr;
   if (s > 1) {
     if (workspace == nullptr || workspace_bytes < w.total)
       return fail(ASRATTN_ERR_WORKSPACE, "decode needs %zu workspace bytes, got %zu", w.total,
@@ -309,8 +320,10 @@ int run_decode(const asrattn_decode_params* params, const asrattn_append_params*
     char* base = static_cast<char*>(workspace);
     ws_o = reinterpret_cast<float*>(base + w.partials);
     ws_ml = reinterpret_cast<float*>(base + w.stats);
+    ws_arrive = reinterpret_cast<unsigned long long*>(base + w.arrive);
   }
-  return from_hip(asrattn::launch_decode(p, append, paged, s, ws_o, ws_ml, static_cast<hipStream_t>(stream)), name);
+  return from_hip(
+      asrattn::launch_decode(p, append, paged, s, ws_o, ws_ml, ws_arrive, static_cast<hipStream_t>(stream)), name);
 }
 
 }  // namespace

@@ -132,15 +132,24 @@ __device__ __forceinline__ uint4 buffer_load16_stream(__amdgpu_buffer_rsrc_t rsr
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
+// A load of memory that nothing writes during the launch, at an address
+// uniform over the wave: through the scalar cache, also in kernels whose
+// atomics make the compiler assume otherwise (it then takes vector loads,
+// which wait behind the ones in flight).
+template <typename T>
+__device__ __forceinline__ T load_uniform(const T* p) {
+  return *reinterpret_cast<const __attribute__((address_space(4))) T*>(reinterpret_cast<uintptr_t>(p));
+}
+
 // Keys sequence b uses in a decoder step: seqused_k, else positions + 1,
 // else all of them; clamped to [0, max_len].
 __device__ __forceinline__ int decode_key_count(const int32_t* seqused, const int64_t* positions,
                                                 int b, int max_len) {
   long long n = max_len;
   if (seqused != nullptr) {
-    n = seqused[b];
+    n = load_uniform(seqused + b);
   } else if (positions != nullptr) {
-    n = positions[b] + 1;
+    n = load_uniform(positions + b) + 1;
   }
   if (n > max_len) n = max_len;
   if (n < 0) n = 0;

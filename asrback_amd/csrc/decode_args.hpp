@@ -13,6 +13,11 @@ struct DecodeArgs {
   int page_shift;            // log2(pk.page_size)
   float* ws_o;   // [batch][heads_q][splits][head_dim]
   float* ws_ml;  // [batch][heads_q][splits][2]
+  // Arrival words of the split launch, [batch][heads_kv]: (tag << 16) | the
+  // splits that have arrived, once some split has tagged the word; tag is the
+  // launch's own, never 0, below 2^48.
+  unsigned long long* ws_arrive;
+  unsigned long long tag;
   int splits;
   float c;  // scale * log2(e)
 };

@@ -18,8 +18,8 @@
 //     LDS.
 //     With enough (sequence, kv head) pairs to fill the GPU there is one
 //     split and the workgroup writes the output; otherwise each split writes
-//     an unnormalized partial (o, max, sum) and a small combine kernel folds
-//     them.  No workgroup waits on another.
+//     an unnormalized partial (o, max, sum) and the split that arrives last
+//     folds them.  No workgroup waits on another.
 //   * Sequence lengths are read from device memory (seqused_k or
 //     positions + 1), and splits past a sequence's end write an empty
 //     partial, so the grid depends only on shapes and the launch can be
@@ -44,6 +44,9 @@ namespace asrattn {
 namespace {
 
 
+// s_waitcnt vmcnt(0) (gfx9 encoding; expcnt and lgkmcnt at their maxima).
+constexpr int kWaitVmem = (0x7 << 4) | (0xF << 8);
+
 template <typename T, int HD, int G, int W>
 struct DecodeShape {
   static constexpr int kEPL = Elem<T>::kPerVec;   // elements per lane per load
@@ -65,9 +68,8 @@ struct DecodeShape {
   // Waves per SIMD the register budget allows: four (128 VGPRs) up to four
   // query heads per kv head, two (256) for eight.
   static constexpr int kOcc = G >= 8 ? 2 : 4;
-  // The cross-wave merge stages every wave's (G x HD) partial output in LDS,
-  // and two waves per SIMD allow at most 8 waves per workgroup.
-  static constexpr bool kFits = W * G * HD * 4 <= 65536 && (kOcc == 4 || W <= 8);
+  // The cross-wave merge stages every wave's (G x HD) partial output in LDS.
+  static constexpr bool kFits = W * G * HD * 4 <= 65536;
   static_assert(kLPK >= 1 && kLPK <= 64 && (64 % kLPK) == 0, "head_dim/lane mapping");
 };
 
@@ -133,22 +135,33 @@ __device__ __forceinline__ float round_to(float x) {
   return x;
 }
 
+// The values of lane l ^ (LPK / 2): a row rotation for 16-lane rows, else
+// through the LDS crossbar.
+template <int LPK>
+__device__ __forceinline__ float half_row_partner(float x) {
+  if constexpr (LPK == 16)
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xF, 0xF, false));  // row_ror:8
+  return __shfl_xor(x, LPK / 2, 64);
+}
+
 // Per-head RMSNorm and rotary embedding of one row slice -- lane `sub` of
 // the LPK lanes holding a head_dim row, EPL elements -- in the reference's
 // rounding order (qwen3_asr.py:322-330): the norm x * rsqrt(mean(x^2) +
 // eps) * w in fp32, rounded once; the rotation x c + r s with r = (-x[d/2:],
 // x[:d/2]) rounded after each product and after the sum.  Element e of lane
 // sub pairs with element e of lane sub ^ LPK/2.  w, cs and sn are the
-// lane's slices of the weights and tables (loaded by the caller); has_norm
-// and has_rot are uniform over the grid.  All lanes of the wave must take
-// part.
+// lane's slices of the weights and tables (loaded by the caller).  norm,
+// weighted and rotated say what this row gets (uniform over its lanes);
+// any_norm and any_rot whether any row of the launch does (uniform over the
+// grid).  All lanes of the wave must take part.
 template <typename T, int HD, int LPK>
-__device__ __forceinline__ uint4 norm_rotate(uint4 raw, bool has_norm, const uint4& w, bool has_rot, const uint4& cs,
-                                             const uint4& sn, float eps, int sub) {
+__device__ __forceinline__ uint4 prologue_row(uint4 raw, bool any_norm, bool norm, bool weighted, const uint4& w,
+                                              bool any_rot, bool rotated, const uint4& cs, const uint4& sn, float eps,
+                                              int sub) {
   constexpr int EPL = Elem<T>::kPerVec;
   float x[EPL];
   unpack<T>(raw, x);
-  if (has_norm) {
+  if (any_norm) {
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) ss = fmaf(x[e], x[e], ss);
@@ -157,38 +170,34 @@ __device__ __forceinline__ uint4 norm_rotate(uint4 raw, bool has_norm, const uin
     float wv[EPL];
     unpack<T>(w, wv);
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) x[e] = round_to<T>(x[e] * r * wv[e]);
+    for (int e = 0; e < EPL; ++e) {
+      const float y = round_to<T>(weighted ? x[e] * r * wv[e] : x[e] * r);
+      x[e] = norm ? y : x[e];
+    }
   }
-  if (has_rot) {
+  if (any_rot) {
     float cv[EPL], sv[EPL];
     unpack<T>(cs, cv);
     unpack<T>(sn, sv);
     const bool lower = sub < LPK / 2;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
-      const float partner = __shfl_xor(x[e], LPK / 2, 64);
+      const float partner = half_row_partner<LPK>(x[e]);
       const float rot = lower ? -partner : partner;
-      x[e] = round_to<T>(round_to<T>(x[e] * cv[e]) + round_to<T>(rot * sv[e]));
+      const float y = round_to<T>(round_to<T>(x[e] * cv[e]) + round_to<T>(rot * sv[e]));
+      x[e] = rotated ? y : x[e];
     }
   }
   return pack<T>(x);
 }
 
-// RMS norm without weights (x / sqrt(mean(x^2) + eps), float32 sums,
-// rounded once to T).
-template <typename T, int HD, int LPK>
-__device__ __forceinline__ uint4 rms_unweighted(uint4 raw, float eps) {
-  constexpr int EPL = Elem<T>::kPerVec;
-  float x[EPL];
-  unpack<T>(raw, x);
-  float ss = 0.f;
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) ss = fmaf(x[e], x[e], ss);
-  ss = group_sum<LPK>(ss);
-  const float r = rsqrtf(ss * (1.f / HD) + eps);
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) x[e] = round_to<T>(x[e] * r);
-  return pack<T>(x);
+// Partials pass between workgroups on different XCDs, whose L2 caches are
+// not coherent: agent-scope accesses go through to memory.
+__device__ __forceinline__ void store_shared(float* p, float x) {
+  __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float load_shared(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Online-softmax state of one stream for the G query heads of a kv head.
@@ -303,12 +312,21 @@ struct Stream {
 // At most 128 VGPRs, so that four waves fit per SIMD (two 8-wave workgroups
 // per CU).
 //
-// APPEND: the fused prologue of asrattn_decode_append.  q and the step's key
-// are normalized and rotated in registers; the cache supplies keys
-// 0 .. positions[b] - 1 and the new key/value join from registers (the last
-// split folds them into its state); the first split writes them to the
-// cache at positions[b].  No workgroup reads that slot, so splits need no
-// ordering among themselves.
+// APPEND: the fused prologue of asrattn_decode_append.  The G query rows, the
+// step's key and its value are normalized and rotated once per workgroup, a
+// lane group each, and shared through LDS (done by every lane group for all
+// rows, the prologue's vector instructions took as long as the memory reads
+// of a small batch: see below); the cache supplies keys 0 .. positions[b] - 1
+// and the new key/value join from LDS (the last split folds them into its
+// state); the first split writes them to the cache at positions[b].  No
+// workgroup reads that slot, so splits need no ordering among themselves.
+//
+// Splits: each stores its partial, waits until the stores have reached
+// memory, and adds one to its pair's arrival word; the one that finds all
+// others arrived folds the partials and clears the word.  The word lives in
+// the caller's workspace, which holds anything before the launch: the splits
+// tag it first (a launch's tag is its own), so no clearing pass is needed
+// and a captured launch finds its word cleared or foreign on every replay.
 //
 // SPEC (plain launches with one split, no window, key counts in device
 // memory and a cache of at least eight first batches; paged, a first page
@@ -347,8 +365,14 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
   const int b = blockIdx.z;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
   const int sub = lane % LPK;
   const int stream = wave * S::kKPW + lane / LPK;
+  const bool split_keys = !SPEC && !PB && a.splits > 1;  // both take one split
+  unsigned long long* const arrive = a.ws_arrive + ((int64_t)b * p.heads_kv + hkv);
+  unsigned long long arrive_old = 0;
+  if (split_keys && threadIdx.x == 0)
+    arrive_old = __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   // K and V of this (sequence, kv head).
   const int64_t kbatch = PAGED ? 0 : (int64_t)b * p.k_batch_stride;
@@ -368,7 +392,7 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
   // too; without the scheduling barrier below, the compiler moves the
   // count's load and its wait above those loads.
   Stream<T, HD, G, W> st;
-  {
+  if constexpr (!APPEND) {
     const T* qp = static_cast<const T*>(p.q) + (int64_t)b * p.q_batch_stride +
                   (int64_t)hkv * G * p.q_head_stride + sub * EPL;
 #pragma unroll
@@ -377,28 +401,36 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
   st.c = a.c;
   st.init();
   // The prologue's inputs load here, before the first K/V batch; its
-  // arithmetic runs after that batch is issued.
+  // arithmetic runs after that batch is issued.  Row r of the prologue: query
+  // head r (r < G), the new key (G), the new value (G + 1); lane group
+  // `stream` takes rows stream, stream + NS, ... (past the last: the last).
   const asrattn_append_params& ap = a.ap;
   const bool has_norm = APPEND && ap.q_norm != nullptr;
   const bool has_vnorm = APPEND && ap.v_norm != 0;
   const bool has_rot = APPEND && ap.cos != nullptr;
-  uint4 knew = {}, vnew = {}, qw = {}, kw = {}, cs = {}, sn = {};
+  constexpr int PR = G + 2;
+  constexpr int kRounds = APPEND ? (PR + NS - 1) / NS : 1;
+  __shared__ uint4 sm_rows[APPEND ? PR : 1][APPEND ? LPK : 1];
+  uint4 praw[kRounds], pw[kRounds], pcs = {}, psn = {};
   if constexpr (APPEND) {
     const T* knp = static_cast<const T*>(ap.k_new) + (int64_t)b * ap.kn_batch_stride + (int64_t)hkv * ap.kn_head_stride;
     const T* vnp = static_cast<const T*>(ap.v_new) + (int64_t)b * ap.vn_batch_stride + (int64_t)hkv * ap.vn_head_stride;
+    const T* qp = static_cast<const T*>(p.q) + (int64_t)b * p.q_batch_stride + (int64_t)hkv * G * p.q_head_stride;
     // Absent weights or tables read k_new's slice instead (and are unused):
     // the loads stay unconditional, so no branch joins their registers and
     // forces a wait before the first K/V batch.
-    const T* qwp = has_norm ? static_cast<const T*>(ap.q_norm) : knp;
-    const T* kwp = has_norm ? static_cast<const T*>(ap.k_norm) : knp;
     const T* csp = has_rot ? static_cast<const T*>(ap.cos) + (int64_t)b * ap.rope_batch_stride : knp;
     const T* snp = has_rot ? static_cast<const T*>(ap.sin) + (int64_t)b * ap.rope_batch_stride : knp;
-    knew = *reinterpret_cast<const uint4*>(knp + sub * EPL);
-    vnew = *reinterpret_cast<const uint4*>(vnp + sub * EPL);
-    qw = *reinterpret_cast<const uint4*>(qwp + sub * EPL);
-    kw = *reinterpret_cast<const uint4*>(kwp + sub * EPL);
-    cs = *reinterpret_cast<const uint4*>(csp + sub * EPL);
-    sn = *reinterpret_cast<const uint4*>(snp + sub * EPL);
+#pragma unroll
+    for (int i = 0; i < kRounds; ++i) {
+      const int r = min(stream + i * NS, PR - 1);
+      const T* rp = r < G ? qp + (int64_t)r * p.q_head_stride : r == G ? knp : vnp;
+      const T* wp = !has_norm || r > G ? knp : static_cast<const T*>(r < G ? ap.q_norm : ap.k_norm);
+      praw[i] = *reinterpret_cast<const uint4*>(rp + sub * EPL);
+      pw[i] = *reinterpret_cast<const uint4*>(wp + sub * EPL);
+    }
+    pcs = *reinterpret_cast<const uint4*>(csp + sub * EPL);
+    psn = *reinterpret_cast<const uint4*>(snp + sub * EPL);
   }
 
   // Two register batches in ping-pong: the next batch is in flight while the
@@ -409,7 +441,7 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
   const int32_t* bt = PAGED ? a.pk.block_table + (int64_t)b * a.pk.bt_stride : nullptr;
   auto pool_page = [&](int pi) -> int {
     if (pi >= a.pk.bt_stride) return -1;
-    const int e = bt[__builtin_amdgcn_readfirstlane(pi)];
+    const int e = load_uniform(bt + __builtin_amdgcn_readfirstlane(pi));
     return e >= 0 && e < a.pk.num_pages ? e : -1;
   };
 
@@ -438,7 +470,7 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
     __builtin_amdgcn_sched_barrier(0);  // the batch's issue stays above the count's load
   }
 
-  const int64_t pos = APPEND ? p.positions[b] : 0;
+  const int64_t pos = APPEND ? load_uniform(p.positions + b) : 0;
   const int n = APPEND ? (int)min(max(pos, (int64_t)0), (int64_t)p.max_len_k)
                        : decode_key_count(p.seqused_k, p.positions, b, p.max_len_k);
   // Sliding window: the query sees its last `window` keys (with the append
@@ -516,13 +548,28 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
   } else {
     ma = load(ka, va, k0);
   }
+  // Tag the pair's arrival word, whose load was issued first of all; the
+  // answer is not waited for.
+  if (split_keys && threadIdx.x == 0 && (arrive_old >> 16) != a.tag)
+    __hip_atomic_compare_exchange_strong(arrive, &arrive_old, a.tag << 16, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
   if constexpr (APPEND) {
     __builtin_amdgcn_sched_barrier(0);  // keep the prologue below the batch's issue
 #pragma unroll
-    for (int g = 0; g < G; ++g) st.q[g] = norm_rotate<T, HD, LPK>(st.q[g], has_norm, qw, has_rot, cs, sn, ap.eps, sub);
-    knew = norm_rotate<T, HD, LPK>(knew, has_norm, kw, has_rot, cs, sn, ap.eps, sub);
-    if (has_vnorm) vnew = rms_unweighted<T, HD, LPK>(vnew, ap.eps);
-    st.seed(knew, vnew, split == a.splits - 1 && stream == 0);
+    for (int i = 0; i < kRounds; ++i) {
+      if (uwave * S::kKPW + i * NS < PR) {  // uniform per wave
+        const int r = min(stream + i * NS, PR - 1);
+        sm_rows[r][sub] = prologue_row<T, HD, LPK>(praw[i], has_norm || has_vnorm, r <= G ? has_norm : has_vnorm,
+                                                   r <= G, pw[i], has_rot, r <= G, pcs, psn, ap.eps, sub);
+      }
+    }
+    // An LDS-only barrier: the K/V batch stays in flight across it.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll
+    for (int g = 0; g < G; ++g) st.q[g] = sm_rows[g][sub];
+    if (uwave == 0) st.seed(sm_rows[G][sub], sm_rows[G + 1][sub], split == a.splits - 1 && stream == 0);
   }
   for (int base = k0; base < k1; base += 2 * STEP) {
     mb = load(kb, vb, base + STEP);
@@ -545,8 +592,8 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
         voff = (int64_t)page * a.pk.v_page_stride * (int64_t)sizeof(T) + slot * vts;
       }
       if (write) {
-        *reinterpret_cast<uint4*>(const_cast<char*>(kbase) + koff + lane_bytes) = knew;
-        *reinterpret_cast<uint4*>(const_cast<char*>(vbase) + voff + lane_bytes) = vnew;
+        *reinterpret_cast<uint4*>(const_cast<char*>(kbase) + koff + lane_bytes) = sm_rows[G][sub];
+        *reinterpret_cast<uint4*>(const_cast<char*>(vbase) + voff + lane_bytes) = sm_rows[G + 1][sub];
       }
     }
   }
@@ -585,61 +632,68 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
       osum = fmaf(sm_o[w][g][d], wt, osum);
     }
     const int hq = hkv * G + g;
-    if (a.splits == 1) {
+    if (!split_keys) {
       T* op = static_cast<T*>(p.out) + (int64_t)b * p.o_batch_stride + (int64_t)hq * p.o_head_stride + d;
       Elem<T>::store1(op, lsum > 0.f ? osum / lsum : 0.f);
     } else {
       const int64_t idx = ((int64_t)b * p.heads_q + hq) * a.splits + split;
-      a.ws_o[idx * HD + d] = osum;
+      store_shared(a.ws_o + idx * HD + d, osum);
       if (d == 0) {
-        a.ws_ml[idx * 2] = mx;
-        a.ws_ml[idx * 2 + 1] = lsum;
+        store_shared(a.ws_ml + idx * 2, mx);
+        store_shared(a.ws_ml + idx * 2 + 1, lsum);
       }
     }
   }
-}
+  if (!split_keys) return;
 
-// Folds the splits' partials of one (sequence, query head) into the output.
-template <typename T, int HD>
-__global__ __launch_bounds__(HD) void decode_combine_kernel(const DecodeArgs a) {
-  const asrattn_decode_params& p = a.p;
-  const int hq = blockIdx.x;
-  const int b = blockIdx.y;
-  const int d = threadIdx.x;
-  const int64_t idx0 = ((int64_t)b * p.heads_q + hq) * a.splits;
-  float lsum = 0.f, osum = 0.f;
-  constexpr int kBatch = 8;  // splits whose partials are loaded in one round trip
-  if (a.splits <= kBatch) {
-    float m[kBatch], l[kBatch], o[kBatch];
-#pragma unroll
-    for (int s = 0; s < kBatch; ++s) {
-      const int t = min(s, a.splits - 1);  // surplus slots repeat the last split, weighted 0
-      m[s] = a.ws_ml[(idx0 + t) * 2];
-      l[s] = a.ws_ml[(idx0 + t) * 2 + 1];
-      o[s] = a.ws_o[(idx0 + t) * HD + d];
-    }
-    float mx = kNegInf;
-#pragma unroll
-    for (int s = 0; s < kBatch; ++s) mx = fmaxf(mx, m[s]);
-    const float mxu = mx == kNegInf ? 0.f : mx;
-#pragma unroll
-    for (int s = 0; s < kBatch; ++s) {
-      const float w = s < a.splits ? fast_exp2(m[s] - mxu) : 0.f;
-      lsum = fmaf(l[s], w, lsum);
-      osum = fmaf(o[s], w, osum);
-    }
-  } else {
-    float mx = kNegInf;
-    for (int s = 0; s < a.splits; ++s) mx = fmaxf(mx, a.ws_ml[(idx0 + s) * 2]);
-    const float mxu = mx == kNegInf ? 0.f : mx;
-    for (int s = 0; s < a.splits; ++s) {
-      const float w = fast_exp2(a.ws_ml[(idx0 + s) * 2] - mxu);
-      lsum = fmaf(a.ws_ml[(idx0 + s) * 2 + 1], w, lsum);
-      osum = fmaf(a.ws_o[(idx0 + s) * HD + d], w, osum);
-    }
+  // Arrive once every wave's partial stores are in memory.
+  __builtin_amdgcn_s_waitcnt(kWaitVmem);
+  __shared__ int sm_last;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned long long before =
+        __hip_atomic_fetch_add(arrive, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sm_last = (int)(before & 0xffffull) == a.splits - 1;
+    if (sm_last) __hip_atomic_store(arrive, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  T* op = static_cast<T*>(p.out) + (int64_t)b * p.o_batch_stride + (int64_t)hq * p.o_head_stride + d;
-  Elem<T>::store1(op, lsum > 0.f ? osum / lsum : 0.f);
+  __syncthreads();
+  if (!sm_last) return;  // uniform over the workgroup
+
+  // Fold the splits' partials into the output.
+  for (int t = threadIdx.x; t < G * HD; t += S::kThreads) {
+    const int g = t / HD;
+    const int d = t % HD;
+    const int hq = hkv * G + g;
+    const int64_t idx0 = ((int64_t)b * p.heads_q + hq) * a.splits;
+    float mx = kNegInf, lsum = 0.f, osum = 0.f;
+    constexpr int kBatch = 8;  // splits whose partials are loaded in one round trip
+    for (int s0 = 0; s0 < a.splits; s0 += kBatch) {
+      float m[kBatch], l[kBatch], o[kBatch];
+#pragma unroll
+      for (int s = 0; s < kBatch; ++s) {
+        const int u = min(s0 + s, a.splits - 1);  // surplus slots repeat the last split, weighted 0
+        m[s] = load_shared(a.ws_ml + (idx0 + u) * 2);
+        l[s] = load_shared(a.ws_ml + (idx0 + u) * 2 + 1);
+        o[s] = load_shared(a.ws_o + (idx0 + u) * HD + d);
+      }
+      float mn = mx;
+#pragma unroll
+      for (int s = 0; s < kBatch; ++s) mn = fmaxf(mn, m[s]);
+      const float mu = mn == kNegInf ? 0.f : mn;
+      const float w0 = fast_exp2(mx - mu);
+      mx = mn;
+      lsum *= w0;
+      osum *= w0;
+#pragma unroll
+      for (int s = 0; s < kBatch; ++s) {
+        const float w = s0 + s < a.splits ? fast_exp2(m[s] - mu) : 0.f;
+        lsum = fmaf(l[s], w, lsum);
+        osum = fmaf(o[s], w, osum);
+      }
+    }
+    T* op = static_cast<T*>(p.out) + (int64_t)b * p.o_batch_stride + (int64_t)hq * p.o_head_stride + d;
+    Elem<T>::store1(op, lsum > 0.f ? osum / lsum : 0.f);
+  }
 }
 
 template <typename T, int HD, int G, int W>
@@ -675,18 +729,12 @@ hipError_t launch_typed(const DecodeArgs& a, bool append, hipStream_t stream) {
     hipLaunchKernelGGL((decode_kernel<T, HD, G, W, false, false, true>), grid, dim3(64 * W), 0, stream, a);
   else
     hipLaunchKernelGGL((decode_kernel<T, HD, G, W, false, false>), grid, dim3(64 * W), 0, stream, a);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess || a.splits == 1) return err;
-  hipLaunchKernelGGL((decode_combine_kernel<T, HD>), dim3(p.heads_q, p.batch), dim3(HD), 0, stream, a);
   return hipGetLastError();
 }
 
-// waves: 4, 8 or 16, lowered to what the merge's LDS allows.
+// waves: 4 or 8, lowered to what the merge's LDS allows.
 template <typename T, int HD, int G>
 hipError_t launch_waves(const DecodeArgs& a, int waves, bool append, hipStream_t stream) {
-  if constexpr (DecodeShape<T, HD, G, 16>::kFits) {
-    if (waves >= 16) return launch_typed<T, HD, G, 16>(a, append, stream);
-  }
   if constexpr (DecodeShape<T, HD, G, 8>::kFits) {
     if (waves >= 8) return launch_typed<T, HD, G, 8>(a, append, stream);
   }

@@ -161,7 +161,7 @@ int asrattn_fwd_fsmn(const asrattn_fwd_params* params, const asrattn_fsmn_params
  * One query per sequence over a key/value cache (decoder step).  A
  * workgroup streams the keys of one (sequence, kv head); when the batch has
  * too few of those to fill the GPU, the keys are split over several
- * workgroups (split-K) and a second kernel merges their partials.
+ * workgroups (split-K) and the last of them to finish merges their partials.
  *
  *   out[b, h, :] = softmax_j(scale * q[b, h, :] . k[b, j, h / g, :]) v[b, j, h / g, :]
  *   for n_b - window <= j < n_b (window > 0) or j < n_b (window == 0),
@@ -179,8 +179,9 @@ int asrattn_fwd_fsmn(const asrattn_fwd_params* params, const asrattn_fsmn_params
  *
  * workspace: device memory of asrattn_decode_workspace_size(params) bytes
  * (0 when a single split is used), 256-byte aligned, owned by the caller;
- * it holds the split partials, needs no initialization, must stay valid
- * until the launch completes and must not be shared by concurrent calls.
+ * it holds the split partials and the splits' arrival counts, needs no
+ * initialization, must stay valid until the launch completes and must not be
+ * shared by concurrent calls.
  *
  * Replaces:
  *   F.scaled_dot_product_attention with the (batch, 1, 1, length) position
