@@ -212,6 +212,35 @@ SIGNATURES = {
 }
 
 
+class PromptParams(ctypes.Structure):
+    """``asrlayer_prompt_params`` (csrc/layers.hpp)."""
+
+    _fields_ = [
+        *[(name, _ptr) for name in ("q", "k", "v", "q_out", "k_out", "v_out", "k_cache", "v_cache")],
+        *[(f"{t}_{axis}_stride", _i64) for t in ("q", "k", "v") for axis in ("batch", "token", "head")],
+        *[(f"{t}_{axis}_stride", _i64) for t in ("kc", "vc") for axis in ("row", "pos", "head")],
+        ("cache_rows", _i64),
+        ("cache_length", _i64),
+        ("rows", _ptr),
+        ("positions", _ptr),
+        ("block_table", _ptr),
+        ("bt_stride", _i64),
+        ("page_size", _i32),
+        ("num_pages", _i32),
+        *[(name, _ptr) for name in ("q_norm", "k_norm", "cos", "sin")],
+        ("rope_batch_stride", _i64),
+        ("rope_token_stride", _i64),
+        *[(name, ctypes.c_float) for name in ("q_eps", "k_eps", "v_eps")],
+        *[(name, _i32) for name in ("v_norm", "batch", "tokens", "heads_q", "heads_kv", "head_dim", "dtype")],
+    ]
+
+
+# The layers' own entry points (csrc/layers.hpp).
+LAYER_SIGNATURES = {
+    "asrlayer_prompt_rows": (ctypes.c_int, [ctypes.POINTER(PromptParams), _ptr]),
+}
+
+
 class AttentionError(RuntimeError):
     """A nonzero status from the C ABI; ``status`` is the ``asrattn_status`` code."""
 
@@ -237,7 +266,7 @@ def load() -> ctypes.CDLL:
                     "(there is no fallback path for the attention kernels)"
                 )
             handle = ctypes.CDLL(str(LIBRARY))
-            for name, (restype, argtypes) in SIGNATURES.items():
+            for name, (restype, argtypes) in (SIGNATURES | LAYER_SIGNATURES).items():
                 function = getattr(handle, name)
                 function.restype = restype
                 function.argtypes = argtypes

@@ -455,4 +455,38 @@ int asrattn_decode_paged(const asrattn_decode_params* params, const asrattn_appe
   return run_decode(params, append, paged, workspace, workspace_bytes, stream, "asrattn_decode_paged");
 }
 
+int asrlayer_prompt_rows(const asrlayer_prompt_params* params, void* stream) {
+  if (params == nullptr) return fail(ASRATTN_ERR_INVALID, "params is NULL");
+  const asrlayer_prompt_params& p = *params;
+  if (p.dtype != ASRATTN_F32 && p.dtype != ASRATTN_BF16) return fail(ASRATTN_ERR_INVALID, "dtype %d", p.dtype);
+  if (p.head_dim != 64 && p.head_dim != 128 && p.head_dim != 256 && p.head_dim != 512)
+    return fail(ASRATTN_ERR_UNSUPPORTED, "head_dim %d (supported: 64, 128, 256, 512)", p.head_dim);
+  if (p.batch < 0 || p.tokens < 0 || p.heads_q <= 0 || (p.k != nullptr && p.heads_kv <= 0))
+    return fail(ASRATTN_ERR_INVALID, "batch and tokens must be >= 0, the head counts positive");
+  if (p.batch == 0 || p.tokens == 0) return ok();
+  const long long rows = (long long)p.heads_q + (p.k != nullptr ? 2LL * p.heads_kv : 0LL);
+  const long long tokens = (long long)p.batch * p.tokens;
+  // Rows are counted in 32 bits, up to a workgroup's past the last.
+  if (tokens > 0x7fffffffLL - 1024 || rows > (0x7fffffffLL - 1024) / tokens)
+    return fail(ASRATTN_ERR_UNSUPPORTED, "more than 2^31 rows");
+  if (p.q == nullptr || p.q_out == nullptr || p.q_norm == nullptr || p.cos == nullptr || p.sin == nullptr ||
+      (p.k != nullptr && (p.v == nullptr || p.k_norm == nullptr || p.k_out == nullptr)) ||
+      (p.k_cache == nullptr) != (p.v_cache == nullptr) || (p.k_cache != nullptr && (p.k == nullptr || p.rows == nullptr)))
+    return fail(ASRATTN_ERR_INVALID, "missing tensors");
+  if (p.block_table != nullptr && (p.positions == nullptr || p.page_size <= 0 || p.bt_stride <= 0 || p.num_pages < 0))
+    return fail(ASRATTN_ERR_INVALID, "a block table takes positions, a page size and a pool");
+  if (!vec_aligned(p.q, p.dtype, {p.q_batch_stride, p.q_token_stride, p.q_head_stride}) ||
+      !vec_aligned(p.q_out, p.dtype, {}) || !vec_aligned(p.q_norm, p.dtype, {}) ||
+      !vec_aligned(p.cos, p.dtype, {p.rope_batch_stride, p.rope_token_stride}) || !vec_aligned(p.sin, p.dtype, {}) ||
+      (p.k != nullptr && (!vec_aligned(p.k, p.dtype, {p.k_batch_stride, p.k_token_stride, p.k_head_stride}) ||
+                          !vec_aligned(p.v, p.dtype, {p.v_batch_stride, p.v_token_stride, p.v_head_stride}) ||
+                          !vec_aligned(p.k_out, p.dtype, {}) || !vec_aligned(p.v_out, p.dtype, {}) ||
+                          !vec_aligned(p.k_norm, p.dtype, {}))) ||
+      (p.k_cache != nullptr && (!vec_aligned(p.k_cache, p.dtype, {p.kc_row_stride, p.kc_pos_stride, p.kc_head_stride}) ||
+                                !vec_aligned(p.v_cache, p.dtype, {p.vc_row_stride, p.vc_pos_stride, p.vc_head_stride}))))
+    return fail(ASRATTN_ERR_INVALID, "tensors need 16-byte aligned pointers and strides that are multiples of 16 bytes");
+  return from_hip(asrattn::launch_prompt_rows(p, (uint32_t)(tokens * rows), static_cast<hipStream_t>(stream)),
+                  "asrlayer_prompt_rows");
+}
+
 }  // extern "C"

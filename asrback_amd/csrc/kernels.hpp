@@ -6,6 +6,7 @@
 
 #include "asrattn.h"
 #include "fsmn.hpp"
+#include "layers.hpp"
 
 namespace asrattn {
 
@@ -63,5 +64,9 @@ size_t local_lds_bytes(const asrattn_local_params& p);
 // size at most kFsmnMaxKernel) for the padded layout of p (values p.v, frame
 // counts p.seqused_k).
 hipError_t launch_fsmn(const asrattn_fwd_params& p, const FsmnArgs& f, hipStream_t stream);
+
+// A prompt pass's rows (asrlayer_prompt_rows; head_dim 64, 128, 256 or 512),
+// total = batch * tokens * (heads_q + 2 heads_kv) of them.
+hipError_t launch_prompt_rows(const asrlayer_prompt_params& p, uint32_t total, hipStream_t stream);
 
 }  // namespace asrattn

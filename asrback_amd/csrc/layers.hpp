@@ -1,0 +1,56 @@
+// Entry points of the package's own model layers (asrback_amd/*.py): the
+// element-wise work around the attention calls of asrattn.h.  Not part of
+// the C ABI that replaces the reference's attention ops; the same
+// conventions hold (device pointers, element strides, a stream, no
+// allocation, no synchronization, asrattn_last_error for messages).
+#pragma once
+
+#include <stdint.h>
+
+#include "asrattn.h"
+
+extern "C" {
+
+// The rows a prompt pass prepares for its attention: per-head RMSNorm and
+// rotary embedding of the queries and keys, the values' RMSNorm without
+// weights (v_norm), and the writes of keys and values to the cache.
+//
+//   q' = rot(norm(q, q_norm), cos, sin)     -> q_out
+//   k' = rot(norm(k, k_norm), cos, sin)     -> k_out and the cache
+//   v' = norm(v, 1) (v_norm != 0; else v)   -> v_out (if given) and the cache
+//
+// with asrattn_decode_append's norm and rot, rounded in the element type as
+// the reference's ops round.  Token t of sequence b (batch x tokens of them)
+// is row b * tokens + t of the outputs, which are contiguous.  Its cache slot
+// is (rows[b * tokens + t], positions[b * tokens + t]), or (rows[b], t) with
+// positions NULL; negative indices count from the end, and slots outside the
+// cache are not written.  With a block table (int32, bt_stride entries per
+// cache row) the slot lies in page block_table[row][position / page_size]
+// of the pool, or in the sink page num_pages where that is outside [0,
+// num_pages).  k NULL: queries only.
+typedef struct asrlayer_prompt_params {
+  const void *q, *k, *v;
+  void *q_out, *k_out, *v_out;
+  void *k_cache, *v_cache;
+  int64_t q_batch_stride, q_token_stride, q_head_stride;
+  int64_t k_batch_stride, k_token_stride, k_head_stride;
+  int64_t v_batch_stride, v_token_stride, v_head_stride;
+  // Cache: row (paged: page), position and head strides, and its extent.
+  int64_t kc_row_stride, kc_pos_stride, kc_head_stride;
+  int64_t vc_row_stride, vc_pos_stride, vc_head_stride;
+  int64_t cache_rows, cache_length;
+  const int64_t *rows, *positions;
+  const int32_t* block_table;
+  int64_t bt_stride;
+  int32_t page_size, num_pages;
+  const void *q_norm, *k_norm;  // (head_dim,)
+  const void *cos, *sin;        // (batch, tokens, head_dim) by the strides below
+  int64_t rope_batch_stride, rope_token_stride;
+  float q_eps, k_eps, v_eps;
+  int32_t v_norm;
+  int32_t batch, tokens, heads_q, heads_kv, head_dim, dtype;
+} asrlayer_prompt_params;
+
+int asrlayer_prompt_rows(const asrlayer_prompt_params* params, void* stream);
+
+}  // extern "C"

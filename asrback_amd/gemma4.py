@@ -31,6 +31,7 @@ from torch import Tensor, nn
 
 from . import _lib
 from .attention import KeyPrefix, decode, decode_append, decode_supported, flash, local_attention
+from .layers import prompt_rows, prompt_rows_takes, unhooked
 
 
 class RMSNorm(nn.Module):
@@ -219,13 +220,44 @@ class TextAttention(nn.Module):
         self.o_proj = nn.Linear(self.heads * self.head_dim, width, bias=False)
 
     def _project(self, x: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor | None, Tensor | None]:
-        shape = (*x.shape[:-1], -1, self.head_dim)
         if self.shared:
-            return rotate(self.q_norm(self.q_proj(x).view(shape)), cos, sin), None, None
-        q, k, v = self.qkv_proj(x).split(self.sizes, dim=-1)
+            return self._norm_rotate(self.q_proj(x), cos, sin)
+        return self._norm_rotate(self.qkv_proj(x), cos, sin)
+
+    def _norm_rotate(self, qkv: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor | None, Tensor | None]:
+        """The norms and the rotation of the projections (of the queries alone
+        on shared layers)."""
+        shape = (*qkv.shape[:-1], -1, self.head_dim)
+        if self.shared:
+            return rotate(self.q_norm(qkv.view(shape)), cos, sin), None, None
+        q, k, v = qkv.split(self.sizes, dim=-1)
         q = rotate(self.q_norm(q.reshape(shape)), cos, sin)
         k = rotate(self.k_norm(k.reshape(shape)), cos, sin)
         return q, k, self.v_norm(v.reshape(shape))
+
+    def _prompt_rows(self, x: Tensor, cache: LayerKV, rows: Tensor, cos: Tensor,
+                     sin: Tensor) -> tuple[Tensor, Tensor | None, Tensor | None]:
+        """The prompts' queries, keys and values, keys and values written to
+        the cache (queries alone on shared layers): one kernel on the tensors
+        it takes (:func:`~asrback_amd.layers.prompt_rows`)."""
+        projected = (self.q_proj if self.shared else self.qkv_proj)(x)
+        plain = x.dim() == 3 and type(self.q_norm) is RMSNorm and self.q_norm.weight is not None
+        if plain and self.shared:
+            q = projected.view(*x.shape[:2], -1, self.head_dim)
+            if prompt_rows_takes(q, None, None, None, None, None, None, self.q_norm, None, cos, sin):
+                return prompt_rows(q, None, None, None, None, None, None, self.q_norm, None, cos, sin)
+        elif plain and type(self.k_norm) is RMSNorm and type(self.v_norm) is RMSNorm:
+            q, k, v = (t.unflatten(-1, (-1, self.head_dim)) for t in projected.split(self.sizes, dim=-1))
+            if (self.k_norm.weight is not None and self.v_norm.weight is None and unhooked(self.v_norm)
+                    and prompt_rows_takes(q, k, v, cache.keys, cache.values, rows, None, self.q_norm, self.k_norm, cos,
+                                          sin)):
+                return prompt_rows(q, k, v, cache.keys, cache.values, rows, None, self.q_norm, self.k_norm, cos, sin,
+                                   v_eps=self.v_norm.eps)
+        q, k, v = self._norm_rotate(projected, cos, sin)
+        if not self.shared:
+            cache.keys[rows, : x.shape[1]] = k
+            cache.values[rows, : x.shape[1]] = v
+        return q, k, v
 
     def prefill(self, x: Tensor, cache: LayerKV, rows: Tensor, kv: dict[str, tuple[Tensor, Tensor]],
                 mask: Tensor | KeyPrefix, cos: Tensor, sin: Tensor) -> Tensor:
@@ -233,13 +265,10 @@ class TextAttention(nn.Module):
         attend causally (within the window on sliding layers) and their keys
         and values go to cache ``rows``.  ``mask`` is either the reference's
         prompt mask or a :class:`KeyPrefix` holding each prompt's size."""
-        q, k, v = self._project(x, cos, sin)
+        q, k, v = self._prompt_rows(x, cache, rows, cos, sin)
         if self.shared:
             k, v = kv[self.layer_type]
         else:
-            length = x.shape[1]
-            cache.keys[rows, :length] = k
-            cache.values[rows, :length] = v
             kv[self.layer_type] = k, v
         sizes = mask.lengths if isinstance(mask, KeyPrefix) else _prompt_sizes(mask)
         output = flash(q, k, v, causal=_lib.CAUSAL_TOP_LEFT, seqused_k=sizes, scale=1.0, window=self.window)

@@ -1,0 +1,129 @@
+"""The element-wise work around the attention calls, as kernels of
+``libasrattn.so`` (``csrc/layers.hpp``).
+
+Each function here computes what a sequence of PyTorch ops in the model
+modules computes, in fewer passes over memory, and each has a ``..._takes``
+predicate: the modules call it on the tensors it takes (plain ROCm tensors
+that need no gradient, in the layouts the kernels address) and run the ops
+otherwise.
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import torch
+from torch import Tensor, nn
+
+from . import _lib
+from .attention import _DTYPES, _stream
+
+_VECTOR = 16  # bytes per lane access
+
+
+def _plain(*tensors: Tensor) -> bool:
+    """Whether the kernels may read these tensors in place of PyTorch ops:
+    ordinary ROCm tensors of one supported dtype, on the current device, with
+    nothing (autograd, forward-mode, autocast, functorch, dispatch modes,
+    tracing) that has to see the ops."""
+    first = tensors[0]
+    dtype, device = first.dtype, first.device
+    if dtype not in _DTYPES or device.type != "cuda" or device.index != torch.cuda.current_device():
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) is not Tensor and type(t) is not nn.Parameter:
+            return False
+        if t.dtype != dtype or t.device != device or (grad and t.requires_grad):
+            return False
+        if torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+    return not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack())
+
+
+def _vectors(t: Tensor) -> bool:
+    """Whether rows of ``t`` (its last axis) can be read 16 bytes at a time."""
+    per = _VECTOR // t.element_size()
+    return t.stride(-1) == 1 and t.data_ptr() % _VECTOR == 0 and all(s % per == 0 for s in t.stride()[:-1])
+
+
+def unhooked(*modules: nn.Module) -> bool:
+    return not any(m._forward_hooks or m._forward_pre_hooks for m in modules)
+
+
+def prompt_rows_takes(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache, v_cache, rows: Tensor | None,
+                      positions: Tensor | None, q_norm: nn.Module, k_norm: nn.Module | None, cos: Tensor,
+                      sin: Tensor) -> bool:
+    """Whether :func:`prompt_rows` takes these (see there): rows ``q``
+    ``(batch, tokens, heads, head_dim)``, tables ``(batch, tokens, head_dim)``
+    or ``(tokens, head_dim)``, caches ``(rows, length, heads, head_dim)``."""
+    norms = [q_norm] if k_norm is None else [q_norm, k_norm]
+    tensors = [q, cos, sin, *(m.weight for m in norms)]
+    if k is not None:
+        tensors += [k, v, k_cache, v_cache]
+    if not _plain(*tensors) or not unhooked(*norms):
+        return False
+    head_dim = q.shape[-1]
+    if head_dim not in (64, 128, 256, 512) or any(m.weight.shape != (head_dim,) for m in norms):
+        return False
+    if cos.shape != sin.shape or cos.stride() != sin.stride() or cos.shape[-2:] != (q.shape[1], head_dim):
+        return False
+    if cos.dim() > 3 or (cos.dim() == 3 and cos.shape[0] not in (1, q.shape[0])):
+        return False
+    if k is not None:
+        slots = (q.shape[0] * q.shape[1],) if positions is not None else (q.shape[0],)
+        for index in (rows, positions):
+            if index is None:
+                continue
+            if (type(index) is not Tensor or index.dtype != torch.int64 or index.shape != slots
+                    or index.device != q.device or not index.is_contiguous()):
+                return False
+        if positions is None and q.shape[1] > k_cache.shape[1]:
+            return False
+        if (k.shape != v.shape or k_cache.shape != v_cache.shape or k_cache.dim() != 4
+                or k_cache.shape[2:] != k.shape[2:] or k.shape[-1] != head_dim):
+            return False
+    return all(_vectors(t) for t in tensors)
+
+
+def prompt_rows(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache: Tensor | None, v_cache: Tensor | None,
+                rows: Tensor | None, positions: Tensor | None, q_norm: nn.Module, k_norm: nn.Module | None, cos: Tensor,
+                sin: Tensor, *, block_table: Tensor | None = None, v_eps: float | None = None):
+    """What a prompt pass does to its projections before the attention
+    (``asrlayer_prompt_rows``; ``qwen3_asr.py:366-390``, ``gemma4.py:515-561``):
+    the per-head norms and the rotation of ``q`` and ``k`` ``(batch, tokens,
+    heads, head_dim)``, with ``v_eps`` the weightless norm of ``v``, and the
+    writes of keys and values to the cache at ``(rows, positions)``, int64 per
+    token, or, without ``positions``, at tokens ``0 .. tokens - 1`` of
+    ``rows[b]``.  With ``block_table`` the caches are page pools whose last
+    page takes what no row owns.  Returns contiguous ``q``, ``k`` and ``v``
+    (``v`` itself where it is not normalized); ``k`` None: ``q`` alone."""
+    batch, tokens, heads, head_dim = q.shape
+    q_out = torch.empty((batch, tokens, heads, head_dim), dtype=q.dtype, device=q.device)
+    rope = (cos.stride(0) if cos.dim() == 3 and cos.shape[0] > 1 else 0, cos.stride(-2))
+    common = (q_norm.weight.data_ptr(), None if k is None else k_norm.weight.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+              *rope, q_norm.eps, 0.0 if k is None else k_norm.eps, v_eps or 0.0, v_eps is not None, batch, tokens, heads)
+    if k is None:
+        params = _lib.PromptParams(
+            q.data_ptr(), None, None, q_out.data_ptr(), None, None, None, None, *q.stride()[:3], *(0,) * 12, 0, 0,
+            None, None, None, 0, 0, 0, *common, 0, head_dim, _DTYPES[q.dtype])
+        k_out = v_out = None
+    else:
+        k_out = torch.empty(k.shape, dtype=q.dtype, device=q.device)
+        v_out = v if v_eps is None else torch.empty(v.shape, dtype=q.dtype, device=q.device)
+        if block_table is None:
+            extent = (k_cache.shape[0], k_cache.shape[1])
+            table = (None, 0, 0, 0)
+        else:
+            extent = (block_table.shape[0], 0)
+            table = (block_table.data_ptr(), block_table.shape[1], k_cache.shape[1], k_cache.shape[0] - 1)
+        params = _lib.PromptParams(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), q_out.data_ptr(), k_out.data_ptr(),
+            None if v_eps is None else v_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+            *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *k_cache.stride()[:3], *v_cache.stride()[:3], *extent,
+            rows.data_ptr(), None if positions is None else positions.data_ptr(), *table, *common, k.shape[2], head_dim,
+            _DTYPES[q.dtype])
+    lib = _lib.load()
+    _lib.check(lib.asrlayer_prompt_rows(ctypes.byref(params), _stream(q.device)), "asrlayer_prompt_rows")
+    return q_out, k_out, v_out

@@ -38,6 +38,7 @@ from torch import Tensor, nn
 
 from . import attention
 from .attention import KeyPrefix, PageTable, decode, decode_append, greedy_choice, varlen_attn
+from .layers import prompt_rows, prompt_rows_takes
 from .transcription import CapturedGraph, to_device
 
 # Positions per row of the KV cache (qwen3_asr.py:57-59).
@@ -270,19 +271,43 @@ class TextAttention(nn.Module):
         self.k_norm = RMSNorm(self.head_dim, config["rms_norm_eps"])
 
     def _project(self, x: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, ...]:
-        shape = (len(x), -1, self.head_dim)
-        q, k, v = self.qkv_proj(x).split(self.sizes, dim=-1)
+        return self._norm_rotate(self.qkv_proj(x), cos, sin)
+
+    def _norm_rotate(self, qkv: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, ...]:
+        shape = (len(qkv), -1, self.head_dim)
+        q, k, v = qkv.split(self.sizes, dim=-1)
         q = rotate(self.q_norm(q.reshape(shape)), cos, sin)
         k = rotate(self.k_norm(k.reshape(shape)), cos, sin)
         return q, k, v.reshape(shape)
 
+    def _prompt_rows(self, x, keys, values, rows, positions, cos, sin) -> tuple[Tensor, Tensor, Tensor]:
+        """The prompt's queries, keys and values, keys and values written to
+        the cache."""
+        shape = (1, len(x), -1, self.head_dim)
+        qkv = self.qkv_proj(x)
+        if x.dim() == 2:
+            q, k, v = (t.view(shape) for t in qkv.split(self.sizes, dim=-1))
+            (key_cache, pages), (value_cache, _) = _cache_layer(keys), _cache_layer(values)
+            table = None if pages is None else pages.block_table
+            if ((table is None or (table.is_contiguous() and table.device == x.device))
+                    and type(self.q_norm) is RMSNorm and type(self.k_norm) is RMSNorm
+                    and prompt_rows_takes(q, k, v, key_cache, value_cache, rows, positions, self.q_norm, self.k_norm,
+                                          cos, sin)):
+                q, k, v = prompt_rows(q, k, v, key_cache, value_cache, rows, positions, self.q_norm, self.k_norm, cos,
+                                      sin, block_table=table)
+                return q[0], k[0], v[0]
+        q, k, v = self._norm_rotate(qkv, cos, sin)
+        keys[rows, positions] = k
+        values[rows, positions] = v
+        return q, k, v
+
     def prefill(self, x, keys, values, rows, positions, segments: Segments, cos, sin) -> Tensor:
         """The prompt pass (``:374-390``): keys and values of the packed
         prompts are stored at (row, position) in the cache, then each prompt
-        attends causally within itself."""
-        q, k, v = self._project(x, cos, sin)
-        keys[rows, positions] = k
-        values[rows, positions] = v
+        attends causally within itself.  The norms, the rotation and the
+        cache writes are one kernel on the tensors it takes
+        (:func:`~asrback_amd.layers.prompt_rows`)."""
+        q, k, v = self._prompt_rows(x, keys, values, rows, positions, cos, sin)
         return self.o_proj(attend(q, k, v, segments, causal=True).flatten(1))
 
     def _fused_step(self, x: Tensor, keys: Tensor) -> bool:

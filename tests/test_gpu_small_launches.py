@@ -133,3 +133,114 @@ def test_append_prologue_rows(ops, device, dtype, hd, heads_q, heads_kv, norms, 
             worst = (got.cpu().float() - want.float()).abs() - ulp * want.float().abs()
             # Sums of rotated pairs may cancel: an absolute floor of one unit of the addends.
             assert float(worst.max()) <= ulp * 4.0
+
+
+def assert_ulps(got, want, dtype, scale):
+    """Within one rounding of ``want`` (2^-7 relative in bf16, 1e-6 in fp32)
+    plus one of addends of size ``scale`` (a rotated pair's sum may cancel),
+    and nearly always the same value in bf16."""
+    ulp = 2.0**-7 if dtype == torch.bfloat16 else 1e-6
+    diff = (got.float() - want.float()).abs()
+    assert float((diff - ulp * want.float().abs()).max()) <= ulp * scale
+    if dtype == torch.bfloat16:
+        assert float((diff > 0).float().mean()) < 0.02
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hd,heads,kv_heads,tokens,paged", [
+    (64, 3, 1, 1, False), (128, 16, 8, 37, False), (128, 4, 2, 130, True), (256, 2, 2, 9, False), (512, 2, 1, 5, True)])
+def test_prompt_rows_match_the_ops(device, dtype, hd, heads, kv_heads, tokens, paged, monkeypatch):
+    """Qwen3's prompt pass with its rows prepared by the kernel against the
+    ops it replaces: attention output, and the whole cache (slab, with rows
+    and positions counted from the end; or pages, rows without a page writing
+    to the sink)."""
+    from asrback_amd import qwen3_asr
+
+    say("prompt rows", dtype, hd, heads, kv_heads, tokens, paged)
+    config = {"hidden_size": 128, "head_dim": hd, "num_attention_heads": heads, "num_key_value_heads": kv_heads,
+              "rms_norm_eps": 1e-6, "rope_theta": 1e6, "num_hidden_layers": 1}
+    torch.manual_seed(3)
+    layer = qwen3_asr.TextAttention(config).to(device, dtype)
+    with torch.no_grad():
+        for norm in (layer.q_norm, layer.k_norm):
+            norm.weight.normal_(1.0, 0.2)
+    first = tokens // 2
+    lengths = [n for n in (first, tokens - first) if n]
+    x = randn(tokens, 128, seed=5, dtype=dtype).to(device)
+    slots = [2, 0][: len(lengths)]
+    rows = torch.cat([torch.full((n,), r) for n, r in zip(lengths, slots)]).to(device)
+    positions = torch.cat([torch.arange(n) for n in lengths]).to(device)
+    cos, sin = qwen3_asr.rope_tables(config, 1024, device, dtype)
+    cos, sin = cos[positions], sin[positions]
+    segments = qwen3_asr.Segments.from_lengths(lengths, device)
+    results = []
+    for fused in (True, False):
+        if not fused:
+            monkeypatch.setattr(qwen3_asr, "prompt_rows_takes", lambda *a: False)
+        else:
+            called = []
+            real = qwen3_asr.prompt_rows
+            monkeypatch.setattr(qwen3_asr, "prompt_rows", lambda *a, **k: called.append(1) or real(*a, **k))
+        with torch.inference_mode():
+            if paged:
+                cache = qwen3_asr.PagedKVCache.allocate(config, 3, 40, 16, device, dtype)
+                cache.assign(2, 24)  # a prompt past its row's pages writes to the sink
+                cache.assign(0, 100)
+                keys, values = cache.keys[0], cache.values[0]
+                stored = [cache.pool_keys[0, :-1], cache.pool_values[0, :-1]]
+                where = rows
+            else:
+                stored = [torch.zeros(3, 128, kv_heads, hd, dtype=dtype, device=device) for _ in range(2)]
+                keys, values = stored
+                where = rows - 3  # negative: from the end
+            out = layer.prefill(x, keys, values, where, positions, segments, cos, sin)
+        results.append((out, *stored))
+    assert called
+    (out, keys, values), (out_ref, keys_ref, values_ref) = results
+    assert_ulps(keys, keys_ref, dtype, 4.0)
+    assert torch.equal(values, values_ref) and bool(values.any())
+    # q and k one rounding apart move the bf16 scores by 2^-8 of a few units.
+    assert_close(out, out_ref, "module", 1e-4 if dtype == torch.float32 else 2e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("layer_type", ["sliding_attention", "full_attention"])
+def test_gemma_prompt_rows_match_the_ops(device, dtype, layer_type, monkeypatch):
+    """Gemma 4's padded prompts (value norm, rotation tables shared by the
+    batch, a shared layer's queries alone) through the kernel and the ops."""
+    from asrback_amd import gemma4
+
+    say("gemma prompt rows", dtype, layer_type)
+    text = {"hidden_size": 128, "head_dim": 256, "global_head_dim": 512, "num_attention_heads": 2,
+            "num_key_value_heads": 1, "sliding_window": 512, "rms_norm_eps": 1e-6}
+    torch.manual_seed(4)
+    own, shared = (gemma4.TextAttention(text, layer_type, s).to(device, dtype) for s in (False, True))
+    with torch.no_grad():
+        for norm in (own.q_norm, own.k_norm, shared.q_norm):
+            norm.weight.normal_(0.1, 0.02)
+    length, hd = 19, own.head_dim
+    x = randn(2, length, 128, seed=6, dtype=dtype).to(device)
+    angle = randn(length, hd // 2, seed=7)
+    cos, sin = (torch.cat((f(angle), f(angle)), -1).to(device, dtype) for f in (torch.cos, torch.sin))
+    sizes = gemma4.KeyPrefix(lengths=torch.tensor([19, 11], dtype=torch.int32, device=device))
+    rows = torch.tensor([2, 0], device=device)
+    results = []
+    for fused in (True, False):
+        if not fused:
+            monkeypatch.setattr(gemma4, "prompt_rows_takes", lambda *a: False)
+        else:
+            called = []
+            real = gemma4.prompt_rows
+            monkeypatch.setattr(gemma4, "prompt_rows", lambda *a, **k: called.append(1) or real(*a, **k))
+        with torch.inference_mode():
+            cache = gemma4.LayerKV(*(torch.zeros(3, 40, 1, hd, dtype=dtype, device=device) for _ in range(2)))
+            kv: dict = {}
+            out = own.prefill(x, cache, rows, kv, sizes, cos, sin)
+            out_shared = shared.prefill(x, cache, rows, kv, sizes, cos, sin)
+        results.append((out, out_shared, cache.keys, cache.values))
+    assert len(called) == 2
+    for got, want in zip(results[0][2:], results[1][2:]):
+        assert bool(want.any())
+        assert_ulps(got, want, dtype, 4.0)
+    for got, want in zip(results[0][:2], results[1][:2]):
+        assert_close(got, want, "module", 1e-4 if dtype == torch.float32 else 2e-2)
