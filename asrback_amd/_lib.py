@@ -235,8 +235,31 @@ class PromptParams(ctypes.Structure):
     ]
 
 
+class LinearParams(ctypes.Structure):
+    """``asrlayer_linear_params`` (csrc/layers.hpp)."""
+
+    _fields_ = [
+        ("x", _ptr),
+        ("x_row_stride", _i64),
+        ("ln_weight", _ptr),
+        ("ln_bias", _ptr),
+        ("w", _ptr * 3),
+        ("b", _ptr * 3),
+        ("out", _ptr * 3),
+        ("residual", _ptr),
+        ("r_row_stride", _i64),
+        ("ln_eps", ctypes.c_float),
+        ("n", _i32 * 3),
+        ("rows", _i32),
+        ("k", _i32),
+        ("act", _i32),
+        ("dtype", _i32),
+    ]
+
+
 # The layers' own entry points (csrc/layers.hpp).
 LAYER_SIGNATURES = {
+    "asrlayer_rows_linear": (ctypes.c_int, [ctypes.POINTER(LinearParams), _ptr]),
     "asrlayer_prompt_rows": (ctypes.c_int, [ctypes.POINTER(PromptParams), _ptr]),
 }
 

@@ -489,4 +489,30 @@ int asrlayer_prompt_rows(const asrlayer_prompt_params* params, void* stream) {
                   "asrlayer_prompt_rows");
 }
 
+int asrlayer_rows_linear(const asrlayer_linear_params* params, void* stream) {
+  if (params == nullptr) return fail(ASRATTN_ERR_INVALID, "params is NULL");
+  const asrlayer_linear_params& p = *params;
+  if (p.dtype != ASRATTN_F32 && p.dtype != ASRATTN_BF16) return fail(ASRATTN_ERR_INVALID, "dtype %d", p.dtype);
+  const int per_vec = 16 / elem_bytes(p.dtype);
+  if (p.rows < 1 || p.rows > 16) return fail(ASRATTN_ERR_UNSUPPORTED, "rows must be in [1, 16], got %d", p.rows);
+  if (p.k < per_vec || p.k % per_vec != 0 || p.k / per_vec > 1024)
+    return fail(ASRATTN_ERR_UNSUPPORTED, "k %d is not 1 .. 1024 vectors of %d", p.k, per_vec);
+  long long columns = 0;
+  for (int i = 0; i < 3; ++i) {
+    if (p.n[i] < 0 || (i > 0 && p.n[i] > 0 && p.n[i - 1] == 0))
+      return fail(ASRATTN_ERR_INVALID, "n[%d] is %d", i, p.n[i]);
+    if (p.n[i] > 0 && (p.w[i] == nullptr || p.out[i] == nullptr || !vec_aligned(p.w[i], p.dtype, {})))
+      return fail(ASRATTN_ERR_INVALID, "w[%d] and out[%d] must be non-NULL, w 16-byte aligned", i, i);
+    columns += p.n[i];
+  }
+  if (columns < 1 || columns > 0x7fffffffLL - 64) return fail(ASRATTN_ERR_INVALID, "%lld output columns", columns);
+  if (p.x == nullptr || !vec_aligned(p.x, p.dtype, {p.x_row_stride}) ||
+      (p.ln_weight == nullptr) != (p.ln_bias == nullptr) || !vec_aligned(p.ln_weight, p.dtype, {}) ||
+      !vec_aligned(p.ln_bias, p.dtype, {}))
+    return fail(ASRATTN_ERR_INVALID, "x and the norm's weight and bias need 16-byte aligned pointers and rows");
+  if (p.act < 0 || p.act > 1 || (p.residual != nullptr && (p.n[1] > 0 || p.act != 0)))
+    return fail(ASRATTN_ERR_INVALID, "act must be 0 or 1; a residual takes one matrix and no activation");
+  return from_hip(asrattn::launch_rows_linear(p, static_cast<hipStream_t>(stream)), "asrlayer_rows_linear");
+}
+
 }  // extern "C"

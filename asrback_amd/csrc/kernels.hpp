@@ -69,4 +69,7 @@ hipError_t launch_fsmn(const asrattn_fwd_params& p, const FsmnArgs& f, hipStream
 // total = batch * tokens * (heads_q + 2 heads_kv) of them.
 hipError_t launch_prompt_rows(const asrlayer_prompt_params& p, uint32_t total, hipStream_t stream);
 
+// A decoder step's linear layers over few rows (asrlayer_rows_linear).
+hipError_t launch_rows_linear(const asrlayer_linear_params& p, hipStream_t stream);
+
 }  // namespace asrattn

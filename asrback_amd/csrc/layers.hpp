@@ -53,4 +53,33 @@ typedef struct asrlayer_prompt_params {
 
 int asrlayer_prompt_rows(const asrlayer_prompt_params* params, void* stream);
 
+// Linear layers over the few rows of a decoder step:
+//
+//   out[i] = act(norm(x) w[i]^T + b[i])             (i < 3, n[i] > 0)
+//   out[i] = residual + (norm(x) w[i]^T + b[i])     (residual given)
+//
+// with norm the layer norm over the k inputs (ln_weight NULL: none), sums in
+// float32 and each result rounded in the element type where the separate
+// torch ops round: after the norm, after the product and bias, after the
+// activation, after the residual sum.  x: (rows, k), rows x_row_stride
+// apart; w[i]: (n[i], k), contiguous; b[i]: (n[i]) or NULL; out[i]: (rows,
+// n[i]), contiguous; residual: (rows, n[0]), with one matrix.  act 0: none,
+// 1: gelu (exact).  rows 1 .. 16; k a multiple of 16 bytes and at most 1024
+// times that.
+typedef struct asrlayer_linear_params {
+  const void* x;
+  int64_t x_row_stride;
+  const void *ln_weight, *ln_bias;
+  const void* w[3];
+  const void* b[3];
+  void* out[3];
+  const void* residual;
+  int64_t r_row_stride;
+  float ln_eps;
+  int32_t n[3];
+  int32_t rows, k, act, dtype;
+} asrlayer_linear_params;
+
+int asrlayer_rows_linear(const asrlayer_linear_params* params, void* stream);
+
 }  // extern "C"

@@ -1,0 +1,247 @@
+// A decoder step's linear layers over at most 16 rows (asrlayer_rows_linear):
+// up to three weight matrices over the same rows, with the layer norm before
+// them and the activation or residual sum after them.
+//
+// Bound by launches and latency at the smallest models (float32, width 384,
+// one row: 0.6 MB of weights a matrix), by reading the weights at larger
+// ones.  As separate operations a Whisper decoder layer's step took 27
+// launches of 4-5 us each (norm, bias copy, product, activation and sum apart);
+// here it takes six of 4.2 us (a kernel that does nothing takes 1.8), besides
+// its two attention launches: 429 -> 200 us for a whole step of four layers.
+//
+// A workgroup takes kCols weight rows (output columns) and spreads the
+// reduction over its threads: thread t holds vector t (16 bytes) of every
+// input row and of each weight row, all loaded at once, so a launch is one
+// round trip to memory, two reductions over the workgroup for the layer norm
+// (statistics in two passes, in registers), and one for the products.  The
+// weight rows are read in whole cache lines, once for each eight input rows
+// (four where the reduction takes more than 512 threads, whose registers then
+// hold no more).
+#include "kernels.hpp"
+#include "layers.hpp"
+#include "row_ops.hpp"
+
+namespace asrattn {
+namespace {
+
+constexpr int kMaxWaves = 16;
+
+template <typename T>
+__device__ __forceinline__ float dot_vec(const uint4& a, const uint4& b);
+
+template <>
+__device__ __forceinline__ float dot_vec<float>(const uint4& a, const uint4& b) {
+  float acc = __uint_as_float(a.x) * __uint_as_float(b.x);
+  acc = fmaf(__uint_as_float(a.y), __uint_as_float(b.y), acc);
+  acc = fmaf(__uint_as_float(a.z), __uint_as_float(b.z), acc);
+  return fmaf(__uint_as_float(a.w), __uint_as_float(b.w), acc);
+}
+
+template <>
+__device__ __forceinline__ float dot_vec<bf16_raw>(const uint4& a, const uint4& b) {
+  float x[8], y[8];
+  unpack<bf16_raw>(a, x);
+  unpack<bf16_raw>(b, y);
+  float acc = x[0] * y[0];
+#pragma unroll
+  for (int e = 1; e < 8; ++e) acc = fmaf(x[e], y[e], acc);
+  return acc;
+}
+
+// Sums each of a wave's R values over its lanes (R a power of two up to 16).
+// While values remain, a step adds the partner lanes' values and leaves each
+// lane half as many; the sum of value i ends in the lanes whose bits
+// (5, 4, ...) spell i, value 0 of v.
+template <int R, int OFF>
+__device__ __forceinline__ void sum_lanes(float* v, int lane) {
+  if constexpr (OFF == 0) {
+    return;
+  } else if constexpr (R > 1) {
+#pragma unroll
+    for (int i = 0; i < R / 2; ++i) {
+      const float a = v[i], b = v[i + R / 2];
+      if constexpr (OFF == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      } else if constexpr (OFF == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      } else {
+        const bool upper = (lane & OFF) != 0;
+        v[i] = (upper ? b : a) + __shfl_xor(upper ? a : b, OFF, 64);
+      }
+    }
+    sum_lanes<R / 2, OFF / 2>(v, lane);
+  } else {
+    v[0] += __shfl_xor(v[0], OFF, 64);
+    sum_lanes<1, OFF / 2>(v, lane);
+  }
+}
+
+// The value sum_lanes<R> leaves in `lane`.
+template <int R>
+__device__ __forceinline__ int summed_value(int lane) {
+  constexpr int kBits = R == 1 ? 0 : R == 2 ? 1 : R == 4 ? 2 : R == 8 ? 3 : 4;
+  return lane >> (6 - kBits);
+}
+
+// Sums v[m] over the workgroup; every thread gets all the sums.
+template <int R>
+__device__ __forceinline__ void sum_workgroup(float* v, float (*sm)[R], int waves, int wave, int lane) {
+  float u[R];
+#pragma unroll
+  for (int m = 0; m < R; ++m) u[m] = v[m];
+  sum_lanes<R, 32>(u, lane);
+  if (lane % (64 / R) == 0) sm[wave][summed_value<R>(lane)] = u[0];
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < R; ++m) v[m] = 0.f;
+  for (int w = 0; w < waves; ++w)
+#pragma unroll
+    for (int m = 0; m < R; ++m) v[m] += sm[w][m];
+}
+
+__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
+
+// R: rows of a workgroup, a power of two (rows past the last repeat it).
+template <typename T, int R, int kCols, int kThreads>
+__global__ __launch_bounds__(kThreads) void rows_linear_kernel(const asrlayer_linear_params p) {
+  constexpr int EPL = Elem<T>::kPerVec;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int waves = blockDim.x >> 6;
+  const int vecs = p.k / EPL;
+  const bool mine = tid < vecs;
+  const int at = (mine ? tid : 0) * EPL;
+
+  __shared__ float sm_norm[2][kMaxWaves][R];
+  __shared__ float sm_dot[kMaxWaves][kCols][R];
+
+  // The column's weight row: matrices one after another.
+  const int n01 = p.n[0] + p.n[1], columns = n01 + p.n[2];
+  const int col0 = blockIdx.x * kCols, row0 = blockIdx.y * R;
+  uint4 x[R], w[kCols], lw = {}, lb = {};
+#pragma unroll
+  for (int m = 0; m < R; ++m)
+    x[m] = *reinterpret_cast<const uint4*>(static_cast<const T*>(p.x) + min(row0 + m, p.rows - 1) * p.x_row_stride + at);
+  const bool norm = p.ln_weight != nullptr;
+  if (norm) {
+    lw = *reinterpret_cast<const uint4*>(static_cast<const T*>(p.ln_weight) + at);
+    lb = *reinterpret_cast<const uint4*>(static_cast<const T*>(p.ln_bias) + at);
+  }
+#pragma unroll
+  for (int c = 0; c < kCols; ++c) {
+    const int col = min(col0 + c, columns - 1);
+    const int i = col < p.n[0] ? 0 : col < n01 ? 1 : 2;
+    const int n = col - (i == 0 ? 0 : i == 1 ? p.n[0] : n01);
+    const void* wp = i == 0 ? p.w[0] : i == 1 ? p.w[1] : p.w[2];
+    w[c] = *reinterpret_cast<const uint4*>(static_cast<const T*>(wp) + (int64_t)n * p.k + at);
+  }
+  if (!mine) {
+#pragma unroll
+    for (int m = 0; m < R; ++m) x[m] = make_uint4(0u, 0u, 0u, 0u);
+  }
+
+  if (norm) {
+    // Rounded once to T, as torch's layer_norm does.
+    float mean[R], var[R];
+#pragma unroll
+    for (int m = 0; m < R; ++m) {
+      float f[EPL];
+      unpack<T>(x[m], f);
+      mean[m] = f[0];
+#pragma unroll
+      for (int e = 1; e < EPL; ++e) mean[m] += f[e];
+    }
+    sum_workgroup<R>(mean, sm_norm[0], waves, wave, lane);
+    const float inv_k = 1.f / (float)p.k;
+#pragma unroll
+    for (int m = 0; m < R; ++m) {
+      mean[m] *= inv_k;
+      float f[EPL];
+      unpack<T>(x[m], f);
+      var[m] = 0.f;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        const float d = f[e] - mean[m];
+        var[m] = fmaf(d, d, var[m]);
+      }
+      var[m] = mine ? var[m] : 0.f;
+    }
+    sum_workgroup<R>(var, sm_norm[1], waves, wave, lane);
+    float g[EPL], b[EPL];
+    unpack<T>(lw, g);
+    unpack<T>(lb, b);
+#pragma unroll
+    for (int m = 0; m < R; ++m) {
+      const float r = rsqrtf(var[m] * inv_k + p.ln_eps);
+      float f[EPL];
+      unpack<T>(x[m], f);
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) f[e] = fmaf((f[e] - mean[m]) * r, g[e], b[e]);
+      const uint4 y = pack<T>(f);
+      x[m] = mine ? y : make_uint4(0u, 0u, 0u, 0u);
+    }
+  }
+
+#pragma unroll
+  for (int c = 0; c < kCols; ++c) {
+    float acc[R];
+#pragma unroll
+    for (int m = 0; m < R; ++m) acc[m] = mine ? dot_vec<T>(x[m], w[c]) : 0.f;
+    sum_lanes<R, 32>(acc, lane);
+    if (lane % (64 / R) == 0) sm_dot[wave][c][summed_value<R>(lane)] = acc[0];
+  }
+  __syncthreads();
+
+  if (tid < kCols * R) {
+    const int c = tid % kCols, m = tid / kCols, row = row0 + m;
+    const int col = col0 + c;
+    if (col < columns && row < p.rows) {
+      const int i = col < p.n[0] ? 0 : col < n01 ? 1 : 2;
+      const int n = col - (i == 0 ? 0 : i == 1 ? p.n[0] : n01);
+      const T* bias = static_cast<const T*>(i == 0 ? p.b[0] : i == 1 ? p.b[1] : p.b[2]);
+      T* out = static_cast<T*>(i == 0 ? p.out[0] : i == 1 ? p.out[1] : p.out[2]);
+      float y = 0.f;
+      for (int v = 0; v < waves; ++v) y += sm_dot[v][c][m];
+      if (bias != nullptr) y += Elem<T>::load1(bias + n);
+      // Rounded where the separate operations round.
+      if (p.act == 1) y = gelu(round_to<T>(y));
+      if (p.residual != nullptr)
+        y = round_to<T>(y) + Elem<T>::load1(static_cast<const T*>(p.residual) + row * p.r_row_stride + n);
+      Elem<T>::store1(out + (int64_t)row * p.n[i == 0 ? 0 : i == 1 ? 1 : 2] + n, y);
+    }
+  }
+}
+
+template <typename T, int R, int kThreads>
+hipError_t launch_rows(const asrlayer_linear_params& p, int threads, hipStream_t stream) {
+  const int columns = p.n[0] + p.n[1] + p.n[2];
+  constexpr int kCols = 4;
+  static_assert(kCols * R <= 64, "an output per thread of one wave");
+  hipLaunchKernelGGL((rows_linear_kernel<T, R, kCols, kThreads>), dim3((columns + kCols - 1) / kCols, (p.rows + R - 1) / R),
+                     dim3(threads), 0, stream, p);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_typed(const asrlayer_linear_params& p, hipStream_t stream) {
+  const int threads = (p.k / Elem<T>::kPerVec + 63) / 64 * 64;
+  if (threads > 512) {
+    if (p.rows <= 1) return launch_rows<T, 1, 1024>(p, threads, stream);
+    if (p.rows <= 2) return launch_rows<T, 2, 1024>(p, threads, stream);
+    return launch_rows<T, 4, 1024>(p, threads, stream);
+  }
+  if (p.rows <= 1) return launch_rows<T, 1, 512>(p, threads, stream);
+  if (p.rows <= 2) return launch_rows<T, 2, 512>(p, threads, stream);
+  if (p.rows <= 4) return launch_rows<T, 4, 512>(p, threads, stream);
+  return launch_rows<T, 8, 512>(p, threads, stream);
+}
+
+}  // namespace
+
+hipError_t launch_rows_linear(const asrlayer_linear_params& p, hipStream_t stream) {
+  return p.dtype == ASRATTN_BF16 ? launch_typed<bf16_raw>(p, stream) : launch_typed<float>(p, stream);
+}
+
+}  // namespace asrattn

@@ -127,3 +127,60 @@ def prompt_rows(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache: Tensor |
     lib = _lib.load()
     _lib.check(lib.asrlayer_prompt_rows(ctypes.byref(params), _stream(q.device)), "asrlayer_prompt_rows")
     return q_out, k_out, v_out
+
+
+# Rows a decoder step's linear layers take (csrc/rows_linear.hip).
+LINEAR_ROWS = 16
+
+
+def rows_linear_takes(x: Tensor, linears: list[nn.Module], norms: list[nn.Module], wide: list[nn.Module]) -> bool:
+    """Whether :func:`rows_linear` takes ``x`` ``(rows, 1, inputs)`` through
+    each of ``linears`` and ``norms``, and ``(rows, 1, outputs)`` of the last of
+    ``linears`` through each of ``wide``."""
+    modules = [*linears, *norms, *wide]
+    if any(type(m) is not nn.Linear for m in (*linears, *wide)) or any(type(m) is not nn.LayerNorm for m in norms):
+        return False
+    tensors = [x]
+    for m in modules:
+        tensors += [m.weight] if m.bias is None else [m.weight, m.bias]
+    if any(t is None for t in tensors) or not _plain(*tensors) or not unhooked(*modules):
+        return False
+    if x.dim() != 3 or x.shape[1] != 1 or not 1 <= x.shape[0] <= LINEAR_ROWS or not _vectors(x[:, 0]):
+        return False
+    inputs, per = x.shape[2], _VECTOR // x.element_size()
+    for width, layers in ((inputs, linears), (linears[-1].out_features, wide)):
+        if not layers:
+            continue
+        if width % per or not 0 < width // per <= 1024:
+            return False
+        for m in layers:
+            if m.in_features != width or not m.weight.is_contiguous() or not _vectors(m.weight):
+                return False
+            if m.bias is not None and not m.bias.is_contiguous():
+                return False
+    return all(m.normalized_shape == (inputs,) and m.bias is not None and _vectors(m.weight) and _vectors(m.bias)
+               for m in norms)
+
+
+def rows_linear(x: Tensor, linears: list[nn.Linear], norm: nn.LayerNorm | None = None, *, gelu: bool = False,
+                residual: Tensor | None = None) -> list[Tensor]:
+    """``[linear(norm(x)) for linear in linears]`` for a decoder step's few
+    rows, in one launch (``asrlayer_rows_linear``): up to three matrices, with
+    ``gelu`` (exact) after them or, with one matrix, ``residual`` ``(rows, 1,
+    outputs)`` of unit last stride added to the result."""
+    rows, _, inputs = x.shape
+    outs = [torch.empty((rows, 1, m.out_features), dtype=x.dtype, device=x.device) for m in linears]
+    params = _lib.LinearParams()
+    params.x, params.x_row_stride = x.data_ptr(), x.stride(0)
+    if norm is not None:
+        params.ln_weight, params.ln_bias, params.ln_eps = norm.weight.data_ptr(), norm.bias.data_ptr(), norm.eps
+    for i, (m, out) in enumerate(zip(linears, outs)):
+        params.w[i], params.out[i], params.n[i] = m.weight.data_ptr(), out.data_ptr(), m.out_features
+        if m.bias is not None:
+            params.b[i] = m.bias.data_ptr()
+    if residual is not None:
+        params.residual, params.r_row_stride = residual.data_ptr(), residual.stride(0)
+    params.rows, params.k, params.act, params.dtype = rows, inputs, int(gelu), _DTYPES[x.dtype]
+    lib = _lib.load()
+    _lib.check(lib.asrlayer_rows_linear(ctypes.byref(params), _stream(x.device)), "asrlayer_rows_linear")
+    return outs

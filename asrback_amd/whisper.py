@@ -32,6 +32,7 @@ from torch import Tensor, nn
 
 from . import attention
 from .attention import KeyPrefix, decode_append, greedy_choice, sdpa
+from .layers import rows_linear, rows_linear_takes
 from .transcription import CapturedGraph, to_device
 
 # Key buckets of the graphed decoder step; max_target_positions is the last
@@ -191,6 +192,35 @@ class DecoderLayer(nn.Module):
         self.fc2 = nn.Linear(config["decoder_ffn_dim"], width)
         self.final_layer_norm = nn.LayerNorm(width)
 
+    def _rows_take(self, x: Tensor) -> bool:
+        """Whether every linear layer of a step on ``x`` runs as
+        :func:`~asrback_amd.layers.rows_linear` (the inputs of all but the
+        first are new contiguous tensors of ``x``'s kind)."""
+        own, cross = self.self_attn, self.encoder_attn
+        return (
+            type(own) is MultiHeadAttention and type(cross) is MultiHeadAttention
+            and rows_linear_takes(x, [own.k_proj, own.v_proj, own.q_proj, own.out_proj, cross.q_proj, cross.out_proj,
+                                      self.fc1],
+                                  [self.self_attn_layer_norm, self.encoder_attn_layer_norm, self.final_layer_norm],
+                                  [self.fc2])
+        )
+
+    def _row_step(self, x: Tensor, cache: tuple[Tensor, Tensor, Tensor, Tensor], positions: Tensor) -> Tensor:
+        """The step with its linear layers, norms, activation and residual sums
+        as six launches beside the two attention launches."""
+        self_keys, self_values, cross_keys, cross_values = cache
+        own, cross = self.self_attn, self.encoder_attn
+        heads = (x.shape[0], own.heads, -1)
+        key, value, query = rows_linear(x, [own.k_proj, own.v_proj, own.q_proj], self.self_attn_layer_norm)
+        output = decode_append(query.view(heads), key.view(heads), value.view(heads), self_keys.transpose(1, 2),
+                               self_values.transpose(1, 2), positions)
+        (x,) = rows_linear(output.view(x.shape), [own.out_proj], residual=x)
+        (query,) = rows_linear(x, [cross.q_proj], self.encoder_attn_layer_norm)
+        output = sdpa(cross._split_heads(query), cross_keys, cross_values)
+        (x,) = rows_linear(output.view(x.shape), [cross.out_proj], residual=x)
+        (hidden,) = rows_linear(x, [self.fc1], self.final_layer_norm, gelu=True)
+        return rows_linear(hidden, [self.fc2], residual=x)[0]
+
     def forward(
         self,
         x: Tensor,
@@ -200,6 +230,9 @@ class DecoderLayer(nn.Module):
         mask: KeyPrefix | Tensor | None,
     ) -> Tensor:
         self_keys, self_values, cross_keys, cross_values = cache
+        if (self.fused_step and length is None and isinstance(mask, KeyPrefix) and mask.positions is positions
+                and self._rows_take(x)):
+            return self._row_step(x, cache, positions)
         hidden = self.self_attn_layer_norm(x)
         key, value = self.self_attn.project_key_value(hidden)
         if self.fused_step and length is None and isinstance(mask, KeyPrefix) and mask.positions is positions:

@@ -244,3 +244,75 @@ def test_gemma_prompt_rows_match_the_ops(device, dtype, layer_type, monkeypatch)
         assert_ulps(got, want, dtype, 4.0)
     for got, want in zip(results[0][:2], results[1][:2]):
         assert_close(got, want, "module", 1e-4 if dtype == torch.float32 else 2e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,inputs,outputs", [
+    (1, 8, (1,)), (1, 384, (384, 384, 384)), (2, 520, (7,)), (3, 1280, (5, 66)), (5, 1536, (384,)), (8, 2048, (9,)),
+    (9, 3072, (13,)), (16, 1280, (1280,))])
+def test_rows_linear(device, dtype, rows, inputs, outputs):
+    """A step's linear layers: odd output counts (columns past the last),
+    rows that fill no workgroup, reductions shorter and longer than a wave and
+    past 512 threads, with and without bias, norm, activation and residual.
+    Against float64 on the same inputs, rounded where the ops round: float32
+    sums of k products (1e-5), or one bf16 rounding after another (2e-2)."""
+    import torch.nn.functional as F
+    from torch import nn
+
+    from asrback_amd import layers
+
+    say("rows linear", dtype, rows, inputs, outputs)
+    torch.manual_seed(8)
+    x = torch.randn(rows, 1, inputs, device=device).mul_(2.0).add_(0.5).to(dtype)
+    linears = [nn.Linear(inputs, n, bias=i != 1) for i, n in enumerate(outputs)]
+    linears = [m.to(device, dtype).requires_grad_(False) for m in linears]
+    norm = nn.LayerNorm(inputs).to(device, dtype).requires_grad_(False)
+    norm.weight.normal_(1.0, 0.2)
+    norm.bias.normal_(0.0, 0.2)
+    residual = torch.randn(rows, 1, outputs[0], device=device).to(dtype)
+    assert layers.rows_linear_takes(x, linears, [norm], [])
+
+    def exact(m, use_norm):
+        h = x.double()
+        if use_norm:
+            h = F.layer_norm(h, (inputs,), norm.weight.double(), norm.bias.double(), norm.eps).to(dtype).double()
+        return F.linear(h, m.weight.double(), None if m.bias is None else m.bias.double())
+
+    for use_norm in (False, True):
+        got = layers.rows_linear(x, linears, norm if use_norm else None)
+        for out, m in zip(got, linears):
+            assert_close(out.cpu(), exact(m, use_norm).cpu(), KIND[dtype])
+        got = layers.rows_linear(x, linears, norm if use_norm else None, gelu=True)
+        for out, m in zip(got, linears):
+            assert_close(out.cpu(), F.gelu(exact(m, use_norm).to(dtype).double()).cpu(), KIND[dtype])
+        (out,) = layers.rows_linear(x, linears[:1], norm if use_norm else None, residual=residual)
+        assert_close(out.cpu(), (residual.double() + exact(linears[0], use_norm)).cpu(), KIND[dtype])
+
+
+def test_rows_linear_leaves_other_programs_to_the_ops(device):
+    """Inputs whose ops something has to see, or the kernel does not address."""
+    from torch import nn
+
+    from asrback_amd import layers
+
+    linear, norm = nn.Linear(64, 64).to(device), nn.LayerNorm(64).to(device)
+    x = torch.randn(2, 1, 64, device=device)
+
+    def takes(x=x):
+        return layers.rows_linear_takes(x, [linear], [norm], [])
+
+    assert not takes()  # weights that collect gradients
+    with torch.no_grad():
+        assert takes()
+        assert not takes(x.double()) and not takes(x[:, :, 1:]) and not takes(x.expand(2, 3, 64))
+        assert not takes(torch.randn(17, 1, 64, device=device)) and not takes(x.cpu())
+        assert not takes(torch.randn(2, 1, 68, device=device)[..., 2:66])  # 8-byte aligned
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert not takes()
+        seen = []
+        torch.vmap(lambda t: seen.append(takes(t)) or t)(x[None])
+        assert seen == [False]
+        hook = norm.register_forward_hook(lambda *a: None)
+        assert not takes()
+        hook.remove()
+        assert takes()
