@@ -26,6 +26,17 @@
 // key row, lanes 32..63 of another).  Buffer resources end at the block's
 // last visible key, so loads past it return zeros without a branch.
 //
+// Head dims 256 and 512 (Gemma 4) split a row block's dimensions over DS waves
+// of 64 each, as the bf16 kernel does: a wave computes its dimensions' part of
+// S^T and writes it to LDS, every wave of the row block sums the parts in the
+// same order behind an LDS-only barrier (two buffers, so one barrier a
+// sub-tile; the operand loads stay in flight across it), runs the same softmax
+// and scales its own output columns.  Sliding windows (WIN) start at the
+// sub-tile of the block's first visible key.  Against the vector ALUs: one
+// prompt of 400 tokens, 8 heads over 4 of 256, window 512: 967 -> 51 us; heads
+// of 512: 1250 -> 92; eight prompts of 820: 2537 -> 298 and 6276 -> 740; the
+// error against float64 falls by a third.
+//
 // Softmax in base 2 with scale * log2(e) folded into one FMA per score; the
 // running max is lazy as in the bf16 kernel (rescale only when a row's max
 // grows by more than 2^8).
@@ -67,8 +78,9 @@ struct Operands {
   float v[F32Shape<HD>::kV];
 };
 
-template <int HD, int KS, int OCC>
-__global__ __launch_bounds__(64 * KS, OCC) void fwd_f32mm_kernel(const FwdArgs a, int q_tiles, int total) {
+// HD: head dimensions of one wave; the head has HD * DS.
+template <int HD, int KS, int OCC, int DS, bool WIN>
+__global__ __launch_bounds__(64 * KS * DS, OCC) void fwd_f32mm_kernel(const FwdArgs a, int q_tiles, int total) {
   using S = F32Shape<HD>;
   constexpr int NQ = S::kQ4, DB = S::kDB;
   const asrattn_fwd_params& p = a.p;
@@ -86,14 +98,17 @@ __global__ __launch_bounds__(64 * KS, OCC) void fwd_f32mm_kernel(const FwdArgs a
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int ks = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ks = wave % KS;   // key split
+  const int dh = wave / KS;   // dimension split: head dims [dh HD, dh HD + HD)
   const int r32 = lane & 31;
   const int half = lane >> 5;
   if (row0 >= len_c) {
     // Rows at or past the key count of a zero-padded batch: zeros.
-    for (int i = tid; i < (min(row0 + 32, sv.len_q) - row0) * (HD / 4); i += 64 * KS) {
-      float* op = static_cast<float*>(p.out) + sv.o_off + (int64_t)(row0 + i / (HD / 4)) * p.o_token_stride +
-                  (i % (HD / 4)) * 4;
+    constexpr int kChunks = HD * DS / 4;
+    for (int i = tid; i < (min(row0 + 32, sv.len_q) - row0) * kChunks; i += 64 * KS * DS) {
+      float* op = static_cast<float*>(p.out) + sv.o_off + (int64_t)(row0 + i / kChunks) * p.o_token_stride +
+                  (i % kChunks) * 4;
       *reinterpret_cast<float4*>(op) = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     return;
@@ -103,12 +118,14 @@ __global__ __launch_bounds__(64 * KS, OCC) void fwd_f32mm_kernel(const FwdArgs a
   const int row_lim = row_ok ? visible_keys(p, sv, row) : 0;  // keys [0, row_lim) of this row
   const int kend = visible_keys(p, sv, min(row0 + 32, len_c) - 1);
   const int n_sub = (kend + 31) / 32;
+  const int row_lo = WIN ? first_key(p, sv, row) : 0;
+  const int sub0 = WIN ? min(first_key(p, sv, row0), kend) / 32 : 0;  // the block's first sub-tile
 
   // Q^T operand: step t takes head dimension 8 (t / 4) + 4 half + t % 4 of the row.
   float qreg[S::kSteps];
   {
     const float* qp = static_cast<const float*>(p.q) + sv.q_off + (int64_t)(row_ok ? row : 0) * p.q_token_stride +
-                      4 * half;
+                      dh * HD + 4 * half;
 #pragma unroll
     for (int j = 0; j < NQ; ++j) {
       const float4 v = row_ok ? *reinterpret_cast<const float4*>(qp + 8 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -127,8 +144,8 @@ __global__ __launch_bounds__(64 * KS, OCC) void fwd_f32mm_kernel(const FwdArgs a
       buffer_rsrc(static_cast<const float*>(p.v) + sv.v_off, (uint32_t)kend * vts);
   // Lane offsets inside a sub-tile: K row r32 at head dimensions 8 j + 4 half;
   // V^T row (head dimension) 32 db + r32 of key 8 (t / 4) + 4 half + t % 4.
-  const uint32_t koff = (uint32_t)r32 * kts + (uint32_t)half * 16;
-  const uint32_t voff = (uint32_t)(4 * half) * vts + (uint32_t)r32 * 4;
+  const uint32_t koff = (uint32_t)r32 * kts + (uint32_t)(dh * HD * 4 + half * 16);
+  const uint32_t voff = (uint32_t)(4 * half) * vts + (uint32_t)(dh * HD * 4 + r32 * 4);
 
   auto load = [&](Operands<HD>& o, int sub) {
     const uint32_t kb = (uint32_t)(sub * 32) * kts + koff;
@@ -150,15 +167,34 @@ __global__ __launch_bounds__(64 * KS, OCC) void fwd_f32mm_kernel(const FwdArgs a
   float m_run = kNegInf;
   float l_run = 0.f;
 
-  auto tile = [&](const Operands<HD>& o, int sub) {
+  // The dimension splits' parts of S^T, lane-major, in two buffers.
+  constexpr int kPart = 16 * 64;
+  __shared__ float part[DS > 1 ? 2 * KS * DS * kPart : 1];
+
+  auto tile = [&](const Operands<HD>& o, int sub, int buffer) {
     f32x16_t s = f32x16_t{};
 #pragma unroll
     for (int t = 0; t < S::kSteps; ++t) s = mfma_f32(o.k[t / 4][t % 4], qreg[t], s);
+    if constexpr (DS > 1) {
+      float* const parts = part + buffer * KS * DS * kPart + lane;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) parts[wave * kPart + r * 64] = s[r];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+      s = f32x16_t{};
+#pragma unroll
+      for (int d = 0; d < DS; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] += parts[(d * KS + ks) * kPart + r * 64];
+    }
     // Keys past the row's limit -> -inf (register r: key 32 sub + 8 (r / 4) + 4 half + r % 4).
     const int kt = sub * 32;
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      if (kt + 8 * (r / 4) + 4 * half + r % 4 >= row_lim) s[r] = kNegInf;
+    for (int r = 0; r < 16; ++r) {
+      const int key = kt + 8 * (r / 4) + 4 * half + r % 4;
+      if (key >= row_lim || (WIN && key < row_lo)) s[r] = kNegInf;
+    }
     float mt = s[0];
 #pragma unroll
     for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
@@ -191,23 +227,28 @@ __global__ __launch_bounds__(64 * KS, OCC) void fwd_f32mm_kernel(const FwdArgs a
   // The loads are unconditional (past the block's last key they read zeros
   // and are never used): a load under a branch makes the compiler drain
   // every load at the join, the prefetch included.
+  // Dimension splits meet at a barrier in every sub-tile, so all waves make as
+  // many rounds as the first key split (past the last key everything is
+  // masked).
   Operands<HD> opa, opb;
-  load(opa, ks);
-  for (int sub = ks; sub < n_sub; sub += 2 * KS) {
+  const int first = sub0 + ks;
+  const int rounds_end = DS > 1 ? n_sub + ks : n_sub;  // the last round's sub-tile is below
+  load(opa, first);
+  for (int sub = first; sub < rounds_end; sub += 2 * KS) {
     load(opb, sub + KS);
-    tile(opa, sub);
-    if (sub + KS >= n_sub) break;
+    tile(opa, sub, 0);
+    if (sub + KS >= rounds_end) break;
     load(opa, sub + 2 * KS);
-    tile(opb, sub + KS);
+    tile(opb, sub + KS, 1);
   }
 
   // Merge the key splits through LDS: waves 1..KS-1 store (O^T, max, sum),
   // wave 0 folds them in and writes the rows.
   if constexpr (KS > 1) {
     constexpr int kPer = (16 * DB + 2) * 64;
-    __shared__ float mf[(KS - 1) * kPer];
+    __shared__ float mf[(KS - 1) * DS * kPer];
     if (ks > 0) {
-      float* dst = mf + (ks - 1) * kPer + lane;
+      float* dst = mf + ((ks - 1) * DS + dh) * kPer + lane;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -219,7 +260,7 @@ __global__ __launch_bounds__(64 * KS, OCC) void fwd_f32mm_kernel(const FwdArgs a
     if (ks > 0) return;
 #pragma unroll
     for (int s2 = 1; s2 < KS; ++s2) {
-      const float* src = mf + (s2 - 1) * kPer + lane;
+      const float* src = mf + ((s2 - 1) * DS + dh) * kPer + lane;
       const float m2 = src[(16 * DB) * 64];
       const float l2 = src[(16 * DB + 1) * 64];
       const float mn = fmaxf(m_run, m2);
@@ -238,7 +279,7 @@ __global__ __launch_bounds__(64 * KS, OCC) void fwd_f32mm_kernel(const FwdArgs a
   // The half waves hold disjoint keys of the same rows.
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
   const float inv = l_tot > 0.f && row_ok ? 1.f / l_tot : 0.f;  // rows past len_c get zeros
-  float* op = static_cast<float*>(p.out) + sv.o_off + (int64_t)row * p.o_token_stride + 4 * half;
+  float* op = static_cast<float*>(p.out) + sv.o_off + (int64_t)row * p.o_token_stride + dh * HD + 4 * half;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -248,49 +289,57 @@ __global__ __launch_bounds__(64 * KS, OCC) void fwd_f32mm_kernel(const FwdArgs a
                       oacc[db][4 * j + 3] * inv);
 }
 
-template <int HD, int KS>
+template <int HD, int KS, int DS, bool WIN>
 hipError_t launch_ks(const FwdArgs& a, hipStream_t stream) {
   const asrattn_fwd_params& p = a.p;
   const int q_tiles = (p.max_len_q + 31) / 32;
   const long long total = (long long)q_tiles * p.heads_q * p.batch;
   if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  // Two waves per SIMD at head_dim 64 (about 240 VGPRs), one at 128.
+  // Two waves per SIMD at 64 head dimensions a wave (about 240 VGPRs), one
+  // at 128.
   constexpr int OCC = HD == 64 ? 2 : 1;
-  hipLaunchKernelGGL((fwd_f32mm_kernel<HD, KS, OCC>), dim3((unsigned)total), dim3(64 * KS), 0, stream, a, q_tiles,
-                     (int)total);
+  hipLaunchKernelGGL((fwd_f32mm_kernel<HD, KS, OCC, DS, WIN>), dim3((unsigned)total), dim3(64 * KS * DS), 0, stream, a,
+                     q_tiles, (int)total);
   return hipGetLastError();
 }
 
-template <int HD>
+template <int HD, int DS, bool WIN>
 hipError_t launch_hd(const FwdArgs& a, hipStream_t stream) {
   const asrattn_fwd_params& p = a.p;
   const long long blocks = (long long)((p.max_len_q + 31) / 32) * p.heads_q * p.batch;
   const int subs = (p.max_len_k + 31) / 32;
   // Key splits: as many waves per row block as the CUs hold at once for
-  // all blocks (two per SIMD at head_dim 64; one at 128, where a wave needs
-  // more than 256 registers), and at least two sub-tiles per split.  A
+  // all blocks (two per SIMD at 64 dimensions a wave; one at 128, where a wave
+  // needs more than 256 registers), and at least two sub-tiles per split.  A
   // second round of workgroups would run on few CUs: Whisper-tiny's 282 row
   // blocks take four splits (1128 waves, one round) in 66 us and took 73.8
   // with eight (2256 waves, two rounds).
-  constexpr int kMaxKs = HD == 64 ? 8 : 4;
+  constexpr int kMaxKs = (HD == 64 ? 8 : 4) / DS;
   constexpr long long kResidentWaves = HD == 64 ? 2048 : 1024;
   int ks = 1;
-  while (ks < kMaxKs && blocks * 2 * ks <= kResidentWaves && subs >= 4 * ks) ks *= 2;
-  switch (ks) {
-    case 1: return launch_ks<HD, 1>(a, stream);
-    case 2: return launch_ks<HD, 2>(a, stream);
-    case 4: return launch_ks<HD, 4>(a, stream);
-    default:
-      if constexpr (HD == 64) return launch_ks<HD, 8>(a, stream);
-      return launch_ks<HD, 4>(a, stream);
+  while (ks < kMaxKs && blocks * 2 * ks * DS <= kResidentWaves && subs >= 4 * ks) ks *= 2;
+  if constexpr (kMaxKs >= 8) {
+    if (ks == 8) return launch_ks<HD, 8, DS, WIN>(a, stream);
   }
+  if constexpr (kMaxKs >= 4) {
+    if (ks == 4) return launch_ks<HD, 4, DS, WIN>(a, stream);
+  }
+  if constexpr (kMaxKs >= 2) {
+    if (ks == 2) return launch_ks<HD, 2, DS, WIN>(a, stream);
+  }
+  return launch_ks<HD, 1, DS, WIN>(a, stream);
+}
+
+template <int HD, int DS>
+hipError_t launch_window(const FwdArgs& a, hipStream_t stream) {
+  return a.p.window > 0 ? launch_hd<HD, DS, true>(a, stream) : launch_hd<HD, DS, false>(a, stream);
 }
 
 }  // namespace
 
 bool fwd_f32mm_supported(const asrattn_fwd_params& p) {
-  if (p.dtype != ASRATTN_F32 || p.window > 0) return false;
-  if (p.head_dim != 64 && p.head_dim != 128) return false;
+  if (p.dtype != ASRATTN_F32) return false;
+  if (p.head_dim != 64 && p.head_dim != 128 && p.head_dim != 256 && p.head_dim != 512) return false;
   // K/V addressed with 32-bit byte offsets from the sequence's first key, up
   // to the prefetch of two rounds of eight 32-key sub-tiles past the last.
   const long long span_k = ((long long)p.max_len_k + 16 * 32 + 32) * p.k_token_stride * 4;
@@ -305,7 +354,12 @@ hipError_t launch_fwd_f32mm(const asrattn_fwd_params& p, hipStream_t stream) {
   a.p = p;
   a.c = p.scale * kLog2e;
   a.f = FsmnArgs{};
-  return p.head_dim == 64 ? launch_hd<64>(a, stream) : launch_hd<128>(a, stream);
+  switch (p.head_dim) {
+    case 64: return launch_window<64, 1>(a, stream);
+    case 128: return launch_window<128, 1>(a, stream);
+    case 256: return launch_window<64, 4>(a, stream);
+    default: return launch_window<64, 8>(a, stream);
+  }
 }
 
 }  // namespace asrattn

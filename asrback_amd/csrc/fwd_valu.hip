@@ -5,10 +5,9 @@
 // which keep its scaled query and output accumulator in registers; the
 // partial dot products of a row's lanes are summed with DPP.  Key/value
 // tiles of BN rows are staged in LDS as fp32 and read by all lanes at the
-// same address (broadcast, no bank conflicts).  This is the fp32 path
-// (Whisper in float32, the reference's CPU/fp32 dtype; Gemma 4 in float32 at
-// head_dim 256 and 512) and the exact-arithmetic twin of the bf16
-// matrix-core kernel.
+// same address (broadcast, no bank conflicts).  This is the
+// exact-arithmetic twin of the matrix-core kernels and the path of layouts
+// they do not address.
 #include "common.hpp"
 #include "fwd_common.hpp"
 #include "kernels.hpp"

@@ -316,3 +316,28 @@ def test_rows_linear_leaves_other_programs_to_the_ops(device):
         assert not takes()
         hook.remove()
         assert takes()
+
+
+@pytest.mark.parametrize("hd,window,causal", [(64, 33, 1), (128, 100, 2), (256, 0, 0), (256, 40, 1), (512, 0, 1), (512, 64, 2)])
+@pytest.mark.parametrize("len_q,len_k,batch", [(1, 1, 1), (32, 32, 2), (33, 97, 2), (200, 200, 1), (1, 300, 3)])
+def test_float32_wide_heads_and_windows(ops, device, hd, window, causal, len_q, len_k, batch):
+    """float32 attention on the matrix cores at head_dim 256 and 512 (a row
+    block's dimensions split over waves) and within sliding windows, around
+    the 32-row and 32-key edges, with grouped heads and per-row key counts
+    (zero keys among them)."""
+    from asrback_amd import _lib
+
+    say("f32 wide", hd, window, causal, len_q, len_k, batch)
+    q = randn(batch, len_q, 4, hd, seed=21)
+    k, v = (randn(batch, len_k, 2, hd, seed=s) for s in (22, 23))
+    used = torch.tensor([len_k, len_k // 2, 0][:batch], dtype=torch.int32)
+    i, j, n = torch.arange(len_q)[:, None], torch.arange(len_k), used[:, None, None]
+    last = i + (n - len_q if causal == _lib.CAUSAL_BOTTOM_RIGHT else 0)
+    visible = (j < n).expand(batch, len_q, len_k)
+    if causal:
+        visible = visible & (j <= last)
+    if window:
+        visible = visible & (j > last - window)
+    out = ops.flash(q.to(device), k.to(device), v.to(device), causal=causal, seqused_k=used.to(device),
+                    window=window)
+    assert_close(out.cpu(), attend(q, k, v, hd**-0.5, visible), "f32")
