@@ -39,7 +39,7 @@
 //      64-byte bank ranges.
 //
 // Workgroups may also split the keys across waves (KS splits, merged through
-// LDS at the end), which shortens the longest workgroups of ragged batches.
+// LDS at the end): the launches of small batches, which leave CUs idle.
 //
 // Work mapping: a flat grid of (sequence, head, query tile) items, taken
 // longest-first in ragged batches, with the query tiles of one (sequence,
@@ -621,7 +621,8 @@ hipError_t launch_hd(const FwdArgs& a, hipStream_t stream) {
   // Four waves (128 query rows) share each 64-key tile through two stages:
   // two workgroups per CU, whose waves pair up on the SIMDs without sharing
   // a barrier.  Key splits (KS > 1) halve the rows a CU holds at two waves
-  // per SIMD, which costs more than they save once the batch fills the GPU.
+  // per SIMD, which costs more than they save once the batch fills the GPU
+  // (smaller launches: below).
   // Head dims 256 and 512 (Gemma 4) split each row block's dimensions over
   // waves (32 rows' queries and outputs of all 256 dimensions fit one wave
   // only at one wave per SIMD, of 512 not without spilling); 32-key tiles.
@@ -641,6 +642,31 @@ hipError_t launch_hd(const FwdArgs& a, hipStream_t stream) {
     return launch_typed<HD, 4, 1, 32, 2, 1, 0, false, 2>(a, stream);
   } else {
     if (win) return launch_typed<HD, 4, 1, 64, 2, 2, 0, true>(a, stream);
+    // Launches that leave CUs idle, or hold one workgroup on each: fewer rows
+    // a workgroup and the keys split over its waves, while that makes at most
+    // one workgroup per CU (two of 128 rows at head_dim 64, where eight waves
+    // then share a CU's SIMDs in pairs).  us per launch, 128 rows unsplit
+    // against the split: 1500 keys, 6 heads x 1500 rows 21.9 -> 14.4 (64 rows),
+    // 20 heads 24.8 -> 20.0 (128 rows; 64 rows 22.9), 2 x 20 heads 34.9 -> 33.5,
+    // 3 x 20 the same; 8 x 12 heads x 4 rows 20.5 -> 14.0 (32 rows; 64 rows
+    // 14.3), 16 x 20 heads x 4 rows (320 workgroups) 30.1 -> 31.1.  head_dim 128:
+    // 4 heads x 300 and 504 rows with the FSMN memory 10.4 -> 9.3 and 13.3 ->
+    // 11.2, 16 causal heads x 430 rows 12.3 -> 11.0, 4 x 16 heads x 430 (448
+    // workgroups of 64 rows) 13.8 -> 14.6.  Where one unsplit tile or two hold
+    // all keys, splitting them only adds the merge (16 x 60 keys: 6.3 -> 6.9).
+    const auto groups = [&](int rows) {
+      return (long long)((a.p.max_len_q + rows - 1) / rows) * a.p.heads_q * a.p.batch;
+    };
+    if constexpr (HD == 64) {
+      if (a.f.memory == nullptr && a.p.max_len_k > 128) {
+        if (groups(32) <= 256) return launch_typed<HD, 1, 4, 32, 2, 2, 0>(a, stream);
+        if (groups(64) <= 256) return launch_typed<HD, 2, 4, 32, 2, 2, 0>(a, stream);
+        if (groups(128) <= 512) return launch_typed<HD, 4, 2, 64, 2, 2, 0>(a, stream);
+      }
+    } else if (a.p.max_len_k > 64 && groups(64) <= 256) {
+      if (a.f.memory != nullptr) return launch_typed<HD, 2, 2, 32, 2, 2, kFsmnFusedKernel>(a, stream);
+      return launch_typed<HD, 2, 2, 32, 2, 2, 0>(a, stream);
+    }
     if (a.f.memory != nullptr) return launch_typed<HD, 4, 1, 64, 2, 2, kFsmnFusedKernel>(a, stream);
     return launch_typed<HD, 4, 1, 64, 2, 2, 0>(a, stream);
   }

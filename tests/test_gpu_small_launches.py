@@ -341,3 +341,43 @@ def test_float32_wide_heads_and_windows(ops, device, hd, window, causal, len_q, 
     out = ops.flash(q.to(device), k.to(device), v.to(device), causal=causal, seqused_k=used.to(device),
                     window=window)
     assert_close(out.cpu(), attend(q, k, v, hd**-0.5, visible), "f32")
+
+
+@pytest.mark.parametrize("hd,heads,kv_heads,causal", [(64, 3, 3, 0), (64, 12, 12, 1), (128, 4, 4, 0), (128, 16, 8, 2)])
+@pytest.mark.parametrize("len_q,len_k,batch", [
+    (4, 129, 2), (4, 1500, 3), (33, 300, 2), (64, 65, 1), (65, 64, 1), (130, 257, 4), (300, 300, 1), (700, 700, 3),
+    (128, 131, 8)])
+def test_small_bf16_launches(ops, device, hd, heads, kv_heads, causal, len_q, len_k, batch):
+    """bf16 launches around the lines where a workgroup's rows and key splits
+    change (32, 64 and 128 rows; one workgroup per CU), with per-row key
+    counts that end splits early or leave them empty."""
+    say("small bf16", hd, heads, kv_heads, causal, len_q, len_k, batch)
+    q = randn(batch, len_q, heads, hd, seed=31, dtype=torch.bfloat16)
+    k, v = (randn(batch, len_k, kv_heads, hd, seed=s, dtype=torch.bfloat16) for s in (32, 33))
+    used = torch.tensor([len_k, 1, len_k // 2, 0] * 2, dtype=torch.int32)[:batch]
+    i, j, n = torch.arange(len_q)[:, None], torch.arange(len_k), used[:, None, None]
+    visible = (j < n).expand(batch, len_q, len_k)
+    if causal:
+        visible = visible & (j <= i + (n - len_q if causal == 2 else 0))
+    out = ops.flash(q.to(device), k.to(device), v.to(device), causal=causal, seqused_k=used.to(device))
+    assert_close(out.float().cpu(), attend(q, k, v, hd**-0.5, visible), "bf16")
+
+
+@pytest.mark.parametrize("frames,batch", [(65, 1), (100, 1), (300, 2), (504, 1), (130, 9)])
+def test_small_sanm_launches(ops, device, frames, batch):
+    """SAN-M attention with its memory in the launches of few utterances: the
+    memory's row blocks follow the attention's."""
+    say("small sanm", frames, batch)
+    x = randn(batch, frames, 1536, seed=41, dtype=torch.bfloat16)
+    weight = randn(512, 1, 11, seed=42, dtype=torch.bfloat16)
+    used = torch.tensor([frames] + [1 + 17 * b for b in range(1, batch)], dtype=torch.int32)
+    q, k, v = (t.view(batch, frames, 4, 128) for t in x.split(512, dim=-1))
+    keep = torch.arange(frames) < used[:, None]
+    ref = attend(q, k, v, 128**-0.5, keep[:, None].expand(batch, frames, frames)) * keep[..., None, None]
+    inside = (v.reshape(batch, frames, 512).double() * keep[..., None]).transpose(1, 2)
+    conv = torch.nn.functional.conv1d(torch.nn.functional.pad(inside, (5, 5)), weight.double(), groups=512)
+    memory_ref = ((conv + inside) * keep[:, None]).transpose(1, 2)
+    q, k, v = (t.view(batch, frames, 4, 128) for t in x.to(device).split(512, dim=-1))
+    out, memory = ops.flash_fsmn(q, k, v, weight.to(device), seqused_k=used.to(device), zero_padded_rows=True)
+    assert_close(out.float().cpu(), ref, "bf16")
+    assert_close(memory.float().cpu(), memory_ref, "bf16")
