@@ -629,39 +629,49 @@ hipError_t launch_hd(const FwdArgs& a, hipStream_t stream) {
   // Sliding windows (causal, Gemma 4) take a variant that starts each
   // workgroup's keys at its first row's window.
   const bool win = a.p.window > 0;
+  const auto groups = [&](int rows) {
+    return (long long)((a.p.max_len_q + rows - 1) / rows) * a.p.heads_q * a.p.batch;
+  };
   if constexpr (HD == 512) {
     // 64 query rows, each row block's dimensions over four waves (eight
     // waves, the whole 160 KB of LDS; 7% faster than two waves per row block).
+    // 32 rows where 64 make at most one workgroup per CU: prompts of 840
+    // tokens, 8 heads, one 53.9 -> 45.5 us, two 54.6 -> 46.5, four (448
+    // workgroups of 64 rows) 82.7 -> 108.
+    if (groups(64) <= 256) {
+      if (win) return launch_typed<HD, 1, 1, 32, 2, 1, 0, true, 4>(a, stream);
+      return launch_typed<HD, 1, 1, 32, 2, 1, 0, false, 4>(a, stream);
+    }
     if (win) return launch_typed<HD, 2, 1, 32, 2, 1, 0, true, 4>(a, stream);
     return launch_typed<HD, 2, 1, 32, 2, 1, 0, false, 4>(a, stream);
   } else if constexpr (HD == 256) {
-    // 128 query rows, each row block's dimensions over two waves (eight
-    // waves, two per SIMD: 9% faster on Gemma 4's prompt pass than four
-    // waves holding all 256 dimensions at one per SIMD).
-    if (win) return launch_typed<HD, 4, 1, 32, 2, 1, 0, true, 2>(a, stream);
-    return launch_typed<HD, 4, 1, 32, 2, 1, 0, false, 2>(a, stream);
+    // 64 query rows, each row block's dimensions over two waves: four waves
+    // in 80 KB of LDS, two workgroups per CU that share no barrier.  Against
+    // 128 rows in eight waves (96 KB, one per CU), 8 heads within 512 keys: 100
+    // tokens 12.6 -> 9.7 us, two prompts of 840 36.1 -> 25.2, four 37.1 -> 33.0,
+    // eight 69.4 -> 55.0 (32 rows: 9.9, 26.3, 49.2, 77.7; 64-key tiles: 10.4,
+    // 25.7, 46.3, 73.7).
+    if (win) return launch_typed<HD, 2, 1, 32, 2, 2, 0, true, 2>(a, stream);
+    return launch_typed<HD, 2, 1, 32, 2, 2, 0, false, 2>(a, stream);
   } else {
     if (win) return launch_typed<HD, 4, 1, 64, 2, 2, 0, true>(a, stream);
     // Launches that leave CUs idle, or hold one workgroup on each: fewer rows
     // a workgroup and the keys split over its waves, while that makes at most
-    // one workgroup per CU (two of 128 rows at head_dim 64, where eight waves
-    // then share a CU's SIMDs in pairs).  us per launch, 128 rows unsplit
+    // one workgroup per CU.  us per launch, 128 rows unsplit
     // against the split: 1500 keys, 6 heads x 1500 rows 21.9 -> 14.4 (64 rows),
-    // 20 heads 24.8 -> 20.0 (128 rows; 64 rows 22.9), 2 x 20 heads 34.9 -> 33.5,
-    // 3 x 20 the same; 8 x 12 heads x 4 rows 20.5 -> 14.0 (32 rows; 64 rows
-    // 14.3), 16 x 20 heads x 4 rows (320 workgroups) 30.1 -> 31.1.  head_dim 128:
+    // 20 heads 24.8 -> 20.0 (128 rows; 64 rows 22.9), 8 x 12 heads x 4 rows
+    // 20.5 -> 14.0 (32 rows; 64 rows 14.3); more workgroups gain or lose a few
+    // percent (2 x 20 heads x 1500 rows 34.9 -> 33.5, 16 x 20 heads x 128 rows
+    // 37.0 -> 38.6, x 4 rows 30.1 -> 31.1).  head_dim 128:
     // 4 heads x 300 and 504 rows with the FSMN memory 10.4 -> 9.3 and 13.3 ->
     // 11.2, 16 causal heads x 430 rows 12.3 -> 11.0, 4 x 16 heads x 430 (448
     // workgroups of 64 rows) 13.8 -> 14.6.  Where one unsplit tile or two hold
     // all keys, splitting them only adds the merge (16 x 60 keys: 6.3 -> 6.9).
-    const auto groups = [&](int rows) {
-      return (long long)((a.p.max_len_q + rows - 1) / rows) * a.p.heads_q * a.p.batch;
-    };
     if constexpr (HD == 64) {
       if (a.f.memory == nullptr && a.p.max_len_k > 128) {
         if (groups(32) <= 256) return launch_typed<HD, 1, 4, 32, 2, 2, 0>(a, stream);
         if (groups(64) <= 256) return launch_typed<HD, 2, 4, 32, 2, 2, 0>(a, stream);
-        if (groups(128) <= 512) return launch_typed<HD, 4, 2, 64, 2, 2, 0>(a, stream);
+        if (groups(128) <= 256) return launch_typed<HD, 4, 2, 64, 2, 2, 0>(a, stream);
       }
     } else if (a.p.max_len_k > 64 && groups(64) <= 256) {
       if (a.f.memory != nullptr) return launch_typed<HD, 2, 2, 32, 2, 2, kFsmnFusedKernel>(a, stream);
