@@ -145,22 +145,21 @@ def _dtype_code(*tensors: Tensor) -> int:
     for tensor in tensors:
         if tensor.dtype != dtype:
             raise TypeError(f"mixed dtypes: {dtype} and {tensor.dtype}")
-        if tensor.device.type != "cuda":
+        if not tensor.is_cuda:
             raise RuntimeError(
                 f"attention kernels run on the GPU only; got a tensor on {tensor.device}"
             )
     return _DTYPES[dtype]
 
 
-def _aligned(t: Tensor, dims: tuple[int, ...]) -> Tensor:
-    """``t`` itself when its rows can be read with 16-byte vectors, else a
-    contiguous copy.  ``dims`` are the strided (non head_dim) axes."""
-    per_vec = 16 // t.element_size()
-    if (
-        t.stride(-1) == 1
-        and t.data_ptr() % 16 == 0
-        and all(t.stride(d) % per_vec == 0 for d in dims)
-    ):
+def _aligned(t: Tensor) -> Tensor:
+    """``t`` itself when its rows (its last axis) can be read with 16-byte
+    vectors, else a contiguous copy."""
+    *strides, last = t.stride()
+    bits = 0
+    for stride in strides:
+        bits |= stride  # a vector is a power of two of elements: one test for all
+    if last == 1 and t.data_ptr() % 16 == 0 and bits % (16 // t.element_size()) == 0:
         return t
     return t.contiguous()
 
@@ -170,7 +169,9 @@ def _ptr(t: Tensor | None) -> int | None:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle (``torch.cuda.current_stream(device)
+    .cuda_stream`` without building a Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _check_device(*tensors: Tensor | None) -> torch.device:
@@ -180,7 +181,8 @@ def _check_device(*tensors: Tensor | None) -> torch.device:
             continue
         if device is None:
             device = tensor.device
-        elif tensor.device != device:
+            index = tensor.get_device()  # -1: the CPU
+        elif tensor.get_device() != index:
             raise RuntimeError(f"tensors on different devices: {device} and {tensor.device}")
     if device.index is not None and device.index != torch.cuda.current_device():
         raise RuntimeError(
@@ -221,22 +223,23 @@ def _fwd_params(
     if packed != (cu_seqlens_k is not None):
         raise ValueError("cu_seqlens_q and cu_seqlens_k go together")
     rank = 3 if packed else 4
-    for name, t in (("q", q), ("k", k), ("v", v)):
-        if t.dim() != rank:
-            raise ValueError(f"{name} must have {rank} dimensions, got shape {tuple(t.shape)}")
-    if k.shape != v.shape:
-        raise ValueError(f"k and v shapes differ: {tuple(k.shape)} vs {tuple(v.shape)}")
-    head_dim = q.shape[-1]
-    heads_q, heads_kv = q.shape[-2], k.shape[-2]
-    if k.shape[-1] != head_dim:
+    q_shape, k_shape = q.shape, k.shape
+    if len(q_shape) != rank or len(k_shape) != rank or v.dim() != rank:
+        for name, t in (("q", q), ("k", k), ("v", v)):
+            if t.dim() != rank:
+                raise ValueError(f"{name} must have {rank} dimensions, got shape {tuple(t.shape)}")
+    if k_shape != v.shape:
+        raise ValueError(f"k and v shapes differ: {tuple(k_shape)} vs {tuple(v.shape)}")
+    heads_q, head_dim = q_shape[-2:]
+    heads_kv = k_shape[-2]
+    if k_shape[-1] != head_dim:
         raise ValueError("q and k head_dim differ")
     if heads_q % heads_kv:
         raise ValueError(f"{heads_q} query heads are not a multiple of {heads_kv} kv heads")
-    strided = (0, 1, 2) if not packed else (0, 1)
-    q, k, v = (_aligned(t, strided) for t in (q, k, v))
+    q, k, v = _aligned(q), _aligned(k), _aligned(v)
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    elif out.shape != q.shape or out.dtype != q.dtype or out.stride(-1) != 1:
+        out = torch.empty(q_shape, dtype=q.dtype, device=q.device)
+    elif out.shape != q_shape or out.dtype != q.dtype or out.stride(-1) != 1:
         # The kernels write each head's head_dim elements contiguously.
         raise ValueError("out must match q's shape and dtype, with a unit last stride")
     device = _check_device(q, k, v, out, cu_seqlens_q, cu_seqlens_k, seqused_k)
@@ -244,46 +247,29 @@ def _fwd_params(
     cu_seqlens_k = _int32(cu_seqlens_k, "cu_seqlens_k")
     seqused_k = _int32(seqused_k, "seqused_k")
 
-    params = _lib.FwdParams()
-    params.q, params.k, params.v, params.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
     if packed:
         if max_len_q is None or max_len_k is None:
             raise ValueError("packed sequences need max_len_q and max_len_k")
         batch = cu_seqlens_q.shape[0] - 1
         if cu_seqlens_k.shape[0] != batch + 1:
             raise ValueError("cu_seqlens_q and cu_seqlens_k have different lengths")
-        for prefix, t in (("q", q), ("k", k), ("v", v), ("o", out)):
-            setattr(params, f"{prefix}_batch_stride", 0)
-            setattr(params, f"{prefix}_token_stride", t.stride(0))
-            setattr(params, f"{prefix}_head_stride", t.stride(1))
+        strides = [0, *q.stride()[:2], 0, *k.stride()[:2], 0, *v.stride()[:2], 0, *out.stride()[:2]]
     else:
-        batch = q.shape[0]
-        if k.shape[0] != batch:
+        batch = q_shape[0]
+        if k_shape[0] != batch:
             raise ValueError("q and k batch sizes differ")
-        max_len_q = q.shape[1] if max_len_q is None else max_len_q
-        max_len_k = k.shape[1] if max_len_k is None else max_len_k
-        if max_len_q > q.shape[1] or max_len_k > k.shape[1]:
+        max_len_q = q_shape[1] if max_len_q is None else max_len_q
+        max_len_k = k_shape[1] if max_len_k is None else max_len_k
+        if max_len_q > q_shape[1] or max_len_k > k_shape[1]:
             raise ValueError("max_len_q / max_len_k exceed the tensors")
-        for prefix, t in (("q", q), ("k", k), ("v", v), ("o", out)):
-            setattr(params, f"{prefix}_batch_stride", t.stride(0))
-            setattr(params, f"{prefix}_token_stride", t.stride(1))
-            setattr(params, f"{prefix}_head_stride", t.stride(2))
+        strides = [*q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3]]
     if seqused_k is not None and seqused_k.shape[0] != batch:
         raise ValueError(f"seqused_k has {seqused_k.shape[0]} entries for {batch} sequences")
-    params.cu_seqlens_q = _ptr(cu_seqlens_q)
-    params.cu_seqlens_k = _ptr(cu_seqlens_k)
-    params.seqused_k = _ptr(seqused_k)
-    params.batch = batch
-    params.heads_q = heads_q
-    params.heads_kv = heads_kv
-    params.head_dim = head_dim
-    params.max_len_q = max_len_q
-    params.max_len_k = max_len_k
-    params.causal = causal
-    params.dtype = dtype
-    params.scale = 1.0 / math.sqrt(head_dim) if scale is None else scale
-    params.flags = flags | (_lib.FWD_FORCE_VALU if force_valu else 0)
-    params.window = window or 0
+    params = _lib.FwdParams(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), *strides, _ptr(cu_seqlens_q), _ptr(cu_seqlens_k),
+        _ptr(seqused_k), batch, heads_q, heads_kv, head_dim, max_len_q, max_len_k, causal, dtype,
+        1.0 / math.sqrt(head_dim) if scale is None else scale, flags | (_lib.FWD_FORCE_VALU if force_valu else 0),
+        window or 0)
     return params, out, device, (q, k, v, cu_seqlens_q, cu_seqlens_k, seqused_k)
 
 
@@ -397,24 +383,11 @@ def _decode_params(
     scale: float | None,
     window: int = 0,
 ) -> _lib.DecodeParams:
-    params = _lib.DecodeParams()
-    params.q, params.k, params.v, params.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
-    params.q_batch_stride, params.q_head_stride = q.stride(0), q.stride(1)
-    params.k_batch_stride, params.k_token_stride, params.k_head_stride = k.stride(0), k.stride(1), k.stride(2)
-    params.v_batch_stride, params.v_token_stride, params.v_head_stride = v.stride(0), v.stride(1), v.stride(2)
-    params.o_batch_stride, params.o_head_stride = out.stride(0), out.stride(1)
-    params.seqused_k = _ptr(seqused_k)
-    params.positions = _ptr(positions)
-    params.batch = q.shape[0]
-    params.heads_q = q.shape[1]
-    params.heads_kv = k.shape[2]
-    params.head_dim = q.shape[2]
-    params.max_len_k = k.shape[1]
-    params.num_splits = num_splits
-    params.dtype = _dtype_code(q, k, v)
-    params.scale = 1.0 / math.sqrt(q.shape[2]) if scale is None else scale
-    params.window = 0 if window is None else window
-    return params
+    head_dim = q.shape[2]
+    return _lib.DecodeParams(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), *q.stride()[:2], *k.stride()[:3], *v.stride()[:3],
+        *out.stride()[:2], _ptr(seqused_k), _ptr(positions), q.shape[0], q.shape[1], k.shape[2], head_dim, k.shape[1],
+        num_splits, _dtype_code(q, k, v), 1.0 / math.sqrt(head_dim) if scale is None else scale, window or 0)
 
 
 def decode(
@@ -454,8 +427,7 @@ def decode(
     if q.shape[1] % k.shape[2]:
         raise ValueError(f"{q.shape[1]} query heads are not a multiple of {k.shape[2]} kv heads")
     _dtype_code(q, k, v)
-    q = _aligned(q, (0, 1))
-    k, v = (_aligned(t, (0, 1, 2)) for t in (k, v))
+    q, k, v = _aligned(q), _aligned(k), _aligned(v)
     if out is None:
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     elif out.shape != q.shape or out.dtype != q.dtype or out.stride(-1) != 1:
@@ -548,8 +520,7 @@ def decode_append(
         raise ValueError(f"norm weights must be ({head_dim},)")
     if cos is not None and (cos.shape != (batch, head_dim) or sin.shape != (batch, head_dim)):
         raise ValueError(f"cos/sin must be ({batch}, {head_dim})")
-    q = _aligned(q, (0, 1))
-    k_new, v_new = (_aligned(t, (0, 1)) for t in (k_new, v_new))
+    q, k_new, v_new = _aligned(q), _aligned(k_new), _aligned(v_new)
     if q_norm is not None:
         q_norm, k_norm = q_norm.contiguous(), k_norm.contiguous()
     if cos is not None:

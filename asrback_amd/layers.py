@@ -11,6 +11,7 @@ otherwise.
 from __future__ import annotations
 
 import ctypes
+import math
 
 import torch
 from torch import Tensor, nn
@@ -27,62 +28,72 @@ def _plain(*tensors: Tensor) -> bool:
     nothing (autograd, forward-mode, autocast, functorch, dispatch modes,
     tracing) that has to see the ops."""
     first = tensors[0]
-    dtype, device = first.dtype, first.device
-    if dtype not in _DTYPES or device.type != "cuda" or device.index != torch.cuda.current_device():
+    dtype, index = first.dtype, first.get_device()
+    if dtype not in _DTYPES or not first.is_cuda or index != torch.cuda.current_device():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
         if type(t) is not Tensor and type(t) is not nn.Parameter:
             return False
-        if t.dtype != dtype or t.device != device or (grad and t.requires_grad):
-            return False
-        if torch._C._functorch.is_functorch_wrapped_tensor(t):
+        if t.dtype != dtype or t.get_device() != index or (grad and t.requires_grad):
             return False
     return not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
-                or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack())
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
+                or torch._C._functorch.maybe_current_level() is not None)
 
 
 def _vectors(t: Tensor) -> bool:
     """Whether rows of ``t`` (its last axis) can be read 16 bytes at a time."""
-    per = _VECTOR // t.element_size()
-    return t.stride(-1) == 1 and t.data_ptr() % _VECTOR == 0 and all(s % per == 0 for s in t.stride()[:-1])
+    *strides, last = t.stride()
+    bits = 0
+    for stride in strides:
+        bits |= stride  # a vector is a power of two of elements: one test for all
+    return last == 1 and t.data_ptr() % _VECTOR == 0 and bits % (_VECTOR // t.element_size()) == 0
 
 
 def unhooked(*modules: nn.Module) -> bool:
     return not any(m._forward_hooks or m._forward_pre_hooks for m in modules)
 
 
+def _strides(t: Tensor) -> tuple[int, int, int]:
+    """Batch, token and head strides of ``(batch, tokens, heads, head_dim)``
+    or ``(tokens, heads, head_dim)`` rows."""
+    strides = t.stride()
+    return strides[:3] if len(strides) == 4 else (0, *strides[:2])
+
+
 def prompt_rows_takes(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache, v_cache, rows: Tensor | None,
                       positions: Tensor | None, q_norm: nn.Module, k_norm: nn.Module | None, cos: Tensor,
                       sin: Tensor) -> bool:
     """Whether :func:`prompt_rows` takes these (see there): rows ``q``
-    ``(batch, tokens, heads, head_dim)``, tables ``(batch, tokens, head_dim)``
-    or ``(tokens, head_dim)``, caches ``(rows, length, heads, head_dim)``."""
+    ``(batch, tokens, heads, head_dim)`` or ``(tokens, heads, head_dim)``,
+    tables ``(batch, tokens, head_dim)`` or ``(tokens, head_dim)``, caches
+    ``(rows, length, heads, head_dim)``."""
     norms = [q_norm] if k_norm is None else [q_norm, k_norm]
     tensors = [q, cos, sin, *(m.weight for m in norms)]
     if k is not None:
         tensors += [k, v, k_cache, v_cache]
     if not _plain(*tensors) or not unhooked(*norms):
         return False
-    head_dim = q.shape[-1]
+    *batch, tokens, _, head_dim = q.shape
     if head_dim not in (64, 128, 256, 512) or any(m.weight.shape != (head_dim,) for m in norms):
         return False
-    if cos.shape != sin.shape or cos.stride() != sin.stride() or cos.shape[-2:] != (q.shape[1], head_dim):
+    if cos.shape != sin.shape or cos.stride() != sin.stride() or cos.shape[-2:] != (tokens, head_dim):
         return False
-    if cos.dim() > 3 or (cos.dim() == 3 and cos.shape[0] not in (1, q.shape[0])):
+    if cos.dim() > 3 or (cos.dim() == 3 and cos.shape[0] not in (1, *batch)):
         return False
     if k is not None:
-        slots = (q.shape[0] * q.shape[1],) if positions is not None else (q.shape[0],)
+        slots = (math.prod(batch) * tokens if positions is not None else math.prod(batch),)
         for index in (rows, positions):
             if index is None:
                 continue
             if (type(index) is not Tensor or index.dtype != torch.int64 or index.shape != slots
                     or index.device != q.device or not index.is_contiguous()):
                 return False
-        if positions is None and q.shape[1] > k_cache.shape[1]:
+        if positions is None and tokens > k_cache.shape[1]:
             return False
         if (k.shape != v.shape or k_cache.shape != v_cache.shape or k_cache.dim() != 4
-                or k_cache.shape[2:] != k.shape[2:] or k.shape[-1] != head_dim):
+                or k_cache.shape[2:] != k.shape[-2:] or k.shape[-1] != head_dim):
             return False
     return all(_vectors(t) for t in tensors)
 
@@ -93,20 +104,22 @@ def prompt_rows(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache: Tensor |
     """What a prompt pass does to its projections before the attention
     (``asrlayer_prompt_rows``; ``qwen3_asr.py:366-390``, ``gemma4.py:515-561``):
     the per-head norms and the rotation of ``q`` and ``k`` ``(batch, tokens,
-    heads, head_dim)``, with ``v_eps`` the weightless norm of ``v``, and the
+    heads, head_dim)`` (no batch: one), with ``v_eps`` the weightless norm of ``v``, and the
     writes of keys and values to the cache at ``(rows, positions)``, int64 per
     token, or, without ``positions``, at tokens ``0 .. tokens - 1`` of
     ``rows[b]``.  With ``block_table`` the caches are page pools whose last
     page takes what no row owns.  Returns contiguous ``q``, ``k`` and ``v``
     (``v`` itself where it is not normalized); ``k`` None: ``q`` alone."""
-    batch, tokens, heads, head_dim = q.shape
-    q_out = torch.empty((batch, tokens, heads, head_dim), dtype=q.dtype, device=q.device)
+    tokens, heads, head_dim = q.shape[-3:]
+    batch = q.shape[0] if q.dim() == 4 else 1
+    q_out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     rope = (cos.stride(0) if cos.dim() == 3 and cos.shape[0] > 1 else 0, cos.stride(-2))
     common = (q_norm.weight.data_ptr(), None if k is None else k_norm.weight.data_ptr(), cos.data_ptr(), sin.data_ptr(),
-              *rope, q_norm.eps, 0.0 if k is None else k_norm.eps, v_eps or 0.0, v_eps is not None, batch, tokens, heads)
+              *rope, q_norm.eps, 0.0 if k is None else k_norm.eps, v_eps or 0.0, v_eps is not None, batch, tokens,
+              heads)
     if k is None:
         params = _lib.PromptParams(
-            q.data_ptr(), None, None, q_out.data_ptr(), None, None, None, None, *q.stride()[:3], *(0,) * 12, 0, 0,
+            q.data_ptr(), None, None, q_out.data_ptr(), None, None, None, None, *_strides(q), *(0,) * 12, 0, 0,
             None, None, None, 0, 0, 0, *common, 0, head_dim, _DTYPES[q.dtype])
         k_out = v_out = None
     else:
@@ -121,8 +134,8 @@ def prompt_rows(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache: Tensor |
         params = _lib.PromptParams(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), q_out.data_ptr(), k_out.data_ptr(),
             None if v_eps is None else v_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-            *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *k_cache.stride()[:3], *v_cache.stride()[:3], *extent,
-            rows.data_ptr(), None if positions is None else positions.data_ptr(), *table, *common, k.shape[2], head_dim,
+            *_strides(q), *_strides(k), *_strides(v), *_strides(k_cache), *_strides(v_cache), *extent,
+            rows.data_ptr(), None if positions is None else positions.data_ptr(), *table, *common, k.shape[-2], head_dim,
             _DTYPES[q.dtype])
     lib = _lib.load()
     _lib.check(lib.asrlayer_prompt_rows(ctypes.byref(params), _stream(q.device)), "asrlayer_prompt_rows")

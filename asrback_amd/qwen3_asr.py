@@ -283,7 +283,7 @@ class TextAttention(nn.Module):
     def _prompt_rows(self, x, keys, values, rows, positions, cos, sin) -> tuple[Tensor, Tensor, Tensor]:
         """The prompt's queries, keys and values, keys and values written to
         the cache."""
-        shape = (1, len(x), -1, self.head_dim)
+        shape = (len(x), -1, self.head_dim)
         qkv = self.qkv_proj(x)
         if x.dim() == 2:
             q, k, v = (t.view(shape) for t in qkv.split(self.sizes, dim=-1))
@@ -293,9 +293,8 @@ class TextAttention(nn.Module):
                     and type(self.q_norm) is RMSNorm and type(self.k_norm) is RMSNorm
                     and prompt_rows_takes(q, k, v, key_cache, value_cache, rows, positions, self.q_norm, self.k_norm,
                                           cos, sin)):
-                q, k, v = prompt_rows(q, k, v, key_cache, value_cache, rows, positions, self.q_norm, self.k_norm, cos,
-                                      sin, block_table=table)
-                return q[0], k[0], v[0]
+                return prompt_rows(q, k, v, key_cache, value_cache, rows, positions, self.q_norm, self.k_norm, cos,
+                                   sin, block_table=table)
         q, k, v = self._norm_rotate(qkv, cos, sin)
         keys[rows, positions] = k
         values[rows, positions] = v
