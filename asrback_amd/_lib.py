@@ -257,8 +257,19 @@ class LinearParams(ctypes.Structure):
     ]
 
 
+class GemmParams(ctypes.Structure):
+    """``asrlayer_gemm_params`` (csrc/layers.hpp)."""
+
+    _fields_ = [
+        *[(name, _ptr) for name in ("x", "w", "bias", "out", "used")],
+        *[(name, _i64) for name in ("x_batch_stride", "x_row_stride", "out_batch_stride", "out_row_stride")],
+        *[(name, _i32) for name in ("batch", "rows", "n", "k", "accumulate")],
+    ]
+
+
 # The layers' own entry points (csrc/layers.hpp).
 LAYER_SIGNATURES = {
+    "asrlayer_gemm": (ctypes.c_int, [ctypes.POINTER(GemmParams), _ptr]),
     "asrlayer_rows_linear": (ctypes.c_int, [ctypes.POINTER(LinearParams), _ptr]),
     "asrlayer_prompt_rows": (ctypes.c_int, [ctypes.POINTER(PromptParams), _ptr]),
 }

@@ -515,4 +515,27 @@ int asrlayer_rows_linear(const asrlayer_linear_params* params, void* stream) {
   return from_hip(asrattn::launch_rows_linear(p, static_cast<hipStream_t>(stream)), "asrlayer_rows_linear");
 }
 
+int asrlayer_gemm(const asrlayer_gemm_params* params, void* stream) {
+  if (params == nullptr) return fail(ASRATTN_ERR_INVALID, "params is NULL");
+  const asrlayer_gemm_params& p = *params;
+  if (p.batch < 0 || p.rows < 0 || p.n <= 0 || p.k <= 0)
+    return fail(ASRATTN_ERR_INVALID, "batch and rows must be >= 0, n and k positive");
+  if (p.k % 64 != 0 || p.n % 8 != 0)
+    return fail(ASRATTN_ERR_UNSUPPORTED, "k (%d) must be a multiple of 64, n (%d) of 8", p.k, p.n);
+  if (p.batch == 0 || p.rows == 0) return ok();
+  if (p.x == nullptr || p.w == nullptr || p.out == nullptr)
+    return fail(ASRATTN_ERR_INVALID, "x, w and out must be non-NULL");
+  if (p.accumulate != 0 && p.bias != nullptr) return fail(ASRATTN_ERR_INVALID, "an accumulating layer takes no bias");
+  if (!vec_aligned(p.x, ASRATTN_BF16, {p.x_batch_stride, p.x_row_stride}) || !vec_aligned(p.w, ASRATTN_BF16, {}) ||
+      !vec_aligned(p.bias, ASRATTN_BF16, {}) ||
+      !vec_aligned(p.out, ASRATTN_BF16, {p.out_batch_stride, p.out_row_stride}))
+    return fail(ASRATTN_ERR_INVALID, "tensors need 16-byte aligned pointers and strides that are multiples of 16 bytes");
+  // A tile's rows are addressed with 32-bit byte offsets; rows may not overlap.
+  if (p.x_row_stride < p.k || p.x_row_stride > (1 << 22) || p.k > (1 << 22) || p.out_row_stride < p.n)
+    return fail(ASRATTN_ERR_UNSUPPORTED, "row strides out of range");
+  if ((long long)p.batch * ((p.rows + 31) / 32) * (((long long)p.n + 31) / 32) > 0x7fffffffLL * 16)
+    return fail(ASRATTN_ERR_UNSUPPORTED, "more than 2^31 output tiles");
+  return from_hip(asrattn::launch_gemm(p, static_cast<hipStream_t>(stream)), "asrlayer_gemm");
+}
+
 }  // extern "C"

@@ -82,4 +82,22 @@ typedef struct asrlayer_linear_params {
 
 int asrlayer_rows_linear(const asrlayer_linear_params* params, void* stream);
 
+// A linear layer over bf16 rows (batch x rows of k inputs, n outputs each):
+//
+//   out[b, t, :] = x[b, t, :] w^T + bias        (accumulate 0; bias or NULL)
+//   out[b, t, :] = out[b, t, :] + x[b, t, :] w^T    (accumulate 1, no bias)
+//
+// with float32 sums, rounded once.  w (n, k) contiguous; rows x_row_stride
+// and out_row_stride apart.  used (int32[batch], device, or NULL): rows t >=
+// used[b] are neither read nor written.  k a multiple of 64, n of 8.
+typedef struct asrlayer_gemm_params {
+  const void *x, *w, *bias;
+  void* out;
+  const int32_t* used;
+  int64_t x_batch_stride, x_row_stride, out_batch_stride, out_row_stride;
+  int32_t batch, rows, n, k, accumulate;
+} asrlayer_gemm_params;
+
+int asrlayer_gemm(const asrlayer_gemm_params* params, void* stream);
+
 }  // extern "C"

@@ -197,3 +197,54 @@ def rows_linear(x: Tensor, linears: list[nn.Linear], norm: nn.LayerNorm | None =
     lib = _lib.load()
     _lib.check(lib.asrlayer_rows_linear(ctypes.byref(params), _stream(x.device)), "asrlayer_rows_linear")
     return outs
+
+
+def gemm_takes(x: Tensor, linear: nn.Module) -> bool:
+    """Whether :func:`gemm` takes ``x`` ``(batch, rows, inputs)`` through
+    ``linear`` (bf16)."""
+    if type(linear) is not nn.Linear or x.dim() != 3 or x.dtype != torch.bfloat16 or linear._forward_hooks:
+        return False
+    weight, bias = linear.weight, linear.bias
+    outputs, inputs = weight.shape
+    if inputs % 64 or outputs % 8 or x.shape[2] != inputs or linear._forward_pre_hooks:
+        return False
+    if not (_plain(x, weight) if bias is None else _plain(x, weight, bias)):
+        return False
+    return (_vectors(x) and inputs <= x.stride(1) <= 1 << 22 and weight.is_contiguous() and _vectors(weight)
+            and (bias is None or _vectors(bias)))
+
+
+def gemm_tiles(x: Tensor) -> int:
+    """32 x 32 tiles of a square layer's outputs over ``x`` ``(batch, rows,
+    inputs)``."""
+    batch, rows, inputs = x.shape
+    return -(-batch * rows // 32) * (-(-inputs // 32))
+
+
+def used_takes(used: Tensor, x: Tensor) -> bool:
+    """Whether ``used`` can count the rows of ``x`` ``(batch, rows, inputs)``
+    that :func:`gemm` computes."""
+    return (type(used) is Tensor and used.dtype == torch.int32 and used.shape == x.shape[:1]
+            and used.get_device() == x.get_device() and used.is_contiguous())
+
+
+def gemm(x: Tensor, linear: nn.Linear, used: Tensor | None = None, into: Tensor | None = None) -> Tensor:
+    """``linear(x)`` for bf16 ``x`` ``(batch, rows, inputs)``, or ``into + x
+    @ linear.weight.T`` written to ``into`` (contiguous; no bias), in one
+    launch (``asrlayer_gemm``).  ``used`` (int32 per batch entry): the rows that
+    are computed; the others hold anything (``into``: what they held)."""
+    batch, rows, inputs = x.shape
+    outputs = linear.out_features
+    out = into
+    if into is None:
+        out = torch.empty((batch, rows, outputs), dtype=x.dtype, device=x.device)
+    bias = None if into is not None or linear.bias is None else linear.bias.data_ptr()
+    x_strides, out_strides = x.stride()[:2], out.stride()[:2]
+    if used is None and x_strides[0] == rows * x_strides[1]:
+        batch, rows = 1, batch * rows  # one run of rows: fewer part-filled tiles
+    params = _lib.GemmParams(
+        x.data_ptr(), linear.weight.data_ptr(), bias, out.data_ptr(), None if used is None else used.data_ptr(),
+        *x_strides, *out_strides, batch, rows, outputs, inputs, into is not None)
+    lib = _lib.load()
+    _lib.check(lib.asrlayer_gemm(ctypes.byref(params), _stream(x.device)), "asrlayer_gemm")
+    return out

@@ -31,6 +31,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from .attention import flash_fsmn
+from .layers import gemm, gemm_takes, used_takes
 
 
 class SANMAttention(nn.Module):
@@ -56,11 +57,16 @@ class SANMAttention(nn.Module):
         frames of row b (the frame mask ``sensevoice.py:548-550`` builds), and
         ``lengths`` (int32) counts them; both are None when every frame is
         real."""
-        qkv = self.linear_q_k_v(x)
-        query, key, value = qkv.split(self.size, dim=-1)
         batch, length, _ = x.shape
         if lengths is None and mask is not None:
             lengths = mask.sum(dim=1, dtype=torch.int32)
+        # With zero_padded_rows nothing reads a padded frame's projections, and
+        # its attention adds nothing to its memory: neither is computed where
+        # the kernels run the linear layers.
+        skip = lengths if self.zero_padded_rows else None
+        project = gemm_takes(x, self.linear_q_k_v) and (skip is None or used_takes(skip, x))
+        qkv = gemm(x, self.linear_q_k_v, skip) if project else self.linear_q_k_v(x)
+        query, key, value = qkv.split(self.size, dim=-1)
         shape = (batch, length, self.heads, self.size // self.heads)
         output, memory = flash_fsmn(
             query.view(shape),
@@ -72,6 +78,9 @@ class SANMAttention(nn.Module):
             zero_padded_rows=self.zero_padded_rows and lengths is not None,
         )
         # linear_out(output) + memory: the bias is in memory already.
+        rows = output.view(batch, length, self.size)
+        if project and gemm_takes(rows, self.linear_out):
+            return gemm(rows, self.linear_out, skip, into=memory)
         memory.view(-1, self.size).addmm_(output.view(-1, self.size), self.linear_out.weight.t())
         return memory
 

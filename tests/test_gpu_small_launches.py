@@ -381,3 +381,35 @@ def test_small_sanm_launches(ops, device, frames, batch):
     out, memory = ops.flash_fsmn(q, k, v, weight.to(device), seqused_k=used.to(device), zero_padded_rows=True)
     assert_close(out.float().cpu(), ref, "bf16")
     assert_close(memory.float().cpu(), memory_ref, "bf16")
+
+
+@pytest.mark.parametrize("batch,rows,inputs,outputs", [
+    (1, 1, 64, 8), (1, 33, 192, 40), (3, 17, 512, 512), (1, 300, 512, 1536), (2, 700, 128, 1000), (5, 504, 512, 1536),
+    (1, 1500, 1280, 136)])
+def test_gemm(device, batch, rows, inputs, outputs):
+    """The bf16 linear layer over both tilings and their edges (rows, outputs
+    and reductions that fill no tile), with and without bias, added to what the
+    output holds, over strided rows, and with row counts, whose other rows stay
+    as they were; against float64, one bf16 rounding (2e-2 of the largest)."""
+    from torch import nn
+
+    from asrback_amd import layers
+
+    say("gemm", batch, rows, inputs, outputs)
+    torch.manual_seed(9)
+    linear = nn.Linear(inputs, outputs).to(device, torch.bfloat16).requires_grad_(False)
+    wide = torch.randn(batch, rows, inputs + 64, device=device).to(torch.bfloat16)
+    used = torch.tensor([rows, rows // 2, 0, 1, rows - 1][:batch], dtype=torch.int32, device=device)
+    keep = torch.arange(rows, device=device) < used[:, None]
+    for x in (wide[..., :inputs].contiguous(), wide[..., 64:]):
+        assert layers.gemm_takes(x, linear)
+        ref = x.double() @ linear.weight.double().T.contiguous()
+        got = layers.gemm(x, linear)
+        assert_close(got.float().cpu(), (ref + linear.bias.double()).cpu(), "bf16")
+        part = layers.gemm(x, linear, used)
+        assert torch.equal(part[keep], got[keep])
+        held = torch.randn(batch, rows, outputs, device=device).to(torch.bfloat16)
+        into = held.clone()
+        assert layers.gemm(x, linear, used, into=into) is into
+        assert torch.equal(into[~keep], held[~keep])
+        assert_close(into[keep].float().cpu(), (held.double() + ref)[keep].cpu(), "bf16")
