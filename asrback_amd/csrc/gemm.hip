@@ -8,18 +8,19 @@
 //   * Few rows: a workgroup takes 32 rows x 32 outputs, its four waves a
 //     quarter of the reduction each, operands straight from memory into
 //     registers, eight steps in flight.  A launch is one or two round trips to
-//     memory, which is what bounds it.
-//   * Many rows: 128 rows x 128 outputs, four waves of 64 x 64, 64-deep tiles of
-//     both operands moved into a two-stage LDS ring by DMA (the attention's
-//     ring: chunks rotated within rows, so operand reads are free of bank
-//     conflicts), 64 KB, two workgroups per CU.  Bound by the matrix cores and
-//     their operand reads.
+//     memory, which is what bounds it (sixteen in flight in two register sets:
+//     300 rows of 512 to 1536 outputs 7.2 -> 10.3 us).
+//   * Many rows: 128 rows x 128 or 192 outputs, four waves of 64 rows x half the
+//     outputs, 64-deep tiles of both operands moved into a two-stage LDS ring by
+//     DMA (the attention's ring: chunks rotated within rows, so operand reads
+//     are free of bank conflicts), 64 or 80 KB, two workgroups per CU.  Bound by
+//     the matrix cores, their operand reads and the last round of workgroups.
 //
 // Rows at or past used[b] of batch entry b are neither read nor written:
 // SenseVoice's padded frames (40% of the rows of a batch of 104-504 frames),
 // whose queries, keys and values nothing reads.  32 x 504 frames of 512, 304 of
-// them real on average, to 1536 outputs: 35 us, against 44 for the library's
-// product of all rows (of all rows here: 45); to 512: 14.9 against 16.8.
+// them real on average, to 1536 outputs: 33.5 us, against 44 for the library's
+// product of all rows (of all rows here: 40); to 512: 14.9 against 16.8.
 #include "kernels.hpp"
 #include "layers.hpp"
 #include "ring_common.hpp"
@@ -116,13 +117,15 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const asrlayer_gemm_par
   if (row0 + m < v.rows && n0 + c < p.n) finish<1>(p, y, v.out + (int64_t)(row0 + m) * p.out_row_stride, n0 + c);
 }
 
-// 128 rows x 128 outputs.
-constexpr int kBM = 128, kBN = 128, kBK = 64;
-constexpr int kTileBytes = 128 * kBK * 2;
-constexpr int kStageBytes = 2 * kTileBytes;
-constexpr int kOutRow = 64 + 4;  // staged floats per row of a wave's 32 x 64 half
+// 128 rows x 64 NB outputs.
+constexpr int kBM = 128, kBK = 64;
 
+template <int NB>
 __global__ __launch_bounds__(256, 2) void gemm_large_kernel(const asrlayer_gemm_params p, int row_tiles, int col_tiles) {
+  constexpr int kBN = 64 * NB;
+  constexpr int kTileBytes = kBM * kBK * 2;  // the X tile
+  constexpr int kStageBytes = kTileBytes + kBN * kBK * 2;
+  constexpr int kOutRow = 32 * NB + 4;  // staged floats per row of a wave's 32 rows
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kStageBytes];
   static_assert(4 * 32 * kOutRow * 4 <= 2 * kStageBytes, "the staged outputs fit the ring");
   const int item = xcd_remap((int)blockIdx.x, (int)gridDim.x);
@@ -143,23 +146,27 @@ __global__ __launch_bounds__(256, 2) void gemm_large_kernel(const asrlayer_gemm_
       buffer_rsrc(v.x + (int64_t)row0 * p.x_row_stride, (uint32_t)(min(kBM, v.rows - row0) - 1) * xs + ws);
   const __amdgpu_buffer_rsrc_t wrs =
       buffer_rsrc(static_cast<const bf16_raw*>(p.w) + (int64_t)n0 * p.k, (uint32_t)min(kBN, p.n - n0) * ws);
-  // DMA instruction 4 wave + i of a tile fills rows 8 (4 wave + i) .. + 7, eight
-  // chunks each, the chunk order rotated as the operand reads expect.
-  uint32_t xoff[4], woff[4];
+  // A DMA instruction fills eight rows of eight chunks, the chunk order rotated
+  // as the operand reads expect; wave w takes instructions 4 w .. of the X tile
+  // and 2 NB w .. of the weights'.
+  uint32_t xoff[4], woff[2 * NB];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 8 * (4 * wave + i) + lane / 8;
-    const uint32_t c = (uint32_t)k_logical<64>(r, lane % 8) * 16;
-    xoff[i] = (uint32_t)r * xs + c;
-    woff[i] = (uint32_t)r * ws + c;
+    xoff[i] = (uint32_t)r * xs + (uint32_t)k_logical<64>(r, lane % 8) * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * NB; ++i) {
+    const int r = 8 * (2 * NB * wave + i) + lane / 8;
+    woff[i] = (uint32_t)r * ws + (uint32_t)k_logical<64>(r, lane % 8) * 16;
   }
   auto issue = [&](int t, int stage) {
-    const uint32_t base = lds_base + (uint32_t)stage * kStageBytes + (uint32_t)wave * 4096;
+    const uint32_t base = lds_base + (uint32_t)stage * kStageBytes;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      dma16(xrs, base + i * 1024, xoff[i] + (uint32_t)t * (kBK * 2));
-      dma16(wrs, base + kTileBytes + i * 1024, woff[i] + (uint32_t)t * (kBK * 2));
-    }
+    for (int i = 0; i < 4; ++i) dma16(xrs, base + (uint32_t)(4 * wave + i) * 1024, xoff[i] + (uint32_t)t * (kBK * 2));
+#pragma unroll
+    for (int i = 0; i < 2 * NB; ++i)
+      dma16(wrs, base + kTileBytes + (uint32_t)(2 * NB * wave + i) * 1024, woff[i] + (uint32_t)t * (kBK * 2));
   };
   // Operand addresses in stage 0 (32-row blocks share the rotation).
   uint32_t xaddr[4], waddr[4];
@@ -167,15 +174,15 @@ __global__ __launch_bounds__(256, 2) void gemm_large_kernel(const asrlayer_gemm_
   for (int kk = 0; kk < 4; ++kk) {
     const uint32_t c = (uint32_t)k_phys<64>(r32, 2 * kk + half) * 16;
     xaddr[kk] = (lds_base + (uint32_t)(64 * wm + r32) * (kBK * 2) + c) & 0x3ffffu;
-    waddr[kk] = (lds_base + kTileBytes + (uint32_t)(64 * wn + r32) * (kBK * 2) + c) & 0x3ffffu;
+    waddr[kk] = (lds_base + kTileBytes + (uint32_t)(32 * NB * wn + r32) * (kBK * 2) + c) & 0x3ffffu;
   }
 
   const bool idle = row0 + 64 * wm >= v.rows;  // none of this wave's rows: it moves tiles only
-  f32x16_t acc[2][2];
+  f32x16_t acc[2][NB];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16_t{};
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x16_t{};
   const int tiles = p.k / kBK;
   issue(0, 0);
   auto tile = [&](int t, int stage) {
@@ -188,16 +195,15 @@ __global__ __launch_bounds__(256, 2) void gemm_large_kernel(const asrlayer_gemm_
     const uint32_t so = (uint32_t)stage * kStageBytes;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
-      bf16x8_t x[2], w[2];
+      bf16x8_t x[2], w[NB];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        x[i] = lds_read16(xaddr[kk] + so + i * 32 * kBK * 2);
-        w[i] = lds_read16(waddr[kk] + so + i * 32 * kBK * 2);
-      }
+      for (int i = 0; i < 2; ++i) x[i] = lds_read16(xaddr[kk] + so + i * 32 * kBK * 2);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) w[j] = lds_read16(waddr[kk] + so + j * 32 * kBK * 2);
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = mfma32(w[j], x[i], acc[i][j]);
+        for (int j = 0; j < NB; ++j) acc[i][j] = mfma32(w[j], x[i], acc[i][j]);
     }
   };
   for (int t = 0; t < tiles; t += 2) {
@@ -206,13 +212,13 @@ __global__ __launch_bounds__(256, 2) void gemm_large_kernel(const asrlayer_gemm_
   }
   __syncthreads();  // the ring is free for the outputs
 
-  // 32 rows at a time, through LDS, for stores of 16 bytes a lane and whole
-  // 128-byte row segments.
+  // 32 rows at a time, through LDS, for stores of 16 bytes a lane and 128 bytes
+  // of a row and more.
   float* const stage = reinterpret_cast<float*>(lds) + wave * 32 * kOutRow;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         *reinterpret_cast<float4*>(stage + r32 * kOutRow + 32 * j + 8 * q + 4 * half) =
@@ -221,12 +227,12 @@ __global__ __launch_bounds__(256, 2) void gemm_large_kernel(const asrlayer_gemm_
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int m = s * 8 + lane / 8, c = lane % 8 * 8;
+    for (int s = 0; s < 2 * NB; ++s) {
+      const int ch = s * 64 + lane, m = ch / (4 * NB), c = ch % (4 * NB) * 8;
       const float4 lo = *reinterpret_cast<const float4*>(stage + m * kOutRow + c);
       const float4 hi = *reinterpret_cast<const float4*>(stage + m * kOutRow + c + 4);
       float y[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-      const int row = row0 + 64 * wm + 32 * i + m, n = n0 + 64 * wn + c;
+      const int row = row0 + 64 * wm + 32 * i + m, n = n0 + 32 * NB * wn + c;
       if (row < v.rows && n < p.n) finish<2>(p, y, v.out + (int64_t)row * p.out_row_stride, n);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -245,13 +251,21 @@ hipError_t launch_gemm(const asrlayer_gemm_params& p, hipStream_t stream) {
   // computed: the tilings sum in different orders, and a row's result does not
   // depend on how the batch is padded.
   const bool small = tiles((long long)p.batch * p.rows, 32) * tiles(p.n, 32) <= 1024;
-  const int row_tiles = (int)tiles(p.rows, small ? 32 : kBM), col_tiles = (int)tiles(p.n, small ? 32 : kBN);
+  // 192 outputs a workgroup where they divide the outputs and leave at least a
+  // round of workgroups (two per CU): five operand reads for six products
+  // instead of four for four, and fewer rounds (16128 rows to 1536 outputs 45
+  // -> 40 us).
+  const bool wide = p.n % 192 == 0 && tiles((long long)p.batch * p.rows, kBM) * (p.n / 192) >= 512;
+  const int row_tiles = (int)tiles(p.rows, small ? 32 : kBM);
+  const int col_tiles = (int)tiles(p.n, small ? 32 : wide ? 192 : 128);
   const long long total = (long long)p.batch * row_tiles * col_tiles;
   if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   if (small)
     hipLaunchKernelGGL(gemm_small_kernel, dim3((unsigned)total), dim3(256), 0, stream, p, row_tiles, col_tiles);
+  else if (wide)
+    hipLaunchKernelGGL((gemm_large_kernel<3>), dim3((unsigned)total), dim3(256), 0, stream, p, row_tiles, col_tiles);
   else
-    hipLaunchKernelGGL(gemm_large_kernel, dim3((unsigned)total), dim3(256), 0, stream, p, row_tiles, col_tiles);
+    hipLaunchKernelGGL((gemm_large_kernel<2>), dim3((unsigned)total), dim3(256), 0, stream, p, row_tiles, col_tiles);
   return hipGetLastError();
 }
 
