@@ -1,5 +1,6 @@
 // Multi-row attention in fp32 on the gfx950 matrix cores
-// (v_mfma_f32_32x32x2_f32: fp32 operands, fp32 accumulation).
+// (v_mfma_f32_32x32x2_f32: fp32 operands, fp32 accumulation), head_dim 128, 256
+// and 512; head_dim 64 runs in fwd_f32row.hip.
 //
 // Workgroup: KS waves over one block of 32 query rows of one (sequence,
 // head); wave ks takes the key sub-tiles ks, ks + KS, ... (32 keys each) and
@@ -310,17 +311,12 @@ hipError_t launch_hd(const FwdArgs& a, hipStream_t stream) {
   const int subs = (p.max_len_k + 31) / 32;
   // Key splits: as many waves per row block as the CUs hold at once for
   // all blocks (two per SIMD at 64 dimensions a wave; one at 128, where a wave
-  // needs more than 256 registers), and at least two sub-tiles per split.  A
-  // second round of workgroups would run on few CUs: Whisper-tiny's 282 row
-  // blocks take four splits (1128 waves, one round) in 66 us and took 73.8
-  // with eight (2256 waves, two rounds).
+  // needs more than 256 registers), and at least two sub-tiles per split: a
+  // second round of workgroups would run on few CUs.
   constexpr int kMaxKs = (HD == 64 ? 8 : 4) / DS;
   constexpr long long kResidentWaves = HD == 64 ? 2048 : 1024;
   int ks = 1;
   while (ks < kMaxKs && blocks * 2 * ks * DS <= kResidentWaves && subs >= 4 * ks) ks *= 2;
-  if constexpr (kMaxKs >= 8) {
-    if (ks == 8) return launch_ks<HD, 8, DS, WIN>(a, stream);
-  }
   if constexpr (kMaxKs >= 4) {
     if (ks == 4) return launch_ks<HD, 4, DS, WIN>(a, stream);
   }
@@ -355,7 +351,7 @@ hipError_t launch_fwd_f32mm(const asrattn_fwd_params& p, hipStream_t stream) {
   a.c = p.scale * kLog2e;
   a.f = FsmnArgs{};
   switch (p.head_dim) {
-    case 64: return launch_window<64, 1>(a, stream);
+    case 64: return launch_fwd_f32row(p, stream);
     case 128: return launch_window<128, 1>(a, stream);
     case 256: return launch_window<64, 4>(a, stream);
     default: return launch_window<64, 8>(a, stream);
