@@ -6,17 +6,16 @@
 // one row: 0.6 MB of weights a matrix), by reading the weights at larger
 // ones.  As separate operations a Whisper decoder layer's step took 27
 // launches of 4-5 us each (norm, bias copy, product, activation and sum apart);
-// here it takes six of 4.2 us (a kernel that does nothing takes 1.8), besides
-// its two attention launches: 429 -> 200 us for a whole step of four layers.
+// here it takes six of 3.3-3.8 us (a kernel that does nothing takes 1.8), besides
+// its two attention launches.
 //
-// A workgroup takes kCols weight rows (output columns) and spreads the
-// reduction over its threads: thread t holds vector t (16 bytes) of every
-// input row and of each weight row, all loaded at once, so a launch is one
-// round trip to memory, two reductions over the workgroup for the layer norm
-// (statistics in two passes, in registers), and one for the products.  The
-// weight rows are read in whole cache lines, once for each eight input rows
-// (four where the reduction takes more than 512 threads, whose registers then
-// hold no more).
+// A wave takes two weight rows (output columns) and spreads the reduction over
+// its lanes: a lane holds up to six 16-byte vectors of every input row and of
+// each weight row, all loaded at once, so a launch is one round trip to memory,
+// two sums over the lanes for the layer norm (statistics in two passes, in
+// registers), and one for the products.  The weight rows are read in whole
+// cache lines, once for each four input rows.  Longer reductions take a
+// workgroup, a vector per thread, and sum over it.
 #include "kernels.hpp"
 #include "layers.hpp"
 #include "row_ops.hpp"
@@ -85,6 +84,20 @@ __device__ __forceinline__ int summed_value(int lane) {
   return lane >> (6 - kBits);
 }
 
+// Output column `col` of the launch: the matrix it belongs to and its row.
+struct Column {
+  int matrix, n;
+};
+__device__ __forceinline__ Column column_of(const asrlayer_linear_params& p, int col) {
+  const int n01 = p.n[0] + p.n[1];
+  const int i = col < p.n[0] ? 0 : col < n01 ? 1 : 2;
+  return {i, col - (i == 0 ? 0 : i == 1 ? p.n[0] : n01)};
+}
+template <typename P>
+__device__ __forceinline__ P pick(P const* three, int i) {
+  return i == 0 ? three[0] : i == 1 ? three[1] : three[2];
+}
+
 // Sums v[m] over the workgroup; every thread gets all the sums.
 template <int R>
 __device__ __forceinline__ void sum_workgroup(float* v, float (*sm)[R], int waves, int wave, int lane) {
@@ -103,9 +116,109 @@ __device__ __forceinline__ void sum_workgroup(float* v, float (*sm)[R], int wave
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
-// R: rows of a workgroup, a power of two (rows past the last repeat it).
-template <typename T, int R, int kCols, int kThreads>
-__global__ __launch_bounds__(kThreads) void rows_linear_kernel(const asrlayer_linear_params p) {
+// Bias, activation and residual of one sum, rounded where the separate
+// operations round, and its store.
+template <typename T>
+__device__ __forceinline__ void finish(const asrlayer_linear_params& p, Column c, int row, float y) {
+  const T* bias = static_cast<const T*>(pick(p.b, c.matrix));
+  T* out = static_cast<T*>(pick(p.out, c.matrix));
+  if (bias != nullptr) y += Elem<T>::load1(bias + c.n);
+  if (p.act == 1) y = gelu(round_to<T>(y));
+  if (p.residual != nullptr)
+    y = round_to<T>(y) + Elem<T>::load1(static_cast<const T*>(p.residual) + row * p.r_row_stride + c.n);
+  Elem<T>::store1(out + (int64_t)row * pick(p.n, c.matrix) + c.n, y);
+}
+
+// A wave for kCols columns: every lane holds NV vectors of each row.
+template <typename T, int R, int NV, int kCols>
+__global__ __launch_bounds__(64) void rows_wave_kernel(const asrlayer_linear_params p) {
+  constexpr int EPL = Elem<T>::kPerVec;
+  const int lane = threadIdx.x;
+  const int vecs = p.k / EPL;
+  const int columns = p.n[0] + p.n[1] + p.n[2];
+  const int col0 = blockIdx.x * kCols, row0 = blockIdx.y * R;
+  uint4 x[R][NV], w[kCols][NV], lw[NV], lb[NV];
+  const bool norm = p.ln_weight != nullptr;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int at = min(v * 64 + lane, vecs - 1) * EPL;
+#pragma unroll
+    for (int m = 0; m < R; ++m)
+      x[m][v] = *reinterpret_cast<const uint4*>(static_cast<const T*>(p.x) + min(row0 + m, p.rows - 1) * p.x_row_stride + at);
+#pragma unroll
+    for (int c = 0; c < kCols; ++c) {
+      const Column k = column_of(p, min(col0 + c, columns - 1));
+      w[c][v] = *reinterpret_cast<const uint4*>(static_cast<const T*>(pick(p.w, k.matrix)) + (int64_t)k.n * p.k + at);
+    }
+    // Without a norm these repeat a weight row (and are unused).
+    const T* lwp = static_cast<const T*>(norm ? p.ln_weight : p.w[0]);
+    const T* lbp = static_cast<const T*>(norm ? p.ln_bias : p.w[0]);
+    lw[v] = *reinterpret_cast<const uint4*>(lwp + at);
+    lb[v] = *reinterpret_cast<const uint4*>(lbp + at);
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+    if (v * 64 + lane >= vecs) {
+#pragma unroll
+      for (int m = 0; m < R; ++m) x[m][v] = make_uint4(0u, 0u, 0u, 0u);
+    }
+  if (norm) {
+    const float inv_k = 1.f / (float)p.k;
+#pragma unroll
+    for (int m = 0; m < R; ++m) {
+      float sum = 0.f;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        float f[EPL];
+        unpack<T>(x[m][v], f);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) sum += f[e];
+      }
+      const float mean = group_sum<64>(sum) * inv_k;
+      float var = 0.f;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        float f[EPL];
+        unpack<T>(x[m][v], f);
+        float part = 0.f;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) part = fmaf(f[e] - mean, f[e] - mean, part);
+        var += v * 64 + lane < vecs ? part : 0.f;
+      }
+      const float r = rsqrtf(group_sum<64>(var) * inv_k + p.ln_eps);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        float f[EPL], g[EPL], b[EPL];
+        unpack<T>(x[m][v], f);
+        unpack<T>(lw[v], g);
+        unpack<T>(lb[v], b);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) f[e] = fmaf((f[e] - mean) * r, g[e], b[e]);
+        const uint4 y = pack<T>(f);
+        x[m][v] = v * 64 + lane < vecs ? y : make_uint4(0u, 0u, 0u, 0u);
+      }
+    }
+  }
+  float acc[kCols * R];
+#pragma unroll
+  for (int c = 0; c < kCols; ++c)
+#pragma unroll
+    for (int m = 0; m < R; ++m) {
+      float y = dot_vec<T>(x[m][0], w[c][0]);
+#pragma unroll
+      for (int v = 1; v < NV; ++v) y += dot_vec<T>(x[m][v], w[c][v]);
+      acc[c * R + m] = y;
+    }
+  sum_lanes<kCols * R, 32>(acc, lane);
+  const int i = summed_value<kCols * R>(lane);
+  const int col = col0 + i / R, row = row0 + i % R;
+  if (lane % (64 / (kCols * R)) == 0 && col < columns && row < p.rows) finish<T>(p, column_of(p, col), row, acc[0]);
+}
+
+// A workgroup for kCols columns, a vector per thread.  R: rows of a workgroup, a
+// power of two (rows past the last repeat it).
+template <typename T, int R, int kCols>
+__global__ __launch_bounds__(1024) void rows_linear_kernel(const asrlayer_linear_params p) {
   constexpr int EPL = Elem<T>::kPerVec;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -118,7 +231,7 @@ __global__ __launch_bounds__(kThreads) void rows_linear_kernel(const asrlayer_li
   __shared__ float sm_dot[kMaxWaves][kCols][R];
 
   // The column's weight row: matrices one after another.
-  const int n01 = p.n[0] + p.n[1], columns = n01 + p.n[2];
+  const int columns = p.n[0] + p.n[1] + p.n[2];
   const int col0 = blockIdx.x * kCols, row0 = blockIdx.y * R;
   uint4 x[R], w[kCols], lw = {}, lb = {};
 #pragma unroll
@@ -132,10 +245,8 @@ __global__ __launch_bounds__(kThreads) void rows_linear_kernel(const asrlayer_li
 #pragma unroll
   for (int c = 0; c < kCols; ++c) {
     const int col = min(col0 + c, columns - 1);
-    const int i = col < p.n[0] ? 0 : col < n01 ? 1 : 2;
-    const int n = col - (i == 0 ? 0 : i == 1 ? p.n[0] : n01);
-    const void* wp = i == 0 ? p.w[0] : i == 1 ? p.w[1] : p.w[2];
-    w[c] = *reinterpret_cast<const uint4*>(static_cast<const T*>(wp) + (int64_t)n * p.k + at);
+    const Column k = column_of(p, col);
+    w[c] = *reinterpret_cast<const uint4*>(static_cast<const T*>(pick(p.w, k.matrix)) + (int64_t)k.n * p.k + at);
   }
   if (!mine) {
 #pragma unroll
@@ -198,28 +309,35 @@ __global__ __launch_bounds__(kThreads) void rows_linear_kernel(const asrlayer_li
     const int c = tid % kCols, m = tid / kCols, row = row0 + m;
     const int col = col0 + c;
     if (col < columns && row < p.rows) {
-      const int i = col < p.n[0] ? 0 : col < n01 ? 1 : 2;
-      const int n = col - (i == 0 ? 0 : i == 1 ? p.n[0] : n01);
-      const T* bias = static_cast<const T*>(i == 0 ? p.b[0] : i == 1 ? p.b[1] : p.b[2]);
-      T* out = static_cast<T*>(i == 0 ? p.out[0] : i == 1 ? p.out[1] : p.out[2]);
       float y = 0.f;
       for (int v = 0; v < waves; ++v) y += sm_dot[v][c][m];
-      if (bias != nullptr) y += Elem<T>::load1(bias + n);
-      // Rounded where the separate operations round.
-      if (p.act == 1) y = gelu(round_to<T>(y));
-      if (p.residual != nullptr)
-        y = round_to<T>(y) + Elem<T>::load1(static_cast<const T*>(p.residual) + row * p.r_row_stride + n);
-      Elem<T>::store1(out + (int64_t)row * p.n[i == 0 ? 0 : i == 1 ? 1 : 2] + n, y);
+      finish<T>(p, column_of(p, col), row, y);
     }
   }
 }
 
-template <typename T, int R, int kThreads>
+template <typename T, int R, int NV>
+hipError_t launch_wave(const asrlayer_linear_params& p, hipStream_t stream) {
+  const int columns = p.n[0] + p.n[1] + p.n[2];
+  constexpr int kCols = 2;
+  hipLaunchKernelGGL((rows_wave_kernel<T, R, NV, kCols>), dim3((columns + kCols - 1) / kCols, (p.rows + R - 1) / R),
+                     dim3(64), 0, stream, p);
+  return hipGetLastError();
+}
+
+template <typename T, int NV>
+hipError_t launch_wave_rows(const asrlayer_linear_params& p, hipStream_t stream) {
+  if (p.rows <= 1) return launch_wave<T, 1, NV>(p, stream);
+  if (p.rows <= 2) return launch_wave<T, 2, NV>(p, stream);
+  return launch_wave<T, 4, NV>(p, stream);
+}
+
+template <typename T, int R>
 hipError_t launch_rows(const asrlayer_linear_params& p, int threads, hipStream_t stream) {
   const int columns = p.n[0] + p.n[1] + p.n[2];
   constexpr int kCols = 4;
   static_assert(kCols * R <= 64, "an output per thread of one wave");
-  hipLaunchKernelGGL((rows_linear_kernel<T, R, kCols, kThreads>), dim3((columns + kCols - 1) / kCols, (p.rows + R - 1) / R),
+  hipLaunchKernelGGL((rows_linear_kernel<T, R, kCols>), dim3((columns + kCols - 1) / kCols, (p.rows + R - 1) / R),
                      dim3(threads), 0, stream, p);
   return hipGetLastError();
 }
@@ -227,15 +345,17 @@ hipError_t launch_rows(const asrlayer_linear_params& p, int threads, hipStream_t
 template <typename T>
 hipError_t launch_typed(const asrlayer_linear_params& p, hipStream_t stream) {
   const int threads = (p.k / Elem<T>::kPerVec + 63) / 64 * 64;
-  if (threads > 512) {
-    if (p.rows <= 1) return launch_rows<T, 1, 1024>(p, threads, stream);
-    if (p.rows <= 2) return launch_rows<T, 2, 1024>(p, threads, stream);
-    return launch_rows<T, 4, 1024>(p, threads, stream);
-  }
-  if (p.rows <= 1) return launch_rows<T, 1, 512>(p, threads, stream);
-  if (p.rows <= 2) return launch_rows<T, 2, 512>(p, threads, stream);
-  if (p.rows <= 4) return launch_rows<T, 4, 512>(p, threads, stream);
-  return launch_rows<T, 8, 512>(p, threads, stream);
+  // A wave per column pair up to six vectors a lane (what its registers hold
+  // for four rows): one row through 384 x 1152 float32 with the norm 4.7 -> 3.5
+  // us against a workgroup per four columns, eight rows 6.0 -> 4.7; 1536 x 384
+  // 4.1 -> 3.8, 1280 x 1280 bf16 with the norm 5.1 -> 4.0.
+  if (threads <= 64) return launch_wave_rows<T, 1>(p, stream);
+  if (threads <= 128) return launch_wave_rows<T, 2>(p, stream);
+  if (threads <= 192) return launch_wave_rows<T, 3>(p, stream);
+  if (threads <= 384) return launch_wave_rows<T, 6>(p, stream);
+  if (p.rows <= 1) return launch_rows<T, 1>(p, threads, stream);
+  if (p.rows <= 2) return launch_rows<T, 2>(p, threads, stream);
+  return launch_rows<T, 4>(p, threads, stream);
 }
 
 }  // namespace
