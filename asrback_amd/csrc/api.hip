@@ -464,11 +464,9 @@ int asrlayer_prompt_rows(const asrlayer_prompt_params* params, void* stream) {
   if (p.batch < 0 || p.tokens < 0 || p.heads_q <= 0 || (p.k != nullptr && p.heads_kv <= 0))
     return fail(ASRATTN_ERR_INVALID, "batch and tokens must be >= 0, the head counts positive");
   if (p.batch == 0 || p.tokens == 0) return ok();
-  const long long rows = (long long)p.heads_q + (p.k != nullptr ? 2LL * p.heads_kv : 0LL);
-  const long long tokens = (long long)p.batch * p.tokens;
-  // Rows are counted in 32 bits, up to a workgroup's past the last.
-  if (tokens > 0x7fffffffLL - 1024 || rows > (0x7fffffffLL - 1024) / tokens)
-    return fail(ASRATTN_ERR_UNSUPPORTED, "more than 2^31 rows");
+  if ((long long)p.batch * p.tokens > 0x7fffffffLL) return fail(ASRATTN_ERR_UNSUPPORTED, "more than 2^31 tokens");
+  if (p.heads_q > (1 << 24) || (p.k != nullptr && p.heads_kv > (1 << 24)))
+    return fail(ASRATTN_ERR_UNSUPPORTED, "more than 2^24 heads");
   if (p.q == nullptr || p.q_out == nullptr || p.q_norm == nullptr || p.cos == nullptr || p.sin == nullptr ||
       (p.k != nullptr && (p.v == nullptr || p.k_norm == nullptr || p.k_out == nullptr)) ||
       (p.k_cache == nullptr) != (p.v_cache == nullptr) || (p.k_cache != nullptr && (p.k == nullptr || p.rows == nullptr)))
@@ -485,8 +483,7 @@ int asrlayer_prompt_rows(const asrlayer_prompt_params* params, void* stream) {
       (p.k_cache != nullptr && (!vec_aligned(p.k_cache, p.dtype, {p.kc_row_stride, p.kc_pos_stride, p.kc_head_stride}) ||
                                 !vec_aligned(p.v_cache, p.dtype, {p.vc_row_stride, p.vc_pos_stride, p.vc_head_stride}))))
     return fail(ASRATTN_ERR_INVALID, "tensors need 16-byte aligned pointers and strides that are multiples of 16 bytes");
-  return from_hip(asrattn::launch_prompt_rows(p, (uint32_t)(tokens * rows), static_cast<hipStream_t>(stream)),
-                  "asrlayer_prompt_rows");
+  return from_hip(asrattn::launch_prompt_rows(p, static_cast<hipStream_t>(stream)), "asrlayer_prompt_rows");
 }
 
 int asrlayer_rows_linear(const asrlayer_linear_params* params, void* stream) {

@@ -67,9 +67,8 @@ size_t local_lds_bytes(const asrattn_local_params& p);
 // counts p.seqused_k).
 hipError_t launch_fsmn(const asrattn_fwd_params& p, const FsmnArgs& f, hipStream_t stream);
 
-// A prompt pass's rows (asrlayer_prompt_rows; head_dim 64, 128, 256 or 512),
-// total = batch * tokens * (heads_q + 2 heads_kv) of them.
-hipError_t launch_prompt_rows(const asrlayer_prompt_params& p, uint32_t total, hipStream_t stream);
+// A prompt pass's rows (asrlayer_prompt_rows; head_dim 64, 128, 256 or 512).
+hipError_t launch_prompt_rows(const asrlayer_prompt_params& p, hipStream_t stream);
 
 // A decoder step's linear layers over few rows (asrlayer_rows_linear).
 hipError_t launch_rows_linear(const asrlayer_linear_params& p, hipStream_t stream);

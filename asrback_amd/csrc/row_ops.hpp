@@ -44,6 +44,16 @@ __device__ __forceinline__ float round_to(float x) {
   return x;
 }
 
+// The same for two values (one conversion instruction in bf16).
+template <typename T>
+__device__ __forceinline__ void round_pair(float& a, float& b) {
+  if constexpr (sizeof(T) == 2) {
+    const uint32_t u = pack_bf16x2(a, b);
+    a = bf16_lo(u);
+    b = bf16_hi(u);
+  }
+}
+
 // The values of lane l ^ (LPK / 2): a row rotation for 16-lane rows, else
 // through the LDS crossbar.
 template <int LPK>
@@ -79,9 +89,12 @@ __device__ __forceinline__ uint4 prologue_row(uint4 raw, bool any_norm, bool nor
     float wv[EPL];
     unpack<T>(w, wv);
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      const float y = round_to<T>(weighted ? x[e] * r * wv[e] : x[e] * r);
-      x[e] = norm ? y : x[e];
+    for (int e = 0; e < EPL; e += 2) {
+      float a = weighted ? x[e] * r * wv[e] : x[e] * r;
+      float b = weighted ? x[e + 1] * r * wv[e + 1] : x[e + 1] * r;
+      round_pair<T>(a, b);
+      x[e] = norm ? a : x[e];
+      x[e + 1] = norm ? b : x[e + 1];
     }
   }
   if (any_rot) {
@@ -92,9 +105,9 @@ __device__ __forceinline__ uint4 prologue_row(uint4 raw, bool any_norm, bool nor
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
       const float partner = half_row_partner<LPK>(x[e]);
-      const float rot = lower ? -partner : partner;
-      const float y = round_to<T>(round_to<T>(x[e] * cv[e]) + round_to<T>(rot * sv[e]));
-      x[e] = rotated ? y : x[e];
+      float a = x[e] * cv[e], b = (lower ? -partner : partner) * sv[e];
+      round_pair<T>(a, b);
+      x[e] = rotated ? a + b : x[e];
     }
   }
   return pack<T>(x);
