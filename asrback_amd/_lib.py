@@ -257,6 +257,16 @@ class LinearParams(ctypes.Structure):
     ]
 
 
+class EmbedParams(ctypes.Structure):
+    """``asrlayer_embed_params`` (csrc/layers.hpp)."""
+
+    _fields_ = [
+        *[(name, _ptr) for name in ("token_weight", "position_weight", "tokens", "positions", "out")],
+        *[(name, _i64) for name in ("token_stride", "vocab", "length")],
+        *[(name, _i32) for name in ("rows", "width", "dtype")],
+    ]
+
+
 class GemmParams(ctypes.Structure):
     """``asrlayer_gemm_params`` (csrc/layers.hpp)."""
 
@@ -269,6 +279,7 @@ class GemmParams(ctypes.Structure):
 
 # The layers' own entry points (csrc/layers.hpp).
 LAYER_SIGNATURES = {
+    "asrlayer_embed_rows": (ctypes.c_int, [ctypes.POINTER(EmbedParams), _ptr]),
     "asrlayer_gemm": (ctypes.c_int, [ctypes.POINTER(GemmParams), _ptr]),
     "asrlayer_rows_linear": (ctypes.c_int, [ctypes.POINTER(LinearParams), _ptr]),
     "asrlayer_prompt_rows": (ctypes.c_int, [ctypes.POINTER(PromptParams), _ptr]),

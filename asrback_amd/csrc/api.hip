@@ -512,6 +512,20 @@ int asrlayer_rows_linear(const asrlayer_linear_params* params, void* stream) {
   return from_hip(asrattn::launch_rows_linear(p, static_cast<hipStream_t>(stream)), "asrlayer_rows_linear");
 }
 
+int asrlayer_embed_rows(const asrlayer_embed_params* params, void* stream) {
+  if (params == nullptr) return fail(ASRATTN_ERR_INVALID, "params is NULL");
+  const asrlayer_embed_params& p = *params;
+  if (p.dtype != ASRATTN_F32 && p.dtype != ASRATTN_BF16) return fail(ASRATTN_ERR_INVALID, "dtype %d", p.dtype);
+  if (p.rows < 0 || p.width <= 0 || p.vocab <= 0 || p.length <= 0)
+    return fail(ASRATTN_ERR_INVALID, "rows must be >= 0, width, vocab and length positive");
+  if (p.rows == 0) return ok();
+  if (p.token_weight == nullptr || p.position_weight == nullptr || p.tokens == nullptr || p.positions == nullptr ||
+      p.out == nullptr || !vec_aligned(p.token_weight, p.dtype, {p.width}) ||
+      !vec_aligned(p.position_weight, p.dtype, {}) || !vec_aligned(p.out, p.dtype, {}))
+    return fail(ASRATTN_ERR_INVALID, "tables and out must be non-NULL, 16-byte aligned, of whole 16-byte vectors");
+  return from_hip(asrattn::launch_embed_rows(p, static_cast<hipStream_t>(stream)), "asrlayer_embed_rows");
+}
+
 int asrlayer_gemm(const asrlayer_gemm_params* params, void* stream) {
   if (params == nullptr) return fail(ASRATTN_ERR_INVALID, "params is NULL");
   const asrlayer_gemm_params& p = *params;

@@ -73,6 +73,9 @@ hipError_t launch_prompt_rows(const asrlayer_prompt_params& p, hipStream_t strea
 // A decoder step's linear layers over few rows (asrlayer_rows_linear).
 hipError_t launch_rows_linear(const asrlayer_linear_params& p, hipStream_t stream);
 
+// Token and position embeddings of a decoder step (asrlayer_embed_rows).
+hipError_t launch_embed_rows(const asrlayer_embed_params& p, hipStream_t stream);
+
 // A linear layer over bf16 rows (asrlayer_gemm).
 hipError_t launch_gemm(const asrlayer_gemm_params& p, hipStream_t stream);
 

@@ -82,6 +82,20 @@ typedef struct asrlayer_linear_params {
 
 int asrlayer_rows_linear(const asrlayer_linear_params* params, void* stream);
 
+// A decoder step's input: out[r] = token_weight[tokens[r * token_stride]] +
+// position_weight[positions[r]], tables (vocab, width) and (length, width), all
+// contiguous; rows whose token or position lies outside are NaN.  width a
+// multiple of 16 bytes.
+typedef struct asrlayer_embed_params {
+  const void *token_weight, *position_weight;
+  const int64_t *tokens, *positions;
+  void* out;
+  int64_t token_stride, vocab, length;
+  int32_t rows, width, dtype;
+} asrlayer_embed_params;
+
+int asrlayer_embed_rows(const asrlayer_embed_params* params, void* stream);
+
 // A linear layer over bf16 rows (batch x rows of k inputs, n outputs each):
 //
 //   out[b, t, :] = x[b, t, :] w^T + bias        (accumulate 0; bias or NULL)

@@ -199,6 +199,67 @@ def rows_linear(x: Tensor, linears: list[nn.Linear], norm: nn.LayerNorm | None =
     return outs
 
 
+# A vocabulary product (51865 outputs) takes up to two rows, and more of the
+# short ones: float rows of 768, 1: 46.2 -> 30.6 us, 4: 36.0 -> 32.0; of 1280, 1:
+# 72.4 -> 46.5, 4: 53.7 -> 55.9; bf16 rows of 384, 4: 13.2 -> 10.1, of 768, 4:
+# 16.9 -> 17.5.  Float rows' worst error against float64 is 5 times smaller (sums
+# of vectors, then trees).
+PRODUCT_ROWS, PRODUCT_VALUES = 4, 2560
+
+
+def rows_product_takes(x: Tensor, weight: Tensor) -> bool:
+    """Whether :func:`rows_product` takes ``x`` ``(rows, inputs)`` and ``weight``
+    ``(outputs, inputs)``."""
+    if not _plain(x, weight) or x.dim() != 2 or weight.dim() != 2 or not 1 <= x.shape[0] <= PRODUCT_ROWS:
+        return False
+    inputs, per = weight.shape[1], _VECTOR // x.element_size()
+    return (x.shape[1] == inputs and x.shape[0] * inputs <= PRODUCT_VALUES and inputs % per == 0 and 0 < inputs // per <= 384 and weight.shape[0] > 0
+            and _vectors(x) and weight.is_contiguous() and _vectors(weight))
+
+
+def rows_product(x: Tensor, weight: Tensor) -> Tensor:
+    """``x @ weight.T`` for a step's few rows (``asrlayer_rows_linear``)."""
+    (rows, inputs), outputs = x.shape, weight.shape[0]
+    out = torch.empty((rows, outputs), dtype=x.dtype, device=x.device)
+    params = _lib.LinearParams()
+    params.x, params.x_row_stride = x.data_ptr(), x.stride(0)
+    params.w[0], params.out[0], params.n[0] = weight.data_ptr(), out.data_ptr(), outputs
+    params.rows, params.k, params.dtype = rows, inputs, _DTYPES[x.dtype]
+    lib = _lib.load()
+    _lib.check(lib.asrlayer_rows_linear(ctypes.byref(params), _stream(x.device)), "asrlayer_rows_linear")
+    return out
+
+
+def embed_rows_takes(tokens: Tensor, positions: Tensor, token_table: nn.Module, position_table: nn.Module) -> bool:
+    """Whether :func:`embed_rows` takes ``tokens`` ``(rows, 1)`` and
+    ``positions`` ``(rows,)`` through these embeddings."""
+    tables = (token_table, position_table)
+    if any(type(m) is not nn.Embedding or m.max_norm is not None for m in tables) or not unhooked(*tables):
+        return False
+    a, b = token_table.weight, position_table.weight
+    if not _plain(a, b) or a.shape[1] != b.shape[1] or a.shape[1] % (_VECTOR // a.element_size()):
+        return False
+    if not (a.is_contiguous() and b.is_contiguous() and _vectors(a) and _vectors(b)):
+        return False
+    return (type(tokens) is Tensor and type(positions) is Tensor and tokens.dtype == positions.dtype == torch.int64
+            and tokens.dim() == 2 and tokens.shape[1] == 1 and positions.shape == tokens.shape[:1]
+            and len(positions) > 0 and positions.is_contiguous()
+            and tokens.get_device() == positions.get_device() == a.get_device())
+
+
+def embed_rows(tokens: Tensor, positions: Tensor, token_table: nn.Embedding, position_table: nn.Embedding) -> Tensor:
+    """``token_table(tokens) + position_table(positions)[:, None]`` for a
+    decoder step, in one launch (``asrlayer_embed_rows``)."""
+    a, b = token_table.weight, position_table.weight
+    rows, width = tokens.shape[0], a.shape[1]
+    out = torch.empty((rows, 1, width), dtype=a.dtype, device=a.device)
+    params = _lib.EmbedParams(a.data_ptr(), b.data_ptr(), tokens.data_ptr(), positions.data_ptr(), out.data_ptr(),
+                              tokens.stride(0), a.shape[0], b.shape[0], rows, width, _DTYPES[a.dtype])
+    lib = _lib.load()
+    _lib.check(lib.asrlayer_embed_rows(ctypes.byref(params), _stream(a.device)), "asrlayer_embed_rows")
+    return out
+
+
 def gemm_takes(x: Tensor, linear: nn.Module) -> bool:
     """Whether :func:`gemm` takes ``x`` ``(batch, rows, inputs)`` through
     ``linear`` (bf16)."""

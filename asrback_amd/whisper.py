@@ -32,7 +32,10 @@ from torch import Tensor, nn
 
 from . import attention
 from .attention import KeyPrefix, decode_append, greedy_choice, sdpa
-from .layers import gemm, gemm_takes, gemm_tiles, rows_linear, rows_linear_takes
+from .layers import (
+    embed_rows, embed_rows_takes, gemm, gemm_takes, gemm_tiles, rows_linear, rows_linear_takes, rows_product,
+    rows_product_takes,
+)
 from .transcription import CapturedGraph, to_device
 
 # Key buckets of the graphed decoder step; max_target_positions is the last
@@ -285,7 +288,10 @@ class WhisperDecoder(nn.Module):
         if length is None:
             # Graphed step over the bucket's cache view: row b is at
             # positions[b] and sees keys 0 .. positions[b] (read on the device).
-            x = self.embed_tokens(tokens) + self.embed_positions(positions)[:, None]
+            if embed_rows_takes(tokens, positions, self.embed_tokens, self.embed_positions):
+                x = embed_rows(tokens, positions, self.embed_tokens, self.embed_positions)
+            else:
+                x = self.embed_tokens(tokens) + self.embed_positions(positions)[:, None]
             mask = KeyPrefix(positions=positions)
         else:
             x = self.embed_tokens(tokens) + self.embed_positions(positions)
@@ -341,6 +347,8 @@ class WhisperForConditionalGeneration(nn.Module):
     def logits(self, hidden: Tensor) -> Tensor:
         weight = self.model.decoder.embed_tokens.weight
         rows = hidden.flatten(0, -2)
+        if rows_product_takes(rows, weight):
+            return rows_product(rows, weight).unflatten(0, hidden.shape[:-1])
         return (weight @ rows.T).T.unflatten(0, hidden.shape[:-1])
 
 

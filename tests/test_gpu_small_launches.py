@@ -289,6 +289,49 @@ def test_rows_linear(device, dtype, rows, inputs, outputs):
         assert_close(out.cpu(), (residual.double() + exact(linears[0], use_norm)).cpu(), KIND[dtype])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,inputs,outputs", [(1, 8, 16384), (1, 1280, 16387), (2, 384, 16389), (2, 1280, 16391),
+                                                 (3, 520, 20001), (4, 640, 51865)])
+def test_vocabulary_product(device, dtype, rows, inputs, outputs):
+    """Few rows through a vocabulary's weights (eight or four columns a wave,
+    counts that fill no wave), against float64: float32 sums of k products
+    (1e-5), or one rounding (2e-2)."""
+    from asrback_amd import layers
+
+    say("vocabulary product", dtype, rows, inputs, outputs)
+    torch.manual_seed(9)
+    x = torch.randn(rows, inputs, device=device).to(dtype)
+    weight = torch.randn(outputs, inputs, device=device).to(dtype)
+    assert layers.rows_product_takes(x, weight)
+    assert not layers.rows_product_takes(x[:, 1:], weight[:, 1:])
+    assert not layers.rows_product_takes(x.requires_grad_(dtype == torch.float32), weight.t().contiguous().t())
+    assert_close(layers.rows_product(x.detach(), weight).cpu(), (x.double() @ weight.double().t()).detach().cpu(),
+                 KIND[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,width", [(1, 8), (3, 384), (17, 1280), (2, 2056)])
+def test_step_embeddings(device, dtype, rows, width):
+    """The sum of token and position embeddings, to the bit, for tokens that
+    are a column of a longer table; rows outside the tables are NaN."""
+    from torch import nn
+
+    from asrback_amd import layers
+
+    torch.manual_seed(10)
+    tables = [nn.Embedding(n, width).to(device, dtype).requires_grad_(False) for n in (101, 40)]
+    tokens = torch.randint(101, (rows, 5), device=device)[:, 2:3]
+    positions = torch.randint(40, (rows,), device=device)
+    assert layers.embed_rows_takes(tokens, positions, *tables)
+    got = layers.embed_rows(tokens, positions, *tables)
+    assert torch.equal(got, tables[0](tokens) + tables[1](positions)[:, None])
+    for bad in (tokens.int(), tokens.expand(rows, 2), tokens[:, 0], tokens.cpu()):
+        assert not layers.embed_rows_takes(bad, positions, *tables)
+    positions[0] = 40
+    got = layers.embed_rows(tokens, positions, *tables)
+    assert bool(got[0].isnan().all()) and not bool(got[1:].isnan().any())
+
+
 def test_rows_linear_leaves_other_programs_to_the_ops(device):
     """Inputs whose ops something has to see, or the kernel does not address."""
     from torch import nn
