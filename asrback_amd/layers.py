@@ -15,6 +15,7 @@ import math
 
 import torch
 from torch import Tensor, nn
+from torch.nn.modules import module as _module
 
 from . import _lib
 from .attention import _DTYPES, _stream
@@ -25,8 +26,8 @@ _VECTOR = 16  # bytes per lane access
 def _plain(*tensors: Tensor) -> bool:
     """Whether the kernels may read these tensors in place of PyTorch ops:
     ordinary ROCm tensors of one supported dtype, on the current device, with
-    nothing (autograd, forward-mode, autocast, functorch, dispatch modes,
-    tracing) that has to see the ops."""
+    nothing (autograd, forward-mode, autocast, functorch, function and
+    dispatch modes, tracing) that has to see the ops."""
     first = tensors[0]
     dtype, index = first.dtype, first.get_device()
     if dtype not in _DTYPES or not first.is_cuda or index != torch.cuda.current_device():
@@ -39,7 +40,7 @@ def _plain(*tensors: Tensor) -> bool:
             return False
     return not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
                 or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
-                or torch._C._functorch.maybe_current_level() is not None)
+                or torch._C._len_torch_function_stack() or torch._C._functorch.maybe_current_level() is not None)
 
 
 def _vectors(t: Tensor) -> bool:
@@ -52,7 +53,10 @@ def _vectors(t: Tensor) -> bool:
 
 
 def unhooked(*modules: nn.Module) -> bool:
-    return not any(m._forward_hooks or m._forward_pre_hooks for m in modules)
+    """Whether a call of each module is its class's ``forward`` and nothing else."""
+    if _module._global_forward_hooks or _module._global_forward_pre_hooks:
+        return False
+    return not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in modules)
 
 
 def _strides(t: Tensor) -> tuple[int, int, int]:
@@ -213,8 +217,9 @@ def rows_product_takes(x: Tensor, weight: Tensor) -> bool:
     if not _plain(x, weight) or x.dim() != 2 or weight.dim() != 2 or not 1 <= x.shape[0] <= PRODUCT_ROWS:
         return False
     inputs, per = weight.shape[1], _VECTOR // x.element_size()
-    return (x.shape[1] == inputs and x.shape[0] * inputs <= PRODUCT_VALUES and inputs % per == 0 and 0 < inputs // per <= 384 and weight.shape[0] > 0
-            and _vectors(x) and weight.is_contiguous() and _vectors(weight))
+    return (x.shape[1] == inputs and 0 < x.shape[0] * inputs <= PRODUCT_VALUES and inputs % per == 0
+            and inputs // per <= 384 and weight.shape[0] > 0 and _vectors(x) and weight.is_contiguous()
+            and _vectors(weight))
 
 
 def rows_product(x: Tensor, weight: Tensor) -> Tensor:
@@ -263,11 +268,11 @@ def embed_rows(tokens: Tensor, positions: Tensor, token_table: nn.Embedding, pos
 def gemm_takes(x: Tensor, linear: nn.Module) -> bool:
     """Whether :func:`gemm` takes ``x`` ``(batch, rows, inputs)`` through
     ``linear`` (bf16)."""
-    if type(linear) is not nn.Linear or x.dim() != 3 or x.dtype != torch.bfloat16 or linear._forward_hooks:
+    if type(linear) is not nn.Linear or x.dim() != 3 or x.dtype != torch.bfloat16:
         return False
     weight, bias = linear.weight, linear.bias
     outputs, inputs = weight.shape
-    if inputs % 64 or outputs % 8 or x.shape[2] != inputs or linear._forward_pre_hooks:
+    if inputs % 64 or outputs % 8 or x.shape[2] != inputs or not unhooked(linear):
         return False
     if not (_plain(x, weight) if bias is None else _plain(x, weight, bias)):
         return False

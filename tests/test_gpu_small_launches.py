@@ -358,6 +358,14 @@ def test_rows_linear_leaves_other_programs_to_the_ops(device):
         hook = norm.register_forward_hook(lambda *a: None)
         assert not takes()
         hook.remove()
+        hook = nn.modules.module.register_module_forward_hook(lambda *a: None)
+        assert not takes()
+        hook.remove()
+        linear.forward = lambda t: t
+        assert not takes()
+        del linear.forward
+        with torch.device("cuda"):  # a function mode
+            assert not takes()
         assert takes()
 
 
