@@ -56,7 +56,10 @@ def unhooked(*modules: nn.Module) -> bool:
     """Whether a call of each module is its class's ``forward`` and nothing else."""
     if _module._global_forward_hooks or _module._global_forward_pre_hooks:
         return False
-    return not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in modules)
+    for m in modules:
+        if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+            return False
+    return True
 
 
 def _strides(t: Tensor) -> tuple[int, int, int]:
