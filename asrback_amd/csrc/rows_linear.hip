@@ -129,10 +129,13 @@ __device__ __forceinline__ void finish(const asrlayer_linear_params& p, Column c
   Elem<T>::store1(out + (int64_t)row * pick(p.n, c.matrix) + c.n, y);
 }
 
-// A wave for kCols columns: every lane holds NV vectors of each row.
+// A wave for kCols columns: every lane holds NV vectors of each row, the first
+// kFull of which lie in the row whatever its length (the launch takes the
+// smallest of 1, 2, 3 and 6 that holds it).
 template <typename T, int R, int NV, int kCols>
 __global__ __launch_bounds__(64) void rows_wave_kernel(const asrlayer_linear_params p) {
   constexpr int EPL = Elem<T>::kPerVec;
+  constexpr int kFull = NV == 6 ? 3 : NV - 1;
   const int lane = threadIdx.x;
   const int vecs = p.k / EPL;
   const int columns = p.n[0] + p.n[1] + p.n[2];
@@ -157,7 +160,7 @@ __global__ __launch_bounds__(64) void rows_wave_kernel(const asrlayer_linear_par
     lb[v] = *reinterpret_cast<const uint4*>(lbp + at);
   }
 #pragma unroll
-  for (int v = 0; v < NV; ++v)
+  for (int v = kFull; v < NV; ++v)
     if (v * 64 + lane >= vecs) {
 #pragma unroll
       for (int m = 0; m < R; ++m) x[m][v] = make_uint4(0u, 0u, 0u, 0u);
@@ -183,7 +186,7 @@ __global__ __launch_bounds__(64) void rows_wave_kernel(const asrlayer_linear_par
         float part = 0.f;
 #pragma unroll
         for (int e = 0; e < EPL; ++e) part = fmaf(f[e] - mean, f[e] - mean, part);
-        var += v * 64 + lane < vecs ? part : 0.f;
+        var += v < kFull || v * 64 + lane < vecs ? part : 0.f;
       }
       const float r = rsqrtf(group_sum<64>(var) * inv_k + p.ln_eps);
 #pragma unroll
@@ -195,7 +198,7 @@ __global__ __launch_bounds__(64) void rows_wave_kernel(const asrlayer_linear_par
 #pragma unroll
         for (int e = 0; e < EPL; ++e) f[e] = fmaf((f[e] - mean) * r, g[e], b[e]);
         const uint4 y = pack<T>(f);
-        x[m][v] = v * 64 + lane < vecs ? y : make_uint4(0u, 0u, 0u, 0u);
+        x[m][v] = v < kFull || v * 64 + lane < vecs ? y : make_uint4(0u, 0u, 0u, 0u);
       }
     }
   }
@@ -204,9 +207,15 @@ __global__ __launch_bounds__(64) void rows_wave_kernel(const asrlayer_linear_par
   for (int c = 0; c < kCols; ++c)
 #pragma unroll
     for (int m = 0; m < R; ++m) {
-      float y = dot_vec<T>(x[m][0], w[c][0]);
+      float y = 0.f;
 #pragma unroll
-      for (int v = 1; v < NV; ++v) y += dot_vec<T>(x[m][v], w[c][v]);
+      for (int v = 0; v < NV; ++v) {
+        // Past the row the weights repeat its last vector: 0 times an infinite
+        // one is not 0.
+        float part = dot_vec<T>(x[m][v], w[c][v]);
+        if (v >= kFull) part = v * 64 + lane < vecs ? part : 0.f;
+        y = v == 0 ? part : y + part;
+      }
       acc[c * R + m] = y;
     }
   sum_lanes<kCols * R, 32>(acc, lane);

@@ -290,6 +290,31 @@ def test_rows_linear(device, dtype, rows, inputs, outputs):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,inputs,outputs", [(1, 8, 5), (2, 384, 7), (4, 520, 9), (5, 1280, 6), (3, 3072, 5),
+                                                 (4, 384, 16391), (1, 1280, 16387)])
+def test_rows_linear_infinite_weights(device, dtype, rows, inputs, outputs):
+    """An infinite weight in the first or last vector of its row gives its
+    output the infinity, as the ops do, and touches no other output: reductions
+    that end inside a wave's vectors, at a wave, and past one."""
+    from torch import nn
+
+    from asrback_amd import layers
+
+    say("rows linear inf", dtype, rows, inputs, outputs)
+    torch.manual_seed(12)
+    x = torch.rand(rows, 1, inputs, device=device).add_(0.5).to(dtype)
+    linear = nn.Linear(inputs, outputs, bias=False).to(device, dtype).requires_grad_(False)
+    linear.weight[1, inputs - 1] = float("inf")
+    linear.weight[3, 0] = float("-inf")
+    assert layers.rows_linear_takes(x, [linear], [], [])
+    (got,) = layers.rows_linear(x, [linear])
+    ref = x.double() @ linear.weight.double().t().contiguous()
+    assert bool((got[..., 1] == float("inf")).all()) and bool((got[..., 3] == float("-inf")).all())
+    keep = [0, 2, *range(4, outputs)]
+    assert_close(got[..., keep].cpu(), ref[..., keep].cpu(), KIND[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows,inputs,outputs", [(1, 8, 16384), (1, 1280, 16387), (2, 384, 16389), (2, 1280, 16391),
                                                  (3, 520, 20001), (4, 640, 51865)])
 def test_vocabulary_product(device, dtype, rows, inputs, outputs):
