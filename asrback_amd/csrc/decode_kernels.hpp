@@ -579,7 +579,7 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
       float m[kBatch], l[kBatch], o[kBatch];
 #pragma unroll
       for (int s = 0; s < kBatch; ++s) {
-        const int u = min(s0 + s, a.splits - 1);  // surplus slots repeat the last split, weighted 0
+        const int u = min(s0 + s, a.splits - 1);  // surplus slots repeat the last split
         m[s] = load_shared(a.ws_ml + (idx0 + u) * 2);
         l[s] = load_shared(a.ws_ml + (idx0 + u) * 2 + 1);
         o[s] = load_shared(a.ws_o + (idx0 + u) * HD + d);
@@ -594,9 +594,10 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
       osum *= w0;
 #pragma unroll
       for (int s = 0; s < kBatch; ++s) {
-        const float w = s0 + s < a.splits ? fast_exp2(m[s] - mu) : 0.f;
-        lsum = fmaf(l[s], w, lsum);
-        osum = fmaf(o[s], w, osum);
+        const float w = fast_exp2(m[s] - mu);
+        const bool in = s0 + s < a.splits;  // a surplus slot's weight of 0 would turn an infinite partial into NaN
+        lsum = in ? fmaf(l[s], w, lsum) : lsum;
+        osum = in ? fmaf(o[s], w, osum) : osum;
       }
     }
     T* op = static_cast<T*>(p.out) + (int64_t)b * p.o_batch_stride + (int64_t)hq * p.o_head_stride + d;

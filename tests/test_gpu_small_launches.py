@@ -83,6 +83,28 @@ def test_split_launch_over_any_workspace(ops, device, dtype, hd, heads_q, heads_
         assert torch.equal(held, out)
 
 
+@pytest.mark.parametrize("dtype,hd,heads_q,heads_kv", [
+    (torch.bfloat16, 128, 4, 2), (torch.float32, 64, 3, 3), (torch.bfloat16, 512, 8, 1)])
+@pytest.mark.parametrize("splits", [1, 2, 3, 8, 9, 17, 0])
+def test_split_launch_with_infinite_values(ops, device, dtype, hd, heads_q, heads_kv, splits):
+    """An infinite value of a key that every row sees is the output's infinity
+    however the keys are split: in the last split's keys, which the fold's
+    surplus slots repeat, and in the first's.  All keys alike, so that no
+    weight is 0."""
+    say("infinite values", dtype, hd, heads_q, heads_kv, splits)
+    length = 600
+    q = randn(2, heads_q, hd, seed=1, dtype=dtype).to(device)
+    k = randn(1, 1, heads_kv, hd, seed=2, dtype=dtype).expand(2, length, -1, -1).contiguous().to(device)
+    v = randn(2, length, heads_kv, hd, seed=3, dtype=dtype).to(device)
+    v[:, -1, :, 5] = float("inf")
+    v[:, 0, :, 9] = float("-inf")
+    out = ops.decode(q, k, v, num_splits=splits)
+    assert bool((out[..., 5] == float("inf")).all()) and bool((out[..., 9] == float("-inf")).all())
+    keep = [i for i in range(hd) if i not in (5, 9)]
+    ref = v.double().mean(1).repeat_interleave(heads_q // heads_kv, dim=1)
+    assert_close(out[..., keep].float().cpu(), ref[..., keep].cpu(), KIND[dtype])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("hd,heads_q,heads_kv", [(64, 8, 1), (128, 2, 2), (128, 8, 1), (256, 8, 1), (512, 8, 1)])
 @pytest.mark.parametrize("norms,rotary,v_norm", [(True, True, True), (True, False, False), (False, True, True)])
