@@ -31,9 +31,10 @@ from torch import Tensor, nn
 
 from . import _lib
 from .attention import KeyPrefix, decode, decode_append, decode_supported, flash, local_attention
-from .layers import prompt_rows, prompt_rows_takes, unhooked
+from .layers import computes, prompt_rows, prompt_rows_takes, unhooked
 
 
+@computes
 class RMSNorm(nn.Module):
     """Root-mean-square normalization as Gemma 4 applies it
     (``gemma4.py:166-180``): the statistics in float32, then an optional

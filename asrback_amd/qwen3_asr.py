@@ -38,7 +38,7 @@ from torch import Tensor, nn
 
 from . import attention
 from .attention import KeyPrefix, PageTable, decode, decode_append, greedy_choice, varlen_attn
-from .layers import prompt_rows, prompt_rows_takes
+from .layers import computes, prompt_rows, prompt_rows_takes
 from .transcription import CapturedGraph, to_device
 
 # Positions per row of the KV cache (qwen3_asr.py:57-59).
@@ -100,6 +100,7 @@ class AudioAttention(nn.Module):
         return self.out_proj(attend(q, k, v, segments, causal=False).flatten(1))
 
 
+@computes
 class RMSNorm(nn.Module):
     def __init__(self, width: int, eps: float) -> None:
         super().__init__()

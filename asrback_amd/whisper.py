@@ -105,6 +105,17 @@ class MultiHeadAttention(nn.Module):
         """Self-attention of ``x`` over itself, no mask (the encoder's)."""
         return self.attend(x, *self.project_key_value(x))
 
+    def steps_as_written(self) -> bool:
+        """Whether a decoder step through this module's methods is the one
+        written here (none of them replaced on the module or its class)."""
+        cls, own = type(self), self.__dict__
+        return all(name not in own and getattr(cls, name) is method for name, method in _STEP_METHODS)
+
+
+# The methods a decoder step goes through.
+_STEP_METHODS = tuple((name, getattr(MultiHeadAttention, name))
+                      for name in ("_split_heads", "project_key_value", "step", "attend"))
+
 
 class EncoderLayer(nn.Module):
     """``whisper.py:113-125``."""
@@ -211,6 +222,7 @@ class DecoderLayer(nn.Module):
         own, cross = self.self_attn, self.encoder_attn
         return (
             type(own) is MultiHeadAttention and type(cross) is MultiHeadAttention
+            and own.steps_as_written() and cross.steps_as_written()
             and rows_linear_takes(x, [own.k_proj, own.v_proj, own.q_proj, own.out_proj, cross.q_proj, cross.out_proj,
                                       self.fc1],
                                   [self.self_attn_layer_norm, self.encoder_attn_layer_norm, self.final_layer_norm],

@@ -511,3 +511,55 @@ def test_gemm(device, batch, rows, inputs, outputs):
         assert layers.gemm(x, linear, used, into=into) is into
         assert torch.equal(into[~keep], held[~keep])
         assert_close(into[keep].float().cpu(), (held.double() + ref)[keep].cpu(), "bf16")
+
+
+@pytest.mark.parametrize("where", ["module", "class"])
+@pytest.mark.parametrize("name", ["project_key_value", "step", "attend", "_split_heads"])
+def test_decoder_step_runs_replaced_methods(device, name, where, monkeypatch):
+    """A method of a step's attention replaced on the module or its class takes
+    effect in the decoder layer."""
+    from asrback_amd import whisper
+    from asrback_amd.attention import KeyPrefix
+
+    config = {"d_model": 128, "decoder_attention_heads": 2, "decoder_ffn_dim": 256}
+    layer = whisper.DecoderLayer(config).to(device).requires_grad_(False)
+    x = torch.randn(3, 1, 128, device=device)
+    cache = tuple(torch.randn(3, 2, 16, 64, device=device) for _ in range(4))
+    positions = torch.tensor([0, 4, 15], device=device)
+    mask = KeyPrefix(positions=positions)
+    assert layer._rows_take(x)
+    called = []
+    method = getattr(whisper.MultiHeadAttention, name)
+    if where == "class":
+        monkeypatch.setattr(whisper.MultiHeadAttention, name,
+                            lambda self, *a, **k: called.append(1) or method(self, *a, **k))
+    else:
+        module = layer.encoder_attn if name == "attend" else layer.self_attn
+        monkeypatch.setattr(module, name, lambda *a, **k: called.append(1) or method(module, *a, **k), raising=False)
+    assert not layer._rows_take(x)
+    layer(x, cache, positions, None, mask)
+    assert called
+
+
+def test_replaced_class_forwards_run(device, monkeypatch):
+    """A forward (or call) replaced on a module's class is not passed over by
+    the kernels that compute it."""
+    from torch import nn
+
+    from asrback_amd import gemma4, layers, qwen3_asr
+
+    linear = nn.Linear(64, 64).to(device, torch.bfloat16).requires_grad_(False)
+    x = torch.randn(1, 4, 64, device=device, dtype=torch.bfloat16)
+    assert layers.gemm_takes(x, linear)
+    for cls in (nn.Linear, nn.LayerNorm, nn.Embedding, qwen3_asr.RMSNorm, gemma4.RMSNorm):
+        module = cls(8, 8) if cls in (nn.Linear, nn.Embedding) else cls(8, eps=1e-6)
+        assert layers.unhooked(module)
+        with monkeypatch.context() as patch:
+            patch.setattr(cls, "forward", lambda self, t: t)
+            assert not layers.unhooked(module)
+            if cls is nn.Linear:
+                assert not layers.gemm_takes(x, linear)
+        with monkeypatch.context() as patch:
+            patch.setattr(nn.Module, "__call__", lambda self, *a: a)
+            assert not layers.unhooked(module)
+        assert layers.unhooked(module)
