@@ -113,6 +113,8 @@ def prompt_rows_takes(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache, v_
                 return False
         if positions is None and tokens > k_cache.shape[1]:
             return False
+        if (k_cache.is_inference() or v_cache.is_inference()) and not torch.is_inference_mode_enabled():
+            return False  # the ops refuse the write
         if (k.shape != v.shape or k_cache.shape != v_cache.shape or k_cache.dim() != 4
                 or k_cache.shape[2:] != k.shape[-2:] or k.shape[-1] != head_dim):
             return False
@@ -160,6 +162,8 @@ def prompt_rows(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache: Tensor |
             _DTYPES[q.dtype])
     lib = _lib.load()
     _lib.check(lib.asrlayer_prompt_rows(ctypes.byref(params), _stream(q.device)), "asrlayer_prompt_rows")
+    if k is not None:
+        torch.autograd.graph.increment_version((k_cache, v_cache))
     return q_out, k_out, v_out
 
 

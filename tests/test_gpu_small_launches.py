@@ -225,6 +225,48 @@ def test_prompt_rows_match_the_ops(device, dtype, hd, heads, kv_heads, tokens, p
     assert_close(out, out_ref, "module", 1e-4 if dtype == torch.float32 else 2e-2)
 
 
+def prompt_layer(device, dtype=torch.float32):
+    """A small Qwen3 attention layer and the rest of its prompt pass's
+    arguments past the cache, five tokens of two prompts."""
+    from asrback_amd import qwen3_asr
+
+    config = {"hidden_size": 64, "head_dim": 64, "num_attention_heads": 2, "num_key_value_heads": 1,
+              "rms_norm_eps": 1e-6, "rope_theta": 1e6, "num_hidden_layers": 1}
+    layer = qwen3_asr.TextAttention(config).to(device, dtype).requires_grad_(False)
+    positions = torch.tensor([0, 1, 2, 0, 1], device=device)
+    cos, sin = (t[positions] for t in qwen3_asr.rope_tables(config, 8, device, dtype))
+    rows = torch.tensor([0, 0, 0, 1, 1], device=device)
+    return layer, (rows, positions, qwen3_asr.Segments.from_lengths([3, 2], device), cos, sin)
+
+
+def test_prompt_rows_marks_the_cache_modified(device, monkeypatch):
+    """The cache writes count as in-place writes, as the ops' do: a backward
+    that saved the cache before them is refused, and so is a cache made in
+    inference mode outside it."""
+    from asrback_amd import qwen3_asr
+
+    layer, rest = prompt_layer(device)
+    called = []
+    real = qwen3_asr.prompt_rows
+    monkeypatch.setattr(qwen3_asr, "prompt_rows", lambda *a, **k: called.append(1) or real(*a, **k))
+    x = torch.randn(5, 64, device=device)
+    for which in (0, 1):
+        cache = [torch.zeros(2, 4, 1, 64, device=device) for _ in range(2)]
+        scale = torch.ones((), device=device, requires_grad=True)
+        loss = (cache[which] * scale).sum()
+        layer.prefill(x, *cache, *rest)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            loss.backward()
+    assert len(called) == 2
+    with torch.inference_mode():
+        cache = [torch.zeros(2, 4, 1, 64, device=device) for _ in range(2)]
+        layer.prefill(x, *cache, *rest)
+    assert len(called) == 3
+    with pytest.raises(RuntimeError, match="inference tensor"):
+        layer.prefill(x, *cache, *rest)
+    assert len(called) == 3
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("layer_type", ["sliding_attention", "full_attention"])
 def test_gemma_prompt_rows_match_the_ops(device, dtype, layer_type, monkeypatch):
