@@ -101,7 +101,7 @@ def prompt_rows_takes(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache, v_
         return False
     if cos.shape != sin.shape or cos.stride() != sin.stride() or cos.shape[-2:] != (tokens, head_dim):
         return False
-    if cos.dim() > 3 or (cos.dim() == 3 and cos.shape[0] not in (1, *batch)):
+    if cos.dim() > q.dim() - 1 or (cos.dim() == 3 and cos.shape[0] not in (1, *batch)):
         return False
     if k is not None:
         slots = (math.prod(batch) * tokens if positions is not None else math.prod(batch),)

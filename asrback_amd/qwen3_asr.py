@@ -288,9 +288,9 @@ class TextAttention(nn.Module):
         qkv = self.qkv_proj(x)
         if x.dim() == 2:
             q, k, v = (t.view(shape) for t in qkv.split(self.sizes, dim=-1))
-            (key_cache, pages), (value_cache, _) = _cache_layer(keys), _cache_layer(values)
+            (key_cache, pages), (value_cache, value_pages) = _cache_layer(keys), _cache_layer(values)
             table = None if pages is None else pages.block_table
-            if ((table is None or (table.is_contiguous() and table.device == x.device))
+            if (pages is value_pages and (table is None or (table.is_contiguous() and table.device == x.device))
                     and type(self.q_norm) is RMSNorm and type(self.k_norm) is RMSNorm
                     and prompt_rows_takes(q, k, v, key_cache, value_cache, rows, positions, self.q_norm, self.k_norm,
                                           cos, sin)):

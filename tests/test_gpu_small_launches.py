@@ -267,6 +267,25 @@ def test_prompt_rows_marks_the_cache_modified(device, monkeypatch):
     assert len(called) == 3
 
 
+def test_prompt_rows_leaves_other_forms_to_the_ops(device, monkeypatch):
+    """Rotation tables with a batch axis that packed prompts do not have, which
+    the pass refuses; keys and values paged by different tables."""
+    from asrback_amd import qwen3_asr
+
+    layer, (rows, positions, segments, cos, sin) = prompt_layer(device)
+    x = torch.randn(5, 64, device=device)
+    cache = [torch.zeros(2, 4, 1, 64, device=device) for _ in range(2)]
+    with pytest.raises((RuntimeError, ValueError, IndexError)):
+        layer.prefill(x, *cache, rows, positions, segments, cos[None], sin[None])
+    pools = [torch.zeros(5, 16, 1, 64, device=device) for _ in range(2)]
+    tables = [qwen3_asr.PageTable(torch.tensor(t, dtype=torch.int32, device=device)) for t in ([[0], [1]], [[3], [2]])]
+    layers = [qwen3_asr.PagedLayer(pool, qwen3_asr.PageTable(t.block_table, 16), 16) for pool, t in zip(pools, tables)]
+    layer.prefill(x, *layers, rows, positions, segments, cos, sin)
+    v = layer.qkv_proj(x).split(layer.sizes, dim=-1)[2].view(5, 1, 64)
+    assert torch.equal(pools[1][3, :3], v[:3]) and torch.equal(pools[1][2, :2], v[3:])
+    assert not bool(pools[1][:2].any()) and bool(pools[0][:2, 0].any()) and not bool(pools[0][2:4].any())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("layer_type", ["sliding_attention", "full_attention"])
 def test_gemma_prompt_rows_match_the_ops(device, dtype, layer_type, monkeypatch):
