@@ -207,6 +207,8 @@ def rows_linear(x: Tensor, linears: list[nn.Linear], norm: nn.LayerNorm | None =
     ``gelu`` (exact) after them or, with one matrix, ``residual`` ``(rows, 1,
     outputs)`` of unit last stride added to the result."""
     rows, _, inputs = x.shape
+    if residual is not None and (residual.shape != (rows, 1, linears[0].out_features) or residual.stride(2) != 1):
+        raise ValueError(f"a residual of {tuple(residual.shape)} for {rows} rows of {linears[0].out_features}")
     outs = [torch.empty((rows, 1, m.out_features), dtype=x.dtype, device=x.device) for m in linears]
     params = _lib.LinearParams()
     params.x, params.x_row_stride = x.data_ptr(), x.stride(0)
@@ -322,6 +324,8 @@ def gemm(x: Tensor, linear: nn.Linear, used: Tensor | None = None, into: Tensor 
     are computed; the others hold anything (``into``: what they held)."""
     batch, rows, inputs = x.shape
     outputs = linear.out_features
+    if into is not None and (into.shape != (batch, rows, outputs) or not into.is_contiguous()):
+        raise ValueError(f"{batch} x {rows} rows of {outputs} outputs added to a {tuple(into.shape)} tensor")
     out = into
     if into is None:
         out = torch.empty((batch, rows, outputs), dtype=x.dtype, device=x.device)

@@ -79,7 +79,7 @@ class SANMAttention(nn.Module):
         )
         # linear_out(output) + memory: the bias is in memory already.
         rows = output.view(batch, length, self.size)
-        if project and gemm_takes(rows, self.linear_out):
+        if project and gemm_takes(rows, self.linear_out) and self.linear_out.out_features == self.size:
             return gemm(rows, self.linear_out, skip, into=memory)
         memory.view(-1, self.size).addmm_(output.view(-1, self.size), self.linear_out.weight.t())
         return memory

@@ -227,6 +227,8 @@ class DecoderLayer(nn.Module):
                                       self.fc1],
                                   [self.self_attn_layer_norm, self.encoder_attn_layer_norm, self.final_layer_norm],
                                   [self.fc2])
+            # What is added to x has its width.
+            and own.out_proj.out_features == cross.out_proj.out_features == self.fc2.out_features == x.shape[2]
         )
 
     def _row_step(self, x: Tensor, cache: tuple[Tensor, Tensor, Tensor, Tensor], positions: Tensor) -> Tensor:

@@ -624,3 +624,51 @@ def test_replaced_class_forwards_run(device, monkeypatch):
             patch.setattr(nn.Module, "__call__", lambda self, *a: a)
             assert not layers.unhooked(module)
         assert layers.unhooked(module)
+
+
+def test_layers_of_other_widths_are_refused(device):
+    """An output layer whose width is not that of what it is added to is
+    refused on the host, by the kernels and by the modules (as their ops
+    refuse it)."""
+    from torch import nn
+
+    from asrback_amd import layers, sensevoice, whisper
+    from asrback_amd.attention import KeyPrefix
+
+    x = torch.randn(2, 1, 128, device=device)
+    for outputs in (64, 256):
+        linear = nn.Linear(128, outputs, bias=False).to(device).requires_grad_(False)
+        with pytest.raises(ValueError, match="residual"):
+            layers.rows_linear(x, [linear], residual=x)
+        half = nn.Linear(128, outputs, bias=False).to(device, torch.bfloat16).requires_grad_(False)
+        with pytest.raises(ValueError, match="added to"):
+            layers.gemm(x.bfloat16(), half, into=torch.zeros(2, 1, 128, device=device, dtype=torch.bfloat16))
+
+        config = {"d_model": 128, "decoder_attention_heads": 2, "decoder_ffn_dim": 256}
+        cache = tuple(torch.randn(2, 2, 16, 64, device=device) for _ in range(4))
+        positions = torch.tensor([0, 4], device=device)
+        for module, name, inputs in (("self_attn", "out_proj", 128), ("encoder_attn", "out_proj", 128), (None, "fc2", 256)):
+            layer = whisper.DecoderLayer(config)
+            setattr(layer if module is None else getattr(layer, module), name, nn.Linear(inputs, outputs))
+            layer = layer.to(device).requires_grad_(False)
+            with pytest.raises(RuntimeError):
+                layer(x, cache, positions, None, KeyPrefix(positions=positions))
+        attention = sensevoice.SANMAttention(128, 128, 1, 11)
+        attention.linear_out = nn.Linear(128, outputs, bias=False)
+        attention = attention.to(device, torch.bfloat16).requires_grad_(False)
+        with pytest.raises(RuntimeError):
+            attention(torch.randn(2, 70, 128, device=device, dtype=torch.bfloat16), None, None)
+
+    class Wrapped(nn.Module):  # a layer that is no nn.Linear and has its weight alone
+        def __init__(self, linear):
+            super().__init__()
+            self.weight, self.bias = linear.weight, linear.bias
+
+        def forward(self, t):
+            return nn.functional.linear(t, self.weight, self.bias)
+
+    layer = whisper.DecoderLayer(config).to(device).requires_grad_(False)
+    want = layer(x, tuple(t.clone() for t in cache), positions, None, KeyPrefix(positions=positions))
+    layer.self_attn.out_proj, layer.fc2 = Wrapped(layer.self_attn.out_proj), Wrapped(layer.fc2)
+    got = layer(x, tuple(t.clone() for t in cache), positions, None, KeyPrefix(positions=positions))
+    assert_close(got.cpu(), want.cpu(), "module", 1e-4)
