@@ -220,14 +220,20 @@ struct Stream {
 // At most 128 VGPRs, so that four waves fit per SIMD (two 8-wave workgroups
 // per CU).
 //
-// APPEND: the fused prologue of asrattn_decode_append.  The G query rows, the
-// step's key and its value are normalized and rotated once per workgroup, a
-// lane group each, and shared through LDS (done by every lane group for all
-// rows, the prologue's vector instructions took as long as the memory reads
-// of a small batch: see below); the cache supplies keys 0 .. positions[b] - 1
-// and the new key/value join from LDS (the last split folds them into its
-// state); the first split writes them to the cache at positions[b].  No
-// workgroup reads that slot, so splits need no ordering among themselves.
+// APPEND: the step's key and value join those of the cache, keys 0 ..
+// positions[b] - 1 (the last split folds them into its state); the first
+// split writes them to the cache at positions[b].  No workgroup reads that
+// slot, so splits need no ordering among themselves.
+//
+// PRO: the prologue of asrattn_decode_append.  The G query rows, the step's
+// key and its value are normalized and rotated once per workgroup, a lane
+// group each, and shared through LDS (done by every lane group for all rows,
+// the prologue's vector instructions took as long as the memory reads of a
+// small batch).  Steps without norms and rotation (Whisper's) take the rows
+// from memory, each lane its slices, without the barrier: 16 rows of 12 heads
+// over 440 bf16 keys 7.01 -> 6.54 us, 13 of 20 over 223 6.07 -> 5.62, few
+// float32 rows over 30 keys 3.8 -> 3.5; 0.95 of the time over 528 shapes, and 3%
+// more at 260 to 320 pairs over 440 float32 keys.
 //
 // Splits: each stores its partial, waits until the stores have reached
 // memory, and adds one to its pair's arrival word; the one that finds all
@@ -256,10 +262,12 @@ struct Stream {
 // block-table read and one pair of buffer resources per batch instead of
 // one per slice (Qwen3's paged step 23.6 -> 22.9 us per launch, same box;
 // the same loads in the same order, so the same bits).
-template <typename T, int HD, int G, int W, bool APPEND, bool PAGED, bool SPEC = false, bool PB = false>
+template <typename T, int HD, int G, int W, bool APPEND, bool PAGED, bool SPEC = false, bool PB = false,
+          bool PRO = APPEND>
 __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void decode_kernel(const DecodeArgs a) {
   static_assert(!SPEC || !APPEND, "speculative first batch: plain launches");
   static_assert(!PB || PAGED, "page-sized batches: paged caches");
+  static_assert(!PRO || APPEND, "the prologue belongs to appending launches");
   using S = DecodeShape<T, HD, G, W>;
   constexpr int EPL = S::kEPL, LPK = S::kLPK, NS = S::kStreams;
   // Keys per stream per load batch.
@@ -300,7 +308,7 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
   // too; without the scheduling barrier below, the compiler moves the
   // count's load and its wait above those loads.
   Stream<T, HD, G, W> st;
-  if constexpr (!APPEND) {
+  if constexpr (!PRO) {
     const T* qp = static_cast<const T*>(p.q) + (int64_t)b * p.q_batch_stride +
                   (int64_t)hkv * G * p.q_head_stride + sub * EPL;
 #pragma unroll
@@ -313,32 +321,37 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
   // head r (r < G), the new key (G), the new value (G + 1); lane group
   // `stream` takes rows stream, stream + NS, ... (past the last: the last).
   const asrattn_append_params& ap = a.ap;
-  const bool has_norm = APPEND && ap.q_norm != nullptr;
-  const bool has_vnorm = APPEND && ap.v_norm != 0;
-  const bool has_rot = APPEND && ap.cos != nullptr;
+  const bool has_norm = PRO && ap.q_norm != nullptr;
+  const bool has_vnorm = PRO && ap.v_norm != 0;
+  const bool has_rot = PRO && ap.cos != nullptr;
   constexpr int PR = G + 2;
-  constexpr int kRounds = APPEND ? (PR + NS - 1) / NS : 1;
-  __shared__ uint4 sm_rows[APPEND ? PR : 1][APPEND ? LPK : 1];
-  uint4 praw[kRounds], pw[kRounds], pcs = {}, psn = {};
+  constexpr int kRounds = PRO ? (PR + NS - 1) / NS : 1;
+  __shared__ uint4 sm_rows[PRO ? PR : 1][PRO ? LPK : 1];
+  uint4 praw[kRounds], pw[kRounds], pcs = {}, psn = {}, knew = {}, vnew = {};
   if constexpr (APPEND) {
     const T* knp = static_cast<const T*>(ap.k_new) + (int64_t)b * ap.kn_batch_stride + (int64_t)hkv * ap.kn_head_stride;
     const T* vnp = static_cast<const T*>(ap.v_new) + (int64_t)b * ap.vn_batch_stride + (int64_t)hkv * ap.vn_head_stride;
-    const T* qp = static_cast<const T*>(p.q) + (int64_t)b * p.q_batch_stride + (int64_t)hkv * G * p.q_head_stride;
-    // Absent weights or tables read k_new's slice instead (and are unused):
-    // the loads stay unconditional, so no branch joins their registers and
-    // forces a wait before the first K/V batch.
-    const T* csp = has_rot ? static_cast<const T*>(ap.cos) + (int64_t)b * ap.rope_batch_stride : knp;
-    const T* snp = has_rot ? static_cast<const T*>(ap.sin) + (int64_t)b * ap.rope_batch_stride : knp;
+    if constexpr (!PRO) {
+      knew = *reinterpret_cast<const uint4*>(knp + sub * EPL);
+      vnew = *reinterpret_cast<const uint4*>(vnp + sub * EPL);
+    } else {
+      const T* qp = static_cast<const T*>(p.q) + (int64_t)b * p.q_batch_stride + (int64_t)hkv * G * p.q_head_stride;
+      // Absent weights or tables read k_new's slice instead (and are unused):
+      // the loads stay unconditional, so no branch joins their registers and
+      // forces a wait before the first K/V batch.
+      const T* csp = has_rot ? static_cast<const T*>(ap.cos) + (int64_t)b * ap.rope_batch_stride : knp;
+      const T* snp = has_rot ? static_cast<const T*>(ap.sin) + (int64_t)b * ap.rope_batch_stride : knp;
 #pragma unroll
-    for (int i = 0; i < kRounds; ++i) {
-      const int r = min(stream + i * NS, PR - 1);
-      const T* rp = r < G ? qp + (int64_t)r * p.q_head_stride : r == G ? knp : vnp;
-      const T* wp = !has_norm || r > G ? knp : static_cast<const T*>(r < G ? ap.q_norm : ap.k_norm);
-      praw[i] = *reinterpret_cast<const uint4*>(rp + sub * EPL);
-      pw[i] = *reinterpret_cast<const uint4*>(wp + sub * EPL);
+      for (int i = 0; i < kRounds; ++i) {
+        const int r = min(stream + i * NS, PR - 1);
+        const T* rp = r < G ? qp + (int64_t)r * p.q_head_stride : r == G ? knp : vnp;
+        const T* wp = !has_norm || r > G ? knp : static_cast<const T*>(r < G ? ap.q_norm : ap.k_norm);
+        praw[i] = *reinterpret_cast<const uint4*>(rp + sub * EPL);
+        pw[i] = *reinterpret_cast<const uint4*>(wp + sub * EPL);
+      }
+      pcs = *reinterpret_cast<const uint4*>(csp + sub * EPL);
+      psn = *reinterpret_cast<const uint4*>(snp + sub * EPL);
     }
-    pcs = *reinterpret_cast<const uint4*>(csp + sub * EPL);
-    psn = *reinterpret_cast<const uint4*>(snp + sub * EPL);
   }
 
   // Two register batches in ping-pong: the next batch is in flight while the
@@ -461,7 +474,7 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
   if (split_keys && threadIdx.x == 0 && (arrive_old >> 16) != a.tag)
     __hip_atomic_compare_exchange_strong(arrive, &arrive_old, a.tag << 16, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
-  if constexpr (APPEND) {
+  if constexpr (PRO) {
     __builtin_amdgcn_sched_barrier(0);  // keep the prologue below the batch's issue
 #pragma unroll
     for (int i = 0; i < kRounds; ++i) {
@@ -478,6 +491,8 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
 #pragma unroll
     for (int g = 0; g < G; ++g) st.q[g] = sm_rows[g][sub];
     if (uwave == 0) st.seed(sm_rows[G][sub], sm_rows[G + 1][sub], split == a.splits - 1 && stream == 0);
+  } else if constexpr (APPEND) {
+    if (uwave == 0) st.seed(knew, vnew, split == a.splits - 1 && stream == 0);
   }
   for (int base = k0; base < k1; base += 2 * STEP) {
     mb = load(kb, vb, base + STEP);
@@ -500,8 +515,8 @@ __global__ __launch_bounds__(64 * W, (DecodeShape<T, HD, G, W>::kOcc)) void deco
         voff = (int64_t)page * a.pk.v_page_stride * (int64_t)sizeof(T) + slot * vts;
       }
       if (write) {
-        *reinterpret_cast<uint4*>(const_cast<char*>(kbase) + koff + lane_bytes) = sm_rows[G][sub];
-        *reinterpret_cast<uint4*>(const_cast<char*>(vbase) + voff + lane_bytes) = sm_rows[G + 1][sub];
+        *reinterpret_cast<uint4*>(const_cast<char*>(kbase) + koff + lane_bytes) = PRO ? sm_rows[G][sub] : knew;
+        *reinterpret_cast<uint4*>(const_cast<char*>(vbase) + voff + lane_bytes) = PRO ? sm_rows[G + 1][sub] : vnew;
       }
     }
   }
@@ -624,8 +639,11 @@ hipError_t launch_typed(const DecodeArgs& a, bool append, hipStream_t stream) {
   // steps get it with SPEC).
   const bool page_batch = paged && a.splits == 1 && p.window <= 0 &&
                           a.pk.page_size >= DecodeShape<T, HD, G, W>::kStep;
+  const bool prologue = a.ap.q_norm != nullptr || a.ap.cos != nullptr || a.ap.v_norm != 0;
   if (append && paged && page_batch)
     hipLaunchKernelGGL((decode_kernel<T, HD, G, W, true, true, false, true>), grid, dim3(64 * W), 0, stream, a);
+  else if (append && !paged && !prologue)
+    hipLaunchKernelGGL((decode_kernel<T, HD, G, W, true, false, false, false, false>), grid, dim3(64 * W), 0, stream, a);
   else if (append && paged)
     hipLaunchKernelGGL((decode_kernel<T, HD, G, W, true, true>), grid, dim3(64 * W), 0, stream, a);
   else if (append)

@@ -107,11 +107,12 @@ def test_split_launch_with_infinite_values(ops, device, dtype, hd, heads_q, head
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("hd,heads_q,heads_kv", [(64, 8, 1), (128, 2, 2), (128, 8, 1), (256, 8, 1), (512, 8, 1)])
-@pytest.mark.parametrize("norms,rotary,v_norm", [(True, True, True), (True, False, False), (False, True, True)])
+@pytest.mark.parametrize("norms,rotary,v_norm", [(True, True, True), (True, False, False), (False, True, True),
+                                                 (False, False, False)])
 def test_append_prologue_rows(ops, device, dtype, hd, heads_q, heads_kv, norms, rotary, v_norm):
     """The prologue's rows (query heads, new key, new value) shared by a
-    workgroup: more rows than lane groups, fewer, and each of its parts alone,
-    over split and unsplit launches.  The written key and value bound the
+    workgroup: more rows than lane groups, fewer, each of its parts alone, and
+    none (the rows as they are), over split and unsplit launches.  The written key and value bound the
     prologue's own rounding: one unit in the last place (2^-7 relative in
     bf16, 1e-6 in fp32)."""
     if dtype == torch.float32 and hd == 512:
