@@ -65,7 +65,8 @@ int decode_splits(const asrattn_decode_params& p) {
   // spread over the 256 CUs (192 and more: Whisper-small's 16 x 12, Qwen3's
   // 64 x 8); fewer get their keys split over at most one workgroup per CU (a
   // 257th costs a second round: 96 pairs over 1500 keys 10.0 us with two
-  // splits, 12.5 with three, 11.5 with one).
+  // splits, 12.5 with three, 11.5 with one; 160 pairs 12.6 unsplit, 14.9 with
+  // two).
   const long long pairs = (long long)p.batch * p.heads_kv;
   if (pairs >= 192) return 1;
   long long s = 256 / (pairs < 1 ? 1 : pairs);
@@ -73,7 +74,11 @@ int decode_splits(const asrattn_decode_params& p) {
   // 1024 slots with 480 in use, 8 pairs: 6.4 us with eight splits, 7.4 with
   // four; Whisper-tiny's 256-key bucket: 4.4 unsplit, 5.7 with two).
   const int span = asrattn::decode_span(p);
-  const long long least = 16384 / p.head_dim;
+  // Eight query heads of 64 a kv head are bound by their arithmetic, not by the
+  // reads: half of that from 512 keys on (one such pair within a window of 512:
+  // 13.6 us with two splits, 11.1 with four; 200 keys: 10.0 unsplit, 10.9 with two).
+  const bool heavy = p.head_dim == 64 && p.heads_q / p.heads_kv >= 8 && span >= 512;
+  const long long least = 16384 / p.head_dim / (heavy ? 2 : 1);
   const long long by_len = (span + least - 1) / least;
   if (s > by_len) s = by_len;
   // The fold reads eight splits a round trip: past sixteen splits, longer

@@ -46,7 +46,8 @@ def attend(q, k, v, scale, visible):
 
 @pytest.mark.parametrize("splits", [2, 3, 8, 9, 17, 64, 0])
 @pytest.mark.parametrize("dtype,hd,heads_q,heads_kv", [
-    (torch.bfloat16, 128, 4, 2), (torch.float32, 64, 3, 3), (torch.bfloat16, 512, 8, 1), (torch.float32, 256, 4, 1)])
+    (torch.bfloat16, 128, 4, 2), (torch.float32, 64, 3, 3), (torch.bfloat16, 512, 8, 1), (torch.float32, 256, 4, 1),
+    (torch.bfloat16, 256, 8, 1), (torch.bfloat16, 512, 4, 1), (torch.float32, 64, 8, 1)])
 def test_split_launch_over_any_workspace(ops, device, dtype, hd, heads_q, heads_kv, splits):
     """Split launches need no cleared workspace and leave it usable: over
     buffers of arbitrary bytes, back to back in one buffer, and replayed from
