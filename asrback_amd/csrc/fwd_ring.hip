@@ -635,10 +635,10 @@ hipError_t launch_hd(const FwdArgs& a, hipStream_t stream) {
   if constexpr (HD == 512) {
     // 64 query rows, each row block's dimensions over four waves (eight
     // waves, the whole 160 KB of LDS; 7% faster than two waves per row block).
-    // 32 rows where 64 make at most one workgroup per CU: prompts of 840
-    // tokens, 8 heads, one 53.9 -> 45.5 us, two 54.6 -> 46.5, four (448
-    // workgroups of 64 rows) 82.7 -> 108.
-    if (groups(64) <= 256) {
+    // 32 rows where they still make at most one workgroup per CU (128 KB of LDS:
+    // one is all that fits): prompts of 840 tokens, 8 heads, one (216 workgroups)
+    // 53.9 -> 45.5 us; two (432) 53.9 -> 69.6, six of 300 (480) 26.1 -> 36.7.
+    if (groups(32) <= 256) {
       if (win) return launch_typed<HD, 1, 1, 32, 2, 1, 0, true, 4>(a, stream);
       return launch_typed<HD, 1, 1, 32, 2, 1, 0, false, 4>(a, stream);
     }

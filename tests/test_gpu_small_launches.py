@@ -524,6 +524,24 @@ def test_small_bf16_launches(ops, device, hd, heads, kv_heads, causal, len_q, le
     assert_close(out.float().cpu(), attend(q, k, v, hd**-0.5, visible), "bf16")
 
 
+@pytest.mark.parametrize("hd,window", [(256, 0), (512, 0), (512, 40)])
+@pytest.mark.parametrize("batch,length", [(1, 1), (1, 65), (4, 256), (5, 257), (12, 100)])
+def test_wide_bf16_prompts(ops, device, hd, window, batch, length):
+    """Prompts at head_dim 256 and 512 on both sides of the line between 32 and
+    64 rows a workgroup (256 workgroups of 32 rows), with row ends inside a
+    block and per-row key counts."""
+    say("wide bf16", hd, window, batch, length)
+    q = randn(batch, length, 8, hd, seed=51, dtype=torch.bfloat16)
+    k, v = (randn(batch, length, 4, hd, seed=s, dtype=torch.bfloat16) for s in (52, 53))
+    used = torch.tensor([max(length - 7 * b, 1) for b in range(batch)], dtype=torch.int32)
+    i, j, n = torch.arange(length)[:, None], torch.arange(length), used[:, None, None]
+    visible = ((j < n) & (j <= i)).expand(batch, length, length)
+    if window:
+        visible = visible & (j > i - window)
+    out = ops.flash(q.to(device), k.to(device), v.to(device), causal=1, seqused_k=used.to(device), window=window)
+    assert_close(out.float().cpu(), attend(q, k, v, hd**-0.5, visible), "bf16")
+
+
 @pytest.mark.parametrize("frames,batch", [(65, 1), (100, 1), (300, 2), (504, 1), (130, 9)])
 def test_small_sanm_launches(ops, device, frames, batch):
     """SAN-M attention with its memory in the launches of few utterances: the
