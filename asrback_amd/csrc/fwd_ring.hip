@@ -665,15 +665,19 @@ hipError_t launch_hd(const FwdArgs& a, hipStream_t stream) {
     // 37.0 -> 38.6, x 4 rows 30.1 -> 31.1).  head_dim 128:
     // 4 heads x 300 and 504 rows with the FSMN memory 10.4 -> 9.3 and 13.3 ->
     // 11.2, 16 causal heads x 430 rows 12.3 -> 11.0, 4 x 16 heads x 430 (448
-    // workgroups of 64 rows) 13.8 -> 14.6.  Where one unsplit tile or two hold
-    // all keys, splitting them only adds the merge (16 x 60 keys: 6.3 -> 6.9).
+    // workgroups of 64 rows) 13.8 -> 14.6.  Over few keys the split only adds
+    // the merge: 128 rows of head_dim 64 over 130, 192, 320 and 400 keys 6.6 ->
+    // 7.2, 6.4 -> 7.1, 7.8 -> 8.1 and 9.5 -> 9.4, 64 rows over 192, 256 and 260 6.3
+    // -> 7.0, 6.9 -> 7.1 and 8.1 -> 7.9; head_dim 128 over 60 keys 5.8
+    // -> 6.4, 100 of 128 7.1 -> 7.4, 200 8.4 -> 8.3, but 100 causal ones 7.2 -> 6.7
+    // (half of the rows see half of them).
     if constexpr (HD == 64) {
       if (a.f.memory == nullptr && a.p.max_len_k > 128) {
         if (groups(32) <= 256) return launch_typed<HD, 1, 4, 32, 2, 2, 0>(a, stream);
-        if (groups(64) <= 256) return launch_typed<HD, 2, 4, 32, 2, 2, 0>(a, stream);
-        if (groups(128) <= 256) return launch_typed<HD, 4, 2, 64, 2, 2, 0>(a, stream);
+        if (groups(64) <= 256 && a.p.max_len_k > 256) return launch_typed<HD, 2, 4, 32, 2, 2, 0>(a, stream);
+        if (groups(128) <= 256 && a.p.max_len_k > 384) return launch_typed<HD, 4, 2, 64, 2, 2, 0>(a, stream);
       }
-    } else if (a.p.max_len_k > 64 && groups(64) <= 256) {
+    } else if (a.p.max_len_k > (a.p.causal == ASRATTN_CAUSAL_NONE ? 256 : 64) && groups(64) <= 256) {
       if (a.f.memory != nullptr) return launch_typed<HD, 2, 2, 32, 2, 2, kFsmnFusedKernel>(a, stream);
       return launch_typed<HD, 2, 2, 32, 2, 2, 0>(a, stream);
     }

@@ -507,7 +507,7 @@ def test_float32_wide_heads_and_windows(ops, device, hd, window, causal, len_q, 
 @pytest.mark.parametrize("hd,heads,kv_heads,causal", [(64, 3, 3, 0), (64, 12, 12, 1), (128, 4, 4, 0), (128, 16, 8, 2)])
 @pytest.mark.parametrize("len_q,len_k,batch", [
     (4, 129, 2), (4, 1500, 3), (33, 300, 2), (64, 65, 1), (65, 64, 1), (130, 257, 4), (300, 300, 1), (700, 700, 3),
-    (128, 131, 8)])
+    (128, 131, 8), (200, 300, 4), (200, 256, 4)])
 def test_small_bf16_launches(ops, device, hd, heads, kv_heads, causal, len_q, len_k, batch):
     """bf16 launches around the lines where a workgroup's rows and key splits
     change (32, 64 and 128 rows; one workgroup per CU), with per-row key
