@@ -1,6 +1,6 @@
 // Multi-row attention in fp32 on the gfx950 matrix cores
-// (v_mfma_f32_32x32x2_f32: fp32 operands, fp32 accumulation), head_dim 128, 256
-// and 512; head_dim 64 runs in fwd_f32row.hip.
+// (v_mfma_f32_32x32x2_f32: fp32 operands, fp32 accumulation), head_dim 64 (the
+// launches fwd_f32row.hip leaves to it), 128, 256 and 512.
 //
 // Workgroup: KS waves over one block of 32 query rows of one (sequence,
 // head); wave ks takes the key sub-tiles ks, ks + KS, ... (32 keys each) and
@@ -99,9 +99,11 @@ __global__ __launch_bounds__(64 * KS * DS, OCC) void fwd_f32mm_kernel(const FwdA
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ks = wave % KS;   // key split
-  const int dh = wave / KS;   // dimension split: head dims [dh HD, dh HD + HD)
+  // (Uniform, the compiler schedules DS = 1's loads later: 260 rows of 20 x 16
+  // heads 72.6 -> 75.7 us.)
+  const int wave = DS > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+  const int ks = DS > 1 ? wave % KS : wave;  // key split
+  const int dh = DS > 1 ? wave / KS : 0;     // dimension split: head dims [dh HD, dh HD + HD)
   const int r32 = lane & 31;
   const int half = lane >> 5;
   if (row0 >= len_c) {
@@ -313,7 +315,8 @@ hipError_t launch_hd(const FwdArgs& a, hipStream_t stream) {
   // all blocks (two per SIMD at 64 dimensions a wave; one at 128, where a wave
   // needs more than 256 registers), and at least two sub-tiles per split: a
   // second round of workgroups would run on few CUs.
-  constexpr int kMaxKs = (HD == 64 ? 8 : 4) / DS;
+  // (head_dim 64 comes here with row blocks enough for two.)
+  constexpr int kMaxKs = HD == 64 ? DS > 1 ? 8 / DS : 2 : 4;
   constexpr long long kResidentWaves = HD == 64 ? 2048 : 1024;
   int ks = 1;
   while (ks < kMaxKs && blocks * 2 * ks * DS <= kResidentWaves && subs >= 4 * ks) ks *= 2;
@@ -351,7 +354,9 @@ hipError_t launch_fwd_f32mm(const asrattn_fwd_params& p, hipStream_t stream) {
   a.c = p.scale * kLog2e;
   a.f = FsmnArgs{};
   switch (p.head_dim) {
-    case 64: return launch_fwd_f32row(p, stream);
+    case 64:
+      if (!fwd_f32row_takes(p)) return launch_hd<64, 1, false>(a, stream);
+      return launch_fwd_f32row(p, stream);
     case 128: return launch_window<128, 1>(a, stream);
     case 256: return launch_window<64, 4>(a, stream);
     default: return launch_window<64, 8>(a, stream);

@@ -48,6 +48,7 @@ __device__ __forceinline__ f32x4_t load4(__amdgpu_buffer_rsrc_t rsrc, uint32_t v
 }
 
 constexpr int kHD = 64;
+constexpr int kFewKeys = 512;
 
 // x and its value in lanes l ^ 16, l ^ 32 and l ^ 48 (the lanes of the same
 // query row), folded by `op`.
@@ -289,18 +290,44 @@ hipError_t launch_rb(const FwdArgs& a, hipStream_t stream) {
 
 }  // namespace
 
+// The 32-row kernel (fwd_f32mm.hip) is faster for launches of many row blocks
+// over few keys, where the merge of this one's key splits weighs most: no
+// window, at least 600 row blocks, and keys of two sub-tiles at most (64 rows, 20
+// x 16 heads 13.5 us here, 11.2 there), or at most 512 (200 causal ones, the rows
+// seeing half of them) while its waves -- a row block each, two where 2048 still
+// hold them all -- fill at least 65% of the rounds they take: 260 rows, 12 x 16
+// heads (1728 waves) 53.9 here, 51.0 there, 20 x 16 (2880) 81.5 and 76.8; 8 x 16
+// (1152) 38.3 and 45.5.
+bool fwd_f32row_takes(const asrattn_fwd_params& p) {
+  if (p.window > 0 || p.max_len_k > kFewKeys) return true;
+  const long long blocks = (long long)((p.max_len_q + 31) / 32) * p.heads_q * p.batch;
+  if (blocks < 600) return true;
+  if (p.max_len_k <= 64) return false;
+  if (p.causal != ASRATTN_CAUSAL_NONE && p.max_len_k > 200) return true;
+  const long long waves = blocks <= 1024 ? 2 * blocks : blocks;
+  const long long rounds = (waves + 2047) / 2048;
+  return waves * 100 < rounds * 2048 * 65;
+}
+
 hipError_t launch_fwd_f32row(const asrattn_fwd_params& p, hipStream_t stream) {
   FwdArgs a;
   a.p = p;
   a.c = p.scale * kLog2e;
   a.f = FsmnArgs{};
-  // Rows per workgroup: the fewest 16-row blocks on the fullest CU, with eight
-  // percent for each block less that shares the operands' loads.  us per launch,
-  // 1500 rows and keys, 16 / 32 / 48 rows: 6 heads 51.7 / 59.7 / 49.1, 12 heads
-  // 79.4 / 87.6 / 85.2, 18 heads 107.9 / 113.0 / 123.9, 20 heads 122.5 / 113.1 /
-  // 125.5, 24 heads 136.3 / 139.1 / 125.9, 64 heads 347.6 / 323.3 / 314.8.
+  // Rows per workgroup: the fewest 16-row blocks on the fullest CU, weighted by
+  // what a block costs in workgroups of one, two and three.  Over many keys the
+  // blocks of a workgroup share the operands' loads, eight percent each: us per
+  // launch, 1500 rows and keys, 16 / 32 / 48 rows: 6 heads 51.7 / 59.7 / 49.1, 12
+  // heads 79.4 / 87.6 / 85.2, 18 heads 107.9 / 113.0 / 123.9, 20 heads 122.5 /
+  // 113.1 / 125.5, 24 heads 136.3 / 139.1 / 125.9, 64 heads 347.6 / 323.3 / 314.8.
+  // Over few keys the loads come from the caches, and causal blocks of fewer rows
+  // meet fewer masked keys (300 causal rows, 8 x 2 heads 11.1 / 13.0 / 16.9, 8 x 16
+  // 35.7 / 38.3 / 41.5; 448, 8 x 16 58.1 / 58.2 / 65.2), while unmasked ones pay for
+  // the merge more often (260 rows, 20 x 8 heads 41.9 / 40.4 / 39.0).
+  const bool few = p.max_len_k <= kFewKeys;
+  const int weight1 = !few ? 112 : p.causal != ASRATTN_CAUSAL_NONE ? 84 : 118;
   auto groups = [&](int rb) { return (long long)((p.max_len_q + 16 * rb - 1) / (16 * rb)) * p.heads_q * p.batch; };
-  auto cost = [&](int rb) { return (groups(rb) + 255) / 256 * rb * (112 + 8 * (1 - rb)); };
+  auto cost = [&](int rb) { return (groups(rb) + 255) / 256 * rb * (rb == 1 ? weight1 : rb == 2 ? 104 : 96); };
   int rb = 3;
   if (cost(2) < cost(rb)) rb = 2;
   if (cost(1) < cost(rb)) rb = 1;

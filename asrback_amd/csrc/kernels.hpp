@@ -48,7 +48,8 @@ hipError_t launch_choose(const float* logits, int64_t rows, int64_t vocab, int64
 // 512, K/V spans addressable with 32-bit offsets).
 hipError_t launch_fwd_f32mm(const asrattn_fwd_params& p, hipStream_t stream);
 bool fwd_f32mm_supported(const asrattn_fwd_params& p);
-// Its head_dim 64 (fwd_f32row.hip).
+// Its head_dim 64 (fwd_f32row.hip), and whether that kernel is the faster one.
+bool fwd_f32row_takes(const asrattn_fwd_params& p);
 hipError_t launch_fwd_f32row(const asrattn_fwd_params& p, hipStream_t stream);
 
 // Multi-row forward on the vector ALUs (fp32 or bf16): the fallback for

@@ -504,6 +504,51 @@ def test_float32_wide_heads_and_windows(ops, device, hd, window, causal, len_q, 
     assert_close(out.cpu(), attend(q, k, v, hd**-0.5, visible), "f32")
 
 
+# heads, batch, rows, keys: the workgroups the launch rules take (csrc/fwd_f32row.hip).
+F32_HEAD64 = [
+    (2, 2, 97, 300),    # one 16-row block, eight key splits (28 workgroups)
+    (8, 4, 70, 70),     # one block, four splits
+    (5, 4, 200, 520),   # two blocks (140 workgroups against 260 of one and 100 of three)
+    (8, 4, 150, 150),   # two (160; 320 of one cost more without a mask)
+    (3, 4, 700, 520),   # three (180 workgroups; 264 of two take two rounds)
+    (8, 4, 300, 300),   # three (224; 608 of one cost more without a mask)
+    (20, 16, 40, 40),   # the 32-row kernel: 640 row blocks over two sub-tiles
+    (12, 8, 200, 200),  # the same, two key splits: 1344 waves of 2048
+    (12, 16, 200, 200),  # the same, unsplit: 1344 row blocks
+]
+
+
+@pytest.mark.parametrize("heads,batch,len_q,len_k", F32_HEAD64)
+@pytest.mark.parametrize("form", ["none", "top-left", "bottom-right", "window", "padded"])
+def test_float32_head64_workgroups(ops, device, heads, batch, len_q, len_k, form):
+    """float32 attention at head_dim 64 through each workgroup size and mask,
+    with per-row key counts that end inside a block (and an empty row), and
+    NaN in the keys and values past them."""
+    from asrback_amd import _lib
+
+    say("f32 head_dim 64", heads, batch, len_q, len_k, form)
+    causal = {"none": 0, "padded": 0, "bottom-right": _lib.CAUSAL_BOTTOM_RIGHT}.get(form, _lib.CAUSAL_TOP_LEFT)
+    window = 33 if form == "window" else 0
+    q = randn(batch, len_q, heads, 64, seed=61)
+    k, v = (randn(batch, len_k, heads, 64, seed=s) for s in (62, 63))
+    used = torch.tensor([(len_k, len_k - 9, len_k // 2 + 1, 0, 1)[b % 5] for b in range(batch)], dtype=torch.int32)
+    i, j, n = torch.arange(len_q)[:, None], torch.arange(len_k), used[:, None, None]
+    last = i + (n - len_q if form == "bottom-right" else 0)
+    visible = (j < n).expand(batch, len_q, len_k)
+    if causal:
+        visible = visible & (j <= last)
+    if window:
+        visible = visible & (j > last - window)
+    if form == "padded":
+        visible = visible & (i < n)
+    ref = attend(q, k, v, 0.125, visible)
+    gone = (torch.arange(len_k) >= used[:, None])[..., None, None]
+    k, v = (t.masked_fill(gone, float("nan")) for t in (k, v))
+    out = ops.flash(q.to(device), k.to(device), v.to(device), causal=causal, seqused_k=used.to(device),
+                    window=window, zero_padded_rows=form == "padded")
+    assert_close(out.cpu(), ref, "f32")
+
+
 @pytest.mark.parametrize("hd,heads,kv_heads,causal", [(64, 3, 3, 0), (64, 12, 12, 1), (128, 4, 4, 0), (128, 16, 8, 2)])
 @pytest.mark.parametrize("len_q,len_k,batch", [
     (4, 129, 2), (4, 1500, 3), (33, 300, 2), (64, 65, 1), (65, 64, 1), (130, 257, 4), (300, 300, 1), (700, 700, 3),
