@@ -1,15 +1,15 @@
 // The projections around a module's attention over rows of bf16
 // (asrlayer_gemm): x w^T, plus a bias or added to what the output holds.
 //
-// Two tilings, both on v_mfma_f32_32x32x16_bf16 with the weight rows as the
-// first operand, so that a lane's accumulators are consecutive outputs of one
-// row:
+// Two tilings, on v_mfma_f32_16x16x32_bf16 and v_mfma_f32_32x32x16_bf16, with
+// the weight rows as the first operand, so that a lane's accumulators are
+// consecutive outputs of one row:
 //
-//   * Few rows: a workgroup takes 32 rows x 32 outputs, its four waves a
-//     quarter of the reduction each, operands straight from memory into
-//     registers, eight steps in flight.  A launch is one or two round trips to
-//     memory, which is what bounds it (sixteen in flight in two register sets:
-//     300 rows of 512 to 1536 outputs 7.2 -> 10.3 us).
+//   * Few rows: a workgroup takes 16 or 32 rows x 16 or 32 outputs, each of its
+//     four waves (eight from 768 inputs on) a part of the reduction, operands
+//     straight from memory into registers, all of a wave's steps in flight up to
+//     1280 inputs.  Bound by a round trip to memory and by what a CU loads (64 x 64
+//     tiles in registers: 300 rows of 512 to 1536 outputs 6.6 -> 8.0 us).
 //   * Many rows: 128 rows x 128 or 192 outputs, four waves of 64 rows x half the
 //     outputs, 64-deep tiles of both operands moved into a two-stage LDS ring by
 //     DMA (the attention's ring: chunks rotated within rows, so operand reads
@@ -68,53 +68,73 @@ __device__ __forceinline__ void finish(const asrlayer_gemm_params& p, float* y, 
     *reinterpret_cast<uint2*>(out + n0) = r[0];
 }
 
-// 32 rows x 32 outputs.
-__global__ __launch_bounds__(256) void gemm_small_kernel(const asrlayer_gemm_params p, int row_tiles, int col_tiles) {
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// 16 RT rows x 16 CT outputs on v_mfma_f32_16x16x32_bf16; NW waves share the
+// reduction, kAhead steps of 32 in flight.
+template <int RT, int CT, int NW, int kAhead>
+__global__ __launch_bounds__(64 * NW) void gemm_small_kernel(const asrlayer_gemm_params p, int row_tiles, int col_tiles) {
   const int item = xcd_remap((int)blockIdx.x, (int)gridDim.x);
-  const int n0 = item % col_tiles * 32;
-  const int row0 = item / col_tiles % row_tiles * 32;
+  const int n0 = item % col_tiles * (16 * CT);
+  const int row0 = item / col_tiles % row_tiles * (16 * RT);
   const RowView v = row_view(p, item / col_tiles / row_tiles);
   if (row0 >= v.rows) return;  // uniform over the workgroup
 
-  const int lane = threadIdx.x & 63, r32 = lane & 31, half = lane >> 5;
+  const int lane = threadIdx.x & 63, r16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int quarter = p.k / 4;
-  const bf16_raw* xp = v.x + (int64_t)min(row0 + r32, v.rows - 1) * p.x_row_stride + wave * quarter + half * 8;
-  const bf16_raw* wp = static_cast<const bf16_raw*>(p.w) + (int64_t)min(n0 + r32, p.n - 1) * p.k + wave * quarter + half * 8;
-  const int steps = quarter / 16;
-  constexpr int kAhead = 8;
-  f32x16_t acc = f32x16_t{};
-  for (int s0 = 0; s0 < steps; s0 += kAhead) {
-    bf16x8_t a[kAhead], b[kAhead];
+  const int part = p.k / NW;
+  const int64_t k0 = wave * part + quad * 8;
+  const bf16_raw *xp[RT], *wp[CT];
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-      const int s = min(s0 + i, steps - 1);  // past the last: repeated, unused
-      a[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wp + s * 16));
-      b[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(xp + s * 16));
+  for (int i = 0; i < RT; ++i) xp[i] = v.x + (int64_t)min(row0 + 16 * i + r16, v.rows - 1) * p.x_row_stride + k0;
+#pragma unroll
+  for (int j = 0; j < CT; ++j)
+    wp[j] = static_cast<const bf16_raw*>(p.w) + (int64_t)min(n0 + 16 * j + r16, p.n - 1) * p.k + k0;
+  const int steps = part / 32;
+  f32x4_t acc[RT][CT] = {};
+  for (int s0 = 0; s0 < steps; s0 += kAhead) {
+    bf16x8_t w[kAhead][CT], x[kAhead][RT];
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) {
+      const int s = min(s0 + a, steps - 1);  // past the last: repeated, unused
+#pragma unroll
+      for (int j = 0; j < CT; ++j) w[a][j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wp[j] + s * 32));
+#pragma unroll
+      for (int i = 0; i < RT; ++i) x[a][i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(xp[i] + s * 32));
     }
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i)
-      if (s0 + i < steps) acc = mfma32(a[i], b[i], acc);
-  }
-  // Sum the quarters: accumulator r of a lane is output 8 (r / 4) + 4 half +
-  // r % 4 of row r32.
-  __shared__ float sm[4][32][36];
+    for (int a = 0; a < kAhead; ++a)
+      if (s0 + a < steps) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    *reinterpret_cast<float4*>(&sm[wave][r32][8 * i + 4 * half]) =
-        make_float4(acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]);
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+          for (int j = 0; j < CT; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[a][j], x[a][i], acc[i][j], 0, 0, 0);
+      }
+  }
+  // Sum the waves' parts: accumulator r of a lane is output 16 j + 4 quad + r of
+  // row 16 i + r16.
+  __shared__ float sm[NW][16 * RT][16 * CT + 4];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j)
+      *reinterpret_cast<float4*>(&sm[wave][16 * i + r16][16 * j + 4 * quad]) =
+          make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
   __syncthreads();
-  const int m = threadIdx.x / 8, c = threadIdx.x % 8 * 4;
-  float y[4] = {};
+  for (int t = threadIdx.x; t < 64 * RT * CT; t += 64 * NW) {
+    const int m = t / (4 * CT), c = t % (4 * CT) * 4;
+    float y[4] = {};
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const float4 part = *reinterpret_cast<const float4*>(&sm[w][m][c]);
-    y[0] += part.x;
-    y[1] += part.y;
-    y[2] += part.z;
-    y[3] += part.w;
+    for (int w = 0; w < NW; ++w) {
+      const float4 one = *reinterpret_cast<const float4*>(&sm[w][m][c]);
+      y[0] += one.x;
+      y[1] += one.y;
+      y[2] += one.z;
+      y[3] += one.w;
+    }
+    if (row0 + m < v.rows && n0 + c < p.n) finish<1>(p, y, v.out + (int64_t)(row0 + m) * p.out_row_stride, n0 + c);
   }
-  if (row0 + m < v.rows && n0 + c < p.n) finish<1>(p, y, v.out + (int64_t)(row0 + m) * p.out_row_stride, n0 + c);
 }
 
 // 128 rows x 64 NB outputs.
@@ -243,30 +263,64 @@ __global__ __launch_bounds__(256, 2) void gemm_large_kernel(const asrlayer_gemm_
 
 }  // namespace
 
+namespace {
+
+template <int RT, int CT, int NW, int kAhead>
+hipError_t launch_waves(const asrlayer_gemm_params& p, hipStream_t stream) {
+  const int row_tiles = (p.rows + 16 * RT - 1) / (16 * RT), col_tiles = (p.n + 16 * CT - 1) / (16 * CT);
+  const long long total = (long long)p.batch * row_tiles * col_tiles;
+  if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((gemm_small_kernel<RT, CT, NW, kAhead>), dim3((unsigned)total), dim3(64 * NW), 0, stream, p,
+                     row_tiles, col_tiles);
+  return hipGetLastError();
+}
+
+// The waves a reduction takes, whole steps each, with all of a wave's steps in
+// flight up to 1280.
+template <int RT, int CT>
+hipError_t launch_small(const asrlayer_gemm_params& p, hipStream_t stream) {
+  if (p.k % 128 != 0) return launch_waves<RT, CT, 2, 8>(p, stream);
+  if (p.k <= 512 || p.k % 256 != 0) return launch_waves<RT, CT, 4, 4>(p, stream);
+  if (p.k <= 768) return launch_waves<RT, CT, 8, 3>(p, stream);
+  return launch_waves<RT, CT, 8, 5>(p, stream);
+}
+
+template <int NB>
+hipError_t launch_large(const asrlayer_gemm_params& p, hipStream_t stream) {
+  const int row_tiles = (p.rows + kBM - 1) / kBM, col_tiles = (p.n + 64 * NB - 1) / (64 * NB);
+  const long long total = (long long)p.batch * row_tiles * col_tiles;
+  if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((gemm_large_kernel<NB>), dim3((unsigned)total), dim3(256), 0, stream, p, row_tiles, col_tiles);
+  return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_gemm(const asrlayer_gemm_params& p, hipStream_t stream) {
-  const auto tiles = [](long long count, int size) { return (count + size - 1) / size; };
-  // Small tiles up to four workgroups per CU (300 rows of 512 to 1536 outputs,
-  // 480 of them: 7.2 us against 9.2 in large tiles; 4 x 300 rows, 1920: 18.3
-  // against 9.9).  Counted over all rows as one run, whatever part of them is
-  // computed: the tilings sum in different orders, and a row's result does not
-  // depend on how the batch is padded.
-  const bool small = tiles((long long)p.batch * p.rows, 32) * tiles(p.n, 32) <= 1024;
+  // Counted over all rows as one run, whatever part of them is computed: the
+  // tilings sum in different orders, and at one padded shape a row's result
+  // does not depend on the counts.
+  const auto tiles = [&](int rows, int outputs) {
+    return (((long long)p.batch * p.rows + rows - 1) / rows) * ((p.n + outputs - 1) / outputs);
+  };
+  // The smallest workgroups that make at most one per CU, for these are bound by
+  // what a CU loads (43 bytes a clock); 16 x 16, 32 x 16 and 32 x 32, us: 32 rows
+  // of 768 to 768 outputs 4.2, 4.8, 5.4 (the library's product: 5.2), 128 rows 5.4,
+  // 4.9, 5.5 (5.3), 32 of 1280 5.0, 6.1, 7.2 (5.5).  32 x 32 up to three or four
+  // per CU: 300 rows of 512 to 1536 outputs (480 of them) 6.6 against 8.7 in large
+  // tiles; within SAN-M's layer, whose operands the kernel before has just
+  // written, 500 rows (768) 25.1 and 25.4 a layer, 600 (912) 26.3 and 24.8; added
+  // to 512 outputs, 1200 rows (608) 27.3 and 30.7, 1800 (912) 29.2 and 31.2, 2048
+  // (1024) 25.0 and 23.4.
+  if (tiles(16, 16) <= 256) return launch_small<1, 1>(p, stream);
+  if (tiles(32, 16) <= 256) return launch_small<2, 1>(p, stream);
+  if (tiles(32, 32) <= (p.accumulate ? 1000 : 800)) return launch_small<2, 2>(p, stream);
   // 192 outputs a workgroup where they divide the outputs and leave at least a
   // round of workgroups (two per CU): five operand reads for six products
   // instead of four for four, and fewer rounds (16128 rows to 1536 outputs 45
   // -> 40 us).
-  const bool wide = p.n % 192 == 0 && tiles((long long)p.batch * p.rows, kBM) * (p.n / 192) >= 512;
-  const int row_tiles = (int)tiles(p.rows, small ? 32 : kBM);
-  const int col_tiles = (int)tiles(p.n, small ? 32 : wide ? 192 : 128);
-  const long long total = (long long)p.batch * row_tiles * col_tiles;
-  if (total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  if (small)
-    hipLaunchKernelGGL(gemm_small_kernel, dim3((unsigned)total), dim3(256), 0, stream, p, row_tiles, col_tiles);
-  else if (wide)
-    hipLaunchKernelGGL((gemm_large_kernel<3>), dim3((unsigned)total), dim3(256), 0, stream, p, row_tiles, col_tiles);
-  else
-    hipLaunchKernelGGL((gemm_large_kernel<2>), dim3((unsigned)total), dim3(256), 0, stream, p, row_tiles, col_tiles);
-  return hipGetLastError();
+  const bool wide = p.n % 192 == 0 && tiles(kBM, 192) >= 512;
+  return wide ? launch_large<3>(p, stream) : launch_large<2>(p, stream);
 }
 
 }  // namespace asrattn

@@ -21,6 +21,7 @@ from . import _lib
 from .attention import _DTYPES, _stream
 
 _VECTOR = 16  # bytes per lane access
+_increment_version = torch.autograd.graph.increment_version
 
 
 def _plain(*tensors: Tensor) -> bool:
@@ -68,11 +69,15 @@ def unhooked(*modules: nn.Module) -> bool:
     else: no hooks, and none of it replaced on the module or the class."""
     if _module._global_forward_hooks or _module._global_forward_pre_hooks or nn.Module.__call__ is not _CALL:
         return False
+    seen = None
     for m in modules:
-        cls = type(m)
-        if (m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
-                or cls.forward is not _FORWARDS.get(cls) or cls.__call__ is not _CALL):
+        own, cls = m.__dict__, type(m)
+        if own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own:
             return False
+        if cls is not seen:
+            if cls.forward is not _FORWARDS.get(cls):
+                return False
+            seen = cls
     return True
 
 
@@ -113,7 +118,7 @@ def prompt_rows_takes(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache, v_
                 return False
         if positions is None and tokens > k_cache.shape[1]:
             return False
-        if (k_cache.is_inference() or v_cache.is_inference()) and not torch.is_inference_mode_enabled():
+        if not torch.is_inference_mode_enabled() and (k_cache.is_inference() or v_cache.is_inference()):
             return False  # the ops refuse the write
         if (k.shape != v.shape or k_cache.shape != v_cache.shape or k_cache.dim() != 4
                 or k_cache.shape[2:] != k.shape[-2:] or k.shape[-1] != head_dim):
@@ -163,7 +168,7 @@ def prompt_rows(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache: Tensor |
     lib = _lib.load()
     _lib.check(lib.asrlayer_prompt_rows(ctypes.byref(params), _stream(q.device)), "asrlayer_prompt_rows")
     if k is not None:
-        torch.autograd.graph.increment_version((k_cache, v_cache))
+        _increment_version((k_cache, v_cache))
     return q_out, k_out, v_out
 
 
@@ -303,11 +308,15 @@ def gemm_takes(x: Tensor, linear: nn.Module) -> bool:
             and (bias is None or _vectors(bias)))
 
 
-def gemm_tiles(x: Tensor) -> int:
-    """32 x 32 tiles of a square layer's outputs over ``x`` ``(batch, rows,
-    inputs)``."""
+def gemm_few(x: Tensor) -> bool:
+    """Whether :func:`gemm` of a square layer over ``x`` ``(batch, rows,
+    inputs)`` takes no longer on the GPU than the library's product (and 10 us
+    less of host time): up to 768 inputs, 256 tiles of 32 x 32 outputs (us against
+    the library's: 32 rows of 768 4.2 and 5.2, 300 rows 5.6 and 5.5, 384 8.1 and
+    6.0); longer rows, 256 of 16 x 16 (32 rows of 1280 5.0 and 5.5, 96 6.2 and 5.7)."""
     batch, rows, inputs = x.shape
-    return -(-batch * rows // 32) * (-(-inputs // 32))
+    tile = 32 if inputs <= 768 else 16
+    return -(-batch * rows // tile) * -(-inputs // tile) <= 256
 
 
 def used_takes(used: Tensor, x: Tensor) -> bool:

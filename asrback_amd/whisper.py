@@ -33,7 +33,7 @@ from torch import Tensor, nn
 from . import attention
 from .attention import KeyPrefix, decode_append, greedy_choice, sdpa
 from .layers import (
-    embed_rows, embed_rows_takes, gemm, gemm_takes, gemm_tiles, rows_linear, rows_linear_takes, rows_product,
+    embed_rows, embed_rows_takes, gemm, gemm_few, gemm_takes, rows_linear, rows_linear_takes, rows_product,
     rows_product_takes,
 )
 from .transcription import CapturedGraph, to_device
@@ -41,11 +41,6 @@ from .transcription import CapturedGraph, to_device
 # Key buckets of the graphed decoder step; max_target_positions is the last
 # one (whisper.py:54).
 KV_BUCKETS = (64, 128, 256)
-# 32 x 32 tiles of a prompt's projection up to which attend() runs it on the
-# package's kernel: at most 15 us on the GPU (300 rows of 1280), against 22 of
-# host time for the library's call; past that the library's kernels are the
-# faster ones (512 rows of 1280: 20 us against 11).
-GEMM_TILES = 512
 # Decoder steps between host checks for finished rows (whisper.py:52).
 EOS_CHECK_INTERVAL = 4
 
@@ -93,9 +88,8 @@ class MultiHeadAttention(nn.Module):
         mask: KeyPrefix | Tensor | None = None,
         is_causal: bool = False,
     ) -> Tensor:
-        # Short prompts: the library's products of few rows cost more host time
-        # than the kernel's.
-        few = x.dim() == 3 and gemm_tiles(x) <= GEMM_TILES and gemm_takes(x, self.q_proj)
+        # Short prompts: no slower on the GPU, and less host time.
+        few = x.dim() == 3 and gemm_few(x) and gemm_takes(x, self.q_proj)
         query = self._split_heads(gemm(x, self.q_proj) if few else self.q_proj(x))
         output = sdpa(query, key, value, mask, is_causal)  # (batch, length, heads, head_dim)
         output = output.reshape(x.shape[0], x.shape[1], -1)
@@ -105,16 +99,19 @@ class MultiHeadAttention(nn.Module):
         """Self-attention of ``x`` over itself, no mask (the encoder's)."""
         return self.attend(x, *self.project_key_value(x))
 
-    def steps_as_written(self) -> bool:
-        """Whether a decoder step through this module's methods is the one
-        written here (none of them replaced on the module or its class)."""
-        cls, own = type(self), self.__dict__
-        return all(name not in own and getattr(cls, name) is method for name, method in _STEP_METHODS)
-
 
 # The methods a decoder step goes through.
-_STEP_METHODS = tuple((name, getattr(MultiHeadAttention, name))
-                      for name in ("_split_heads", "project_key_value", "step", "attend"))
+_STEP_METHODS = {name: getattr(MultiHeadAttention, name)
+                 for name in ("_split_heads", "project_key_value", "step", "attend")}
+
+
+def _steps_as_written(*modules: MultiHeadAttention) -> bool:
+    """Whether a decoder step through the modules' methods is the one written
+    here: none of them replaced on a module or on the class."""
+    for name, method in _STEP_METHODS.items():
+        if getattr(MultiHeadAttention, name) is not method:
+            return False
+    return all(_STEP_METHODS.keys().isdisjoint(m.__dict__) for m in modules)
 
 
 class EncoderLayer(nn.Module):
@@ -222,7 +219,7 @@ class DecoderLayer(nn.Module):
         own, cross = self.self_attn, self.encoder_attn
         return (
             type(own) is MultiHeadAttention and type(cross) is MultiHeadAttention
-            and own.steps_as_written() and cross.steps_as_written()
+            and _steps_as_written(own, cross)
             and rows_linear_takes(x, [own.k_proj, own.v_proj, own.q_proj, own.out_proj, cross.q_proj, cross.out_proj,
                                       self.fc1],
                                   [self.self_attn_layer_norm, self.encoder_attn_layer_norm, self.final_layer_norm],

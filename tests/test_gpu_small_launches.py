@@ -609,7 +609,9 @@ def test_small_sanm_launches(ops, device, frames, batch):
 
 @pytest.mark.parametrize("batch,rows,inputs,outputs", [
     (1, 1, 64, 8), (1, 33, 192, 40), (3, 17, 512, 512), (1, 300, 512, 1536), (2, 700, 128, 1000), (5, 504, 512, 1536),
-    (1, 1500, 1280, 136)])
+    (1, 1500, 1280, 136),
+    # 16 x 16 tiles, 32 x 16, and reductions of two, four and eight waves.
+    (1, 32, 1280, 1280), (2, 31, 768, 760), (1, 5, 320, 24), (1, 100, 768, 768), (3, 50, 1024, 1000), (1, 90, 2048, 512)])
 def test_gemm(device, batch, rows, inputs, outputs):
     """The bf16 linear layer over both tilings and their edges (rows, outputs
     and reductions that fill no tile), with and without bias, added to what the
