@@ -172,8 +172,12 @@ def prompt_rows(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache: Tensor |
     return q_out, k_out, v_out
 
 
-# Rows a decoder step's linear layers take (csrc/rows_linear.hip).
-LINEAR_ROWS = 16
+# Rows a decoder step's linear layers take (csrc/rows_linear.hip), and in bf16
+# with a reduction of more than 4096 inputs among them (whole decoder layers
+# against the ops, 64 encoder frames: bf16, width 1280, fc2 of 5120 inputs, 8 rows
+# 66 us and 90, 12 rows 83 and 93, 13 to 16 101 and 85-92; width 1024, 16 rows 62
+# and 81; float32, width 768, 16 rows 52 and 87, 1024, 12 rows 71 and 96).
+LINEAR_ROWS, LONG_LINEAR_ROWS = 16, 12
 
 
 def rows_linear_takes(x: Tensor, linears: list[nn.Module], norms: list[nn.Module], wide: list[nn.Module]) -> bool:
@@ -194,7 +198,7 @@ def rows_linear_takes(x: Tensor, linears: list[nn.Module], norms: list[nn.Module
     for width, layers in ((inputs, linears), (linears[-1].out_features, wide)):
         if not layers:
             continue
-        if width % per or not 0 < width // per <= 1024:
+        if width % per or not 0 < width // per <= 1024 or (per == 8 and width > 4096 and x.shape[0] > LONG_LINEAR_ROWS):
             return False
         for m in layers:
             if m.in_features != width or not m.weight.is_contiguous() or not _vectors(m.weight):
@@ -232,11 +236,13 @@ def rows_linear(x: Tensor, linears: list[nn.Linear], norm: nn.LayerNorm | None =
 
 
 # A vocabulary product (51865 outputs) takes up to two rows, and more of the
-# short ones: float rows of 768, 1: 46.2 -> 30.6 us, 4: 36.0 -> 32.0; of 1280, 1:
-# 72.4 -> 46.5, 4: 53.7 -> 55.9; bf16 rows of 384, 4: 13.2 -> 10.1, of 768, 4:
-# 16.9 -> 17.5.  Float rows' worst error against float64 is 5 times smaller (sums
-# of vectors, then trees).
-PRODUCT_ROWS, PRODUCT_VALUES = 4, 2560
+# short ones: float rows of 768, 1: 46.2 -> 30.6 us, 3: 28.1 -> 25.6, 4: 36.0 ->
+# 32.0; of 1280, 1: 72.4 -> 46.5, 4: 53.7 -> 55.9; bf16 rows of 384, 4: 13.2 ->
+# 10.1, of 512, 4: 13.8 -> 11.5, of 768, 3: 16.5 -> 17.1, of 1280, 2: 23.4 -> 23.2
+# (of 640, a width that no Whisper has, 4: 14.6 -> 16.4).
+# Float rows' worst error against float64 is 5 times smaller (sums of vectors,
+# then trees).
+PRODUCT_ROWS, PRODUCT_VALUES, PRODUCT_INPUTS_BF16 = 4, 2560, 640
 
 
 def rows_product_takes(x: Tensor, weight: Tensor) -> bool:
@@ -245,6 +251,8 @@ def rows_product_takes(x: Tensor, weight: Tensor) -> bool:
     if not _plain(x, weight) or x.dim() != 2 or weight.dim() != 2 or not 1 <= x.shape[0] <= PRODUCT_ROWS:
         return False
     inputs, per = weight.shape[1], _VECTOR // x.element_size()
+    if x.shape[0] > 2 and per == 8 and inputs > PRODUCT_INPUTS_BF16:
+        return False
     return (x.shape[1] == inputs and 0 < x.shape[0] * inputs <= PRODUCT_VALUES and inputs % per == 0
             and inputs // per <= 384 and weight.shape[0] > 0 and _vectors(x) and weight.is_contiguous()
             and _vectors(weight))

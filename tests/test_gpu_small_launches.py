@@ -739,3 +739,51 @@ def test_layers_of_other_widths_are_refused(device):
     layer.self_attn.out_proj, layer.fc2 = Wrapped(layer.self_attn.out_proj), Wrapped(layer.fc2)
     got = layer(x, tuple(t.clone() for t in cache), positions, None, KeyPrefix(positions=positions))
     assert_close(got.cpu(), want.cpu(), "module", 1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width,rows", [(384, 9), (768, 16), (1024, 13), (1280, 12), (1280, 13), (1280, 16)])
+def test_decoder_layer_rows_match_the_ops(device, dtype, width, rows, monkeypatch):
+    """A whole decoder layer's step at nine to sixteen rows through the row
+    kernels against its ops (float32: the same sums in another order; bf16:
+    every activation rounded at the same places), and the lines past which
+    the ops run."""
+    from asrback_amd import whisper
+    from asrback_amd.attention import KeyPrefix
+
+    say("decoder layer", dtype, width, rows)
+    heads = width // 64
+    config = {"d_model": width, "decoder_attention_heads": heads, "decoder_ffn_dim": 4 * width}
+    torch.manual_seed(14)
+    layer = whisper.DecoderLayer(config).to(device, dtype).requires_grad_(False)
+    with torch.no_grad():
+        for name, weight in layer.named_parameters():
+            if "norm" in name:
+                weight.normal_(float("weight" in name), 0.2)
+    x = torch.randn(rows, 1, width, device=device).to(dtype)
+    cache = [torch.randn(rows, heads, n, 64, device=device).to(dtype) for n in (64, 64, 90, 90)]
+    positions = torch.arange(rows, device=device) * 3
+    taken = layer._rows_take(x)
+    # fc2's inputs: at most 1024 vectors of 16 bytes, and bf16 4096 past twelve rows.
+    assert taken == (4 * width <= (4096 if dtype == torch.float32 or rows > 12 else 8192))
+    results = []
+    for fused in (True, False):
+        if not fused:
+            monkeypatch.setattr(whisper, "rows_linear_takes", lambda *a: False)
+        copies = tuple(t.clone() for t in cache)
+        results.append((layer(x, copies, positions, None, KeyPrefix(positions=positions)), *copies[:2]))
+    tolerance = 1e-4 if dtype == torch.float32 else 2e-2
+    for got, want in zip(*results):
+        assert_close(got.float().cpu(), want.float().cpu(), "module", tolerance)
+
+
+def test_vocabulary_product_lines(device):
+    """Rows go to the kernel up to 2560 values, three and four bf16 ones up to
+    640 inputs."""
+    from asrback_amd import layers
+
+    for dtype, rows, inputs, takes in ((torch.bfloat16, 3, 768, False), (torch.bfloat16, 4, 640, True),
+                                       (torch.bfloat16, 2, 1280, True), (torch.float32, 3, 768, True),
+                                       (torch.float32, 4, 768, False), (torch.bfloat16, 5, 384, False)):
+        x, weight = (torch.randn(n, inputs, device=device).to(dtype) for n in (rows, 1000))
+        assert layers.rows_product_takes(x, weight) == takes
