@@ -670,10 +670,11 @@ def workspace(buffer: Tensor):
     """Use ``buffer`` -- caller-owned uint8 device memory -- for the split
     partials of every :func:`decode`, :func:`decode_append` and
     :func:`greedy_choice` call of this thread inside the block that passes
-    no ``workspace`` of its own.  Size it once, at the largest shape the
-    block runs (:func:`decode_workspace_size`,
-    :func:`choice_workspace_size`); a call that needs more raises.  Its
-    address stays fixed, so graphs captured inside the block replay it.
+    no ``workspace`` of its own.  Size it once, for the most that a shape the
+    block runs needs (:func:`decode_workspace_size`,
+    :func:`choice_workspace_size`): the largest batch that splits at all covers
+    the smaller ones.  A call that needs more raises.  Its address stays fixed,
+    so graphs captured inside the block replay it.
     Calls that share one buffer must run in stream order.
 
     Without a buffer, each call that splits takes a temporary from torch's
@@ -710,7 +711,7 @@ def decode_workspace_size(batch: int, heads_q: int, heads_kv: int, head_dim: int
                           dtype: torch.dtype = torch.bfloat16, num_splits: int = 0) -> int:
     """Bytes of split partials a :func:`decode` / :func:`decode_append` call
     of these sizes needs (``asrattn_decode_workspace_size``; 0 when it runs
-    unsplit).  Raises for sizes the library does not take."""
+    unsplit), and with ``num_splits`` 0 any smaller batch's.  Raises for sizes the library does not take."""
     params = _lib.DecodeParams()
     params.batch, params.heads_q, params.heads_kv, params.head_dim = batch, heads_q, heads_kv, head_dim
     params.max_len_k, params.num_splits, params.scale = max_len_k, num_splits, 1.0

@@ -59,6 +59,25 @@ int from_hip(hipError_t err, const char* what) {
   return fail(ASRATTN_ERR_HIP, "%s: %s", what, hipGetErrorString(err));
 }
 
+// The most splits a launch's keys are worth, whatever its batch.
+int key_splits(const asrattn_decode_params& p) {
+  // At least 256 keys of head_dim 64 per split, 128 of 128, and so on (Qwen3's
+  // 1024 slots with 480 in use, 8 pairs: 6.4 us with eight splits, 7.4 with
+  // four; Whisper-tiny's 256-key bucket: 4.4 unsplit, 5.7 with two).
+  const int span = asrattn::decode_span(p);
+  // Eight query heads of 64 a kv head are bound by their arithmetic, not by the
+  // reads: half of that from 512 keys on (one such pair within a window of 512:
+  // 13.6 us with two splits, 11.1 with four; 200 keys: 10.0 unsplit, 10.9 with two).
+  const bool heavy = p.head_dim == 64 && p.heads_q / p.heads_kv >= 8 && span >= 512;
+  const int least = 16384 / p.head_dim / (heavy ? 2 : 1);
+  int s = span / least + (span % least != 0);
+  // The fold reads eight splits a round trip: past sixteen splits, longer
+  // ones (1024 keys).
+  const int most = span / 1024 > 16 ? span / 1024 : 16;
+  if (s > most) s = most;
+  return s > 64 ? 64 : s < 1 ? 1 : s;
+}
+
 int decode_splits(const asrattn_decode_params& p) {
   if (p.num_splits > 0) return p.num_splits;
   // One workgroup per (sequence, kv head) once there are enough of them to
@@ -68,26 +87,10 @@ int decode_splits(const asrattn_decode_params& p) {
   // splits, 12.5 with three, 11.5 with one; 160 pairs 12.6 unsplit, 14.9 with
   // two).
   const long long pairs = (long long)p.batch * p.heads_kv;
-  if (pairs >= 192) return 1;
-  long long s = 256 / (pairs < 1 ? 1 : pairs);
-  // At least 256 keys of head_dim 64 per split, 128 of 128, and so on (Qwen3's
-  // 1024 slots with 480 in use, 8 pairs: 6.4 us with eight splits, 7.4 with
-  // four; Whisper-tiny's 256-key bucket: 4.4 unsplit, 5.7 with two).
-  const int span = asrattn::decode_span(p);
-  // Eight query heads of 64 a kv head are bound by their arithmetic, not by the
-  // reads: half of that from 512 keys on (one such pair within a window of 512:
-  // 13.6 us with two splits, 11.1 with four; 200 keys: 10.0 unsplit, 10.9 with two).
-  const bool heavy = p.head_dim == 64 && p.heads_q / p.heads_kv >= 8 && span >= 512;
-  const long long least = 16384 / p.head_dim / (heavy ? 2 : 1);
-  const long long by_len = (span + least - 1) / least;
-  if (s > by_len) s = by_len;
-  // The fold reads eight splits a round trip: past sixteen splits, longer
-  // ones (1024 keys).
-  const long long most = span / 1024 > 16 ? span / 1024 : 16;
-  if (s > most) s = most;
-  if (s > 64) s = 64;
-  if (s < 1) s = 1;
-  return (int)s;
+  if (pairs > 128) return 1;
+  const int by_pairs = (int)(256 / (pairs < 1 ? 1 : pairs));
+  const int by_keys = key_splits(p);
+  return by_pairs < by_keys ? by_pairs : by_keys;
 }
 
 int check_decode(const asrattn_decode_params* p) {
@@ -116,15 +119,20 @@ struct DecodeWorkspace {
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-DecodeWorkspace decode_workspace(const asrattn_decode_params& p, int splits) {
+// rows: splits times sequences.
+DecodeWorkspace workspace_of(const asrattn_decode_params& p, size_t rows) {
   DecodeWorkspace w{0, 0, 0, 0};
-  if (splits == 1) return w;
-  const size_t rows = (size_t)p.batch * p.heads_q * splits;
+  rows *= p.heads_q;
   w.partials = 0;
   w.stats = align256(rows * (size_t)p.head_dim * sizeof(float));
   w.arrive = w.stats + rows * 2 * sizeof(float);
   w.total = w.stats + align256(rows * 2 * sizeof(float) + (size_t)p.batch * p.heads_kv * sizeof(unsigned long long));
   return w;
+}
+
+DecodeWorkspace decode_workspace(const asrattn_decode_params& p, int splits) {
+  if (splits == 1) return {0, 0, 0, 0};
+  return workspace_of(p, (size_t)p.batch * splits);
 }
 
 }  // namespace
@@ -133,7 +141,13 @@ extern "C" {
 
 size_t asrattn_decode_workspace_size(const asrattn_decode_params* params) {
   if (check_decode(params) != ASRATTN_OK) return (size_t)-1;
-  return decode_workspace(*params, decode_splits(*params)).total;
+  const asrattn_decode_params& p = *params;
+  const int splits = decode_splits(p);
+  if (splits == 1 || p.num_splits > 0) return decode_workspace(p, splits).total;
+  // Every smaller batch's too, which may take more: 256 / pairs splits are
+  // rounded down.
+  const size_t most = 256 / p.heads_kv, all = (size_t)p.batch * key_splits(p);
+  return workspace_of(p, most < all ? most : all).total;
 }
 
 const char* asrattn_last_error(void) { return g_last_error.c_str(); }

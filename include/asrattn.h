@@ -217,7 +217,9 @@ typedef struct asrattn_decode_params {
 } asrattn_decode_params;
 
 /* Bytes of workspace asrattn_decode needs for these parameters (pointers are
- * not read).  Returns 0 for a single split, or (size_t)-1 on invalid params. */
+ * not read), and with num_splits = 0 for every smaller batch of them.  Returns 0
+ * for a single split (which batches of many (sequence, kv head) pairs take and
+ * smaller ones may not), or (size_t)-1 on invalid params. */
 size_t asrattn_decode_workspace_size(const asrattn_decode_params* params);
 
 /* The split count asrattn_decode uses for these parameters. */
@@ -235,8 +237,9 @@ int asrattn_decode(const asrattn_decode_params* params, void* workspace,
  * The split partials go to a static device array of
  * ASRATTN_DECODE_NOALLOC_MAX_BYTES bytes that the library holds on each GPU
  * it runs on until the process ends.  That size covers every split count
- * the library chooses itself (num_splits = 0; at most 6 MiB, head_dim 512
- * with 8 query heads per kv head); parameters whose partials need more
+ * the library chooses itself (num_splits = 0; at most 256 partials a query
+ * head of the group: 4 MiB at head_dim 512 with 8 query heads per kv head);
+ * parameters whose partials need more
  * (asrattn_decode_workspace_size) are rejected with ASRATTN_ERR_WORKSPACE.
  * The array needs no clearing: every launch writes all of the partials it
  * reads.  All calls on one GPU share its array, so calls that may overlap on

@@ -331,6 +331,30 @@ def test_workspace_size_and_split_choice(lib):
     assert lib.asrattn_decode(ctypes.byref(p), None, 0, None) == _lib.ERR_WORKSPACE
 
 
+def test_workspace_covers_smaller_batches(lib):
+    """A workspace sized for a batch holds what every smaller batch of the same
+    heads and cache needs (pairs and splits are whole numbers: 64 pairs take
+    four splits, 100 take two)."""
+    from asrback_amd import _lib
+
+    for heads_q, heads_kv, head_dim, length in ((20, 20, 64, 1500), (16, 8, 128, 1024), (8, 1, 512, 300), (4, 4, 256, 5000)):
+        p = _lib.DecodeParams()
+        p.heads_q, p.heads_kv, p.head_dim, p.max_len_k = heads_q, heads_kv, head_dim, length
+        p.dtype, p.scale = _lib.BF16, 0.125
+        largest = 0
+        for batch in range(1, 200):
+            p.batch, p.num_splits = batch, 0
+            size = lib.asrattn_decode_workspace_size(ctypes.byref(p))
+            splits = lib.asrattn_decode_num_splits(ctypes.byref(p))
+            assert (size == 0) == (splits == 1)
+            assert splits == 1 or batch * heads_kv * splits <= 256
+            p.num_splits = splits
+            need = lib.asrattn_decode_workspace_size(ctypes.byref(p))  # this batch's alone
+            largest = max(largest, need)
+            if size:
+                assert size >= largest
+
+
 def test_choose_workspace_size_and_errors(lib):
     """Qwen3's (64, 151936) logits split each row over 32 workgroups
     (one 16-byte partial each); small vocabularies need no workspace; a
