@@ -481,14 +481,16 @@ def test_rows_linear_leaves_other_programs_to_the_ops(device):
 
 @pytest.mark.parametrize("hd,window,causal", [(64, 33, 1), (128, 100, 2), (256, 0, 0), (256, 40, 1), (512, 0, 1), (512, 64, 2)])
 @pytest.mark.parametrize("len_q,len_k,batch", [(1, 1, 1), (32, 32, 2), (33, 97, 2), (200, 200, 1), (1, 300, 3)])
-def test_float32_wide_heads_and_windows(ops, device, hd, window, causal, len_q, len_k, batch):
+@pytest.mark.parametrize("valu", [False, True])
+def test_float32_wide_heads_and_windows(ops, device, hd, window, causal, len_q, len_k, batch, valu):
     """float32 attention on the matrix cores at head_dim 256 and 512 (a row
-    block's dimensions split over waves) and within sliding windows, around
+    block's dimensions split over waves) and within sliding windows, and on the
+    vector-ALU twin (several lanes a row, keys from the window's start), around
     the 32-row and 32-key edges, with grouped heads and per-row key counts
     (zero keys among them)."""
     from asrback_amd import _lib
 
-    say("f32 wide", hd, window, causal, len_q, len_k, batch)
+    say("f32 wide", hd, window, causal, len_q, len_k, batch, valu)
     q = randn(batch, len_q, 4, hd, seed=21)
     k, v = (randn(batch, len_k, 2, hd, seed=s) for s in (22, 23))
     used = torch.tensor([len_k, len_k // 2, 0][:batch], dtype=torch.int32)
@@ -500,7 +502,7 @@ def test_float32_wide_heads_and_windows(ops, device, hd, window, causal, len_q, 
     if window:
         visible = visible & (j > last - window)
     out = ops.flash(q.to(device), k.to(device), v.to(device), causal=causal, seqused_k=used.to(device),
-                    window=window)
+                    window=window, force_valu=valu)
     assert_close(out.cpu(), attend(q, k, v, hd**-0.5, visible), "f32")
 
 
@@ -605,6 +607,76 @@ def test_small_sanm_launches(ops, device, frames, batch):
     out, memory = ops.flash_fsmn(q, k, v, weight.to(device), seqused_k=used.to(device), zero_padded_rows=True)
     assert_close(out.float().cpu(), ref, "bf16")
     assert_close(memory.float().cpu(), memory_ref, "bf16")
+
+
+@pytest.mark.parametrize("kernel_size", [11, 15])
+@pytest.mark.parametrize("frames,batch", [(70, 3), (300, 2), (504, 9)])
+def test_sanm_reads_nothing_past_a_count(ops, device, frames, batch, kernel_size):
+    """Queries, keys and values of padded frames are NaN (the projection leaves
+    them unwritten): the valid frames come out as over zeros there, bit for bit,
+    and the padded ones finite.  Launches without and with key splits (300
+    frames), of many utterances, and filters past what the attention's launch
+    computes."""
+    say("sanm nan", frames, batch, kernel_size)
+    x = randn(batch, frames, 1536, seed=45, dtype=torch.bfloat16)
+    weight = randn(512, 1, kernel_size, seed=46, dtype=torch.bfloat16).to(device)
+    used = torch.tensor([(frames, frames - 1, frames // 2, 1, 64, 0, frames - 63)[b % 7] for b in range(batch)],
+                        dtype=torch.int32)
+    gone = (torch.arange(frames) >= used[:, None])[..., None]
+    results = []
+    for fill in (0.0, float("nan")):
+        q, k, v = (t.view(batch, frames, 4, 128) for t in x.masked_fill(gone, fill).to(device).split(512, dim=-1))
+        results.append(ops.flash_fsmn(q, k, v, weight, seqused_k=used.to(device), zero_padded_rows=True))
+    for clean, dirty in zip(*results):
+        clean, dirty = (t.reshape(batch, frames, 512) for t in (clean, dirty))
+        assert bool(dirty.isfinite().all()) and torch.equal(clean, dirty)
+
+
+@pytest.mark.parametrize("frames,batch", [(70, 3), (300, 2), (504, 12)])
+def test_sanm_module_over_nan_padding(device, frames, batch):
+    """The bf16 module with NaN in the padded frames of its input: the valid
+    frames as over zeros there, and no NaN in the others."""
+    from asrback_amd import sensevoice
+
+    say("sanm module nan", frames, batch)
+    torch.manual_seed(15)
+    layer = sensevoice.SANMAttention(512, 512, 4, 11).to(device, torch.bfloat16).requires_grad_(False)
+    lengths = torch.tensor([(frames, frames - 1, frames // 2, 1, 64, 0, frames - 63)[b % 7] for b in range(batch)],
+                           dtype=torch.int32, device=device)
+    mask = torch.arange(frames, device=device) < lengths[:, None]
+    x = torch.randn(batch, frames, 512, device=device).bfloat16()
+    clean, dirty = (layer(x.masked_fill(~mask[..., None], fill), mask, lengths) for fill in (0.0, float("nan")))
+    assert bool(dirty.isfinite().all()) and torch.equal(clean[mask], dirty[mask])
+
+
+@pytest.mark.parametrize("batch,rows,inputs", [(1, 8130, 64), (1, 8200, 192), (33, 250, 192), (65, 127, 128)])
+def test_gemm_wide_tiles(device, batch, rows, inputs):
+    """The 128 x 192 tiles of large outputs: 1536 outputs are 8 of 192, and 64 or
+    65 tiles of 128 rows make 512 workgroups and more, the line.  Rows that end
+    inside a tile, and row counts below, at and past 64 and 128 (waves without
+    rows, tiles without any)."""
+    from torch import nn
+
+    from asrback_amd import layers
+
+    say("gemm wide", batch, rows, inputs)
+    assert -(-batch * rows // 128) * (1536 // 192) >= 512
+    torch.manual_seed(16)
+    linear = nn.Linear(inputs, 1536).to(device, torch.bfloat16).requires_grad_(False)
+    x = torch.randn(batch, rows, inputs, device=device).bfloat16()
+    counts = [min(n, rows) for n in (rows, 0, 1, 63, 64, 65, 127, 128, 129, 192, 193, rows - 1)]
+    used = torch.tensor([counts[b % len(counts)] for b in range(batch)], dtype=torch.int32, device=device)
+    keep = torch.arange(rows, device=device) < used[:, None]
+    assert layers.gemm_takes(x, linear)
+    ref = x.double() @ linear.weight.double().t().contiguous()
+    got = layers.gemm(x, linear)
+    assert_close(got.float().cpu(), (ref + linear.bias.double()).cpu(), "bf16")
+    assert torch.equal(layers.gemm(x, linear, used)[keep], got[keep])
+    held = torch.randn(batch, rows, 1536, device=device).bfloat16()
+    into = held.clone()
+    layers.gemm(x, linear, used, into=into)
+    assert torch.equal(into[~keep], held[~keep])
+    assert_close(into[keep].float().cpu(), (held.double() + ref)[keep].cpu(), "bf16")
 
 
 @pytest.mark.parametrize("batch,rows,inputs,outputs", [
