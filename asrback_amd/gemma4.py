@@ -242,18 +242,20 @@ class TextAttention(nn.Module):
         the cache (queries alone on shared layers): one kernel on the tensors
         it takes (:func:`~asrback_amd.layers.prompt_rows`)."""
         projected = (self.q_proj if self.shared else self.qkv_proj)(x)
-        plain = x.dim() == 3 and type(self.q_norm) is RMSNorm and self.q_norm.weight is not None
+        q_norm = self.q_norm
+        plain = x.dim() == 3 and type(q_norm) is RMSNorm and q_norm.weight is not None
         if plain and self.shared:
             q = projected.view(*x.shape[:2], -1, self.head_dim)
-            if prompt_rows_takes(q, None, None, None, None, None, None, self.q_norm, None, cos, sin):
-                return prompt_rows(q, None, None, None, None, None, None, self.q_norm, None, cos, sin)
-        elif plain and type(self.k_norm) is RMSNorm and type(self.v_norm) is RMSNorm:
-            q, k, v = (t.unflatten(-1, (-1, self.head_dim)) for t in projected.split(self.sizes, dim=-1))
-            if (self.k_norm.weight is not None and self.v_norm.weight is None and unhooked(self.v_norm)
-                    and prompt_rows_takes(q, k, v, cache.keys, cache.values, rows, None, self.q_norm, self.k_norm, cos,
-                                          sin)):
-                return prompt_rows(q, k, v, cache.keys, cache.values, rows, None, self.q_norm, self.k_norm, cos, sin,
-                                   v_eps=self.v_norm.eps)
+            if prompt_rows_takes(q, None, None, None, None, None, None, q_norm, None, cos, sin):
+                return prompt_rows(q, None, None, None, None, None, None, q_norm, None, cos, sin)
+        elif plain:
+            k_norm, v_norm = self.k_norm, self.v_norm
+            if (type(k_norm) is RMSNorm and type(v_norm) is RMSNorm and k_norm.weight is not None
+                    and v_norm.weight is None and unhooked(v_norm)):
+                q, k, v = (t.unflatten(-1, (-1, self.head_dim)) for t in projected.split(self.sizes, dim=-1))
+                if prompt_rows_takes(q, k, v, cache.keys, cache.values, rows, None, q_norm, k_norm, cos, sin):
+                    return prompt_rows(q, k, v, cache.keys, cache.values, rows, None, q_norm, k_norm, cos, sin,
+                                       v_eps=v_norm.eps)
         q, k, v = self._norm_rotate(projected, cos, sin)
         if not self.shared:
             cache.keys[rows, : x.shape[1]] = k

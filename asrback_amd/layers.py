@@ -96,13 +96,14 @@ def prompt_rows_takes(q: Tensor, k: Tensor | None, v: Tensor | None, k_cache, v_
     tables ``(batch, tokens, head_dim)`` or ``(tokens, head_dim)``, caches
     ``(rows, length, heads, head_dim)``."""
     norms = [q_norm] if k_norm is None else [q_norm, k_norm]
-    tensors = [q, cos, sin, *(m.weight for m in norms)]
+    weights = [m.weight for m in norms]
+    tensors = [q, cos, sin, *weights]
     if k is not None:
         tensors += [k, v, k_cache, v_cache]
     if not _plain(*tensors) or not unhooked(*norms):
         return False
     *batch, tokens, _, head_dim = q.shape
-    if head_dim not in (64, 128, 256, 512) or any(m.weight.shape != (head_dim,) for m in norms):
+    if head_dim not in (64, 128, 256, 512) or any(w.shape != (head_dim,) for w in weights):
         return False
     if cos.shape != sin.shape or cos.stride() != sin.stride() or cos.shape[-2:] != (tokens, head_dim):
         return False
@@ -184,29 +185,33 @@ def rows_linear_takes(x: Tensor, linears: list[nn.Module], norms: list[nn.Module
     """Whether :func:`rows_linear` takes ``x`` ``(rows, 1, inputs)`` through
     each of ``linears`` and ``norms``, and ``(rows, 1, outputs)`` of the last of
     ``linears`` through each of ``wide``."""
-    modules = [*linears, *norms, *wide]
+    modules = [*linears, *wide, *norms]
     if any(type(m) is not nn.Linear for m in (*linears, *wide)) or any(type(m) is not nn.LayerNorm for m in norms):
         return False
+    held = [(m.weight, m.bias) for m in modules]  # each looked up once
     tensors = [x]
-    for m in modules:
-        tensors += [m.weight] if m.bias is None else [m.weight, m.bias]
+    for weight, bias in held:
+        tensors += [weight] if bias is None else [weight, bias]
     if any(t is None for t in tensors) or not _plain(*tensors) or not unhooked(*modules):
         return False
     if x.dim() != 3 or x.shape[1] != 1 or not 1 <= x.shape[0] <= LINEAR_ROWS or not _vectors(x[:, 0]):
         return False
     inputs, per = x.shape[2], _VECTOR // x.element_size()
-    for width, layers in ((inputs, linears), (linears[-1].out_features, wide)):
+    last = len(linears)
+    if any(weight.dim() != 2 for weight, _ in held[:last + len(wide)]):
+        return False
+    for width, layers in ((inputs, held[:last]), (held[last - 1][0].shape[0], held[last:last + len(wide)])):
         if not layers:
             continue
         if width % per or not 0 < width // per <= 1024 or (per == 8 and width > 4096 and x.shape[0] > LONG_LINEAR_ROWS):
             return False
-        for m in layers:
-            if m.in_features != width or not m.weight.is_contiguous() or not _vectors(m.weight):
+        for weight, bias in layers:
+            if weight.shape[1] != width or not weight.is_contiguous() or not _vectors(weight):
                 return False
-            if m.bias is not None and not m.bias.is_contiguous():
+            if bias is not None and (bias.shape != weight.shape[:1] or not bias.is_contiguous()):
                 return False
-    return all(m.normalized_shape == (inputs,) and m.bias is not None and _vectors(m.weight) and _vectors(m.bias)
-               for m in norms)
+    return all(m.normalized_shape == weight.shape == (inputs,) and bias is not None and bias.shape == weight.shape and _vectors(weight) and _vectors(bias)
+               for m, (weight, bias) in zip(norms, held[last + len(wide):]))
 
 
 def rows_linear(x: Tensor, linears: list[nn.Linear], norm: nn.LayerNorm | None = None, *, gelu: bool = False,
@@ -216,17 +221,19 @@ def rows_linear(x: Tensor, linears: list[nn.Linear], norm: nn.LayerNorm | None =
     ``gelu`` (exact) after them or, with one matrix, ``residual`` ``(rows, 1,
     outputs)`` of unit last stride added to the result."""
     rows, _, inputs = x.shape
-    if residual is not None and (residual.shape != (rows, 1, linears[0].out_features) or residual.stride(2) != 1):
-        raise ValueError(f"a residual of {tuple(residual.shape)} for {rows} rows of {linears[0].out_features}")
-    outs = [torch.empty((rows, 1, m.out_features), dtype=x.dtype, device=x.device) for m in linears]
+    weights = [m.weight for m in linears]
+    outs = [torch.empty((rows, 1, w.shape[0]), dtype=x.dtype, device=x.device) for w in weights]
+    if residual is not None and (residual.shape != outs[0].shape or residual.stride(2) != 1):
+        raise ValueError(f"a residual of {tuple(residual.shape)} for {rows} rows of {outs[0].shape[2]}")
     params = _lib.LinearParams()
     params.x, params.x_row_stride = x.data_ptr(), x.stride(0)
     if norm is not None:
         params.ln_weight, params.ln_bias, params.ln_eps = norm.weight.data_ptr(), norm.bias.data_ptr(), norm.eps
-    for i, (m, out) in enumerate(zip(linears, outs)):
-        params.w[i], params.out[i], params.n[i] = m.weight.data_ptr(), out.data_ptr(), m.out_features
-        if m.bias is not None:
-            params.b[i] = m.bias.data_ptr()
+    for i, (m, weight, out) in enumerate(zip(linears, weights, outs)):
+        params.w[i], params.out[i], params.n[i] = weight.data_ptr(), out.data_ptr(), weight.shape[0]
+        bias = m.bias
+        if bias is not None:
+            params.b[i] = bias.data_ptr()
     if residual is not None:
         params.residual, params.r_row_stride = residual.data_ptr(), residual.stride(0)
     params.rows, params.k, params.act, params.dtype = rows, inputs, int(gelu), _DTYPES[x.dtype]
@@ -307,7 +314,12 @@ def gemm_takes(x: Tensor, linear: nn.Module) -> bool:
     if type(linear) is not nn.Linear or x.dim() != 3 or x.dtype != torch.bfloat16:
         return False
     weight, bias = linear.weight, linear.bias
-    outputs, inputs = weight.shape
+    shape = weight.shape
+    if len(shape) != 2:
+        return False
+    outputs, inputs = shape
+    if bias is not None and bias.numel() != outputs:
+        return False
     if inputs % 64 or outputs % 8 or x.shape[2] != inputs or not unhooked(linear):
         return False
     if not (_plain(x, weight) if bias is None else _plain(x, weight, bias)):
@@ -340,19 +352,21 @@ def gemm(x: Tensor, linear: nn.Linear, used: Tensor | None = None, into: Tensor 
     launch (``asrlayer_gemm``).  ``used`` (int32 per batch entry): the rows that
     are computed; the others hold anything (``into``: what they held)."""
     batch, rows, inputs = x.shape
-    outputs = linear.out_features
+    weight = linear.weight
+    outputs = weight.shape[0]
     if into is not None and (into.shape != (batch, rows, outputs) or not into.is_contiguous()):
-        raise ValueError(f"{batch} x {rows} rows of {outputs} outputs added to a {tuple(into.shape)} tensor")
+        raise RuntimeError(f"{batch} x {rows} rows of {outputs} outputs added to a {tuple(into.shape)} tensor")
     out = into
     if into is None:
         out = torch.empty((batch, rows, outputs), dtype=x.dtype, device=x.device)
-    bias = None if into is not None or linear.bias is None else linear.bias.data_ptr()
+    bias = linear.bias if into is None else None
     x_strides, out_strides = x.stride()[:2], out.stride()[:2]
     if used is None and x_strides[0] == rows * x_strides[1]:
         batch, rows = 1, batch * rows  # one run of rows: fewer part-filled tiles
     params = _lib.GemmParams(
-        x.data_ptr(), linear.weight.data_ptr(), bias, out.data_ptr(), None if used is None else used.data_ptr(),
-        *x_strides, *out_strides, batch, rows, outputs, inputs, into is not None)
+        x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(),
+        None if used is None else used.data_ptr(), *x_strides, *out_strides, batch, rows, outputs, inputs,
+        into is not None)
     lib = _lib.load()
     _lib.check(lib.asrlayer_gemm(ctypes.byref(params), _stream(x.device)), "asrlayer_gemm")
     return out

@@ -290,12 +290,12 @@ class TextAttention(nn.Module):
             q, k, v = (t.view(shape) for t in qkv.split(self.sizes, dim=-1))
             (key_cache, pages), (value_cache, value_pages) = _cache_layer(keys), _cache_layer(values)
             table = None if pages is None else pages.block_table
+            q_norm, k_norm = self.q_norm, self.k_norm
             if (pages is value_pages and (table is None or (table.is_contiguous() and table.device == x.device))
-                    and type(self.q_norm) is RMSNorm and type(self.k_norm) is RMSNorm
-                    and prompt_rows_takes(q, k, v, key_cache, value_cache, rows, positions, self.q_norm, self.k_norm,
-                                          cos, sin)):
-                return prompt_rows(q, k, v, key_cache, value_cache, rows, positions, self.q_norm, self.k_norm, cos,
-                                   sin, block_table=table)
+                    and type(q_norm) is RMSNorm and type(k_norm) is RMSNorm
+                    and prompt_rows_takes(q, k, v, key_cache, value_cache, rows, positions, q_norm, k_norm, cos, sin)):
+                return prompt_rows(q, k, v, key_cache, value_cache, rows, positions, q_norm, k_norm, cos, sin,
+                                   block_table=table)
         q, k, v = self._norm_rotate(qkv, cos, sin)
         keys[rows, positions] = k
         values[rows, positions] = v

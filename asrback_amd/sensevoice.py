@@ -64,8 +64,9 @@ class SANMAttention(nn.Module):
         # its attention adds nothing to its memory: neither is computed where
         # the kernels run the linear layers.
         skip = lengths if self.zero_padded_rows else None
-        project = gemm_takes(x, self.linear_q_k_v) and (skip is None or used_takes(skip, x))
-        qkv = gemm(x, self.linear_q_k_v, skip) if project else self.linear_q_k_v(x)
+        linear_in, linear_out = self.linear_q_k_v, self.linear_out
+        project = gemm_takes(x, linear_in) and (skip is None or used_takes(skip, x))
+        qkv = gemm(x, linear_in, skip) if project else linear_in(x)
         query, key, value = qkv.split(self.size, dim=-1)
         shape = (batch, length, self.heads, self.size // self.heads)
         output, memory = flash_fsmn(
@@ -74,14 +75,14 @@ class SANMAttention(nn.Module):
             value.view(shape),
             self.fsmn_block.weight,
             seqused_k=lengths,
-            bias=self.linear_out.bias,
+            bias=linear_out.bias,
             zero_padded_rows=self.zero_padded_rows and lengths is not None,
         )
         # linear_out(output) + memory: the bias is in memory already.
         rows = output.view(batch, length, self.size)
-        if project and gemm_takes(rows, self.linear_out) and self.linear_out.out_features == self.size:
-            return gemm(rows, self.linear_out, skip, into=memory)
-        memory.view(-1, self.size).addmm_(output.view(-1, self.size), self.linear_out.weight.t())
+        if project and gemm_takes(rows, linear_out):
+            return gemm(rows, linear_out, skip, into=memory)
+        memory.view(-1, self.size).addmm_(output.view(-1, self.size), linear_out.weight.t())
         return memory
 
 

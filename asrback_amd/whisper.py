@@ -89,11 +89,12 @@ class MultiHeadAttention(nn.Module):
         is_causal: bool = False,
     ) -> Tensor:
         # Short prompts: no slower on the GPU, and less host time.
-        few = x.dim() == 3 and gemm_few(x) and gemm_takes(x, self.q_proj)
-        query = self._split_heads(gemm(x, self.q_proj) if few else self.q_proj(x))
+        q_proj, out_proj = self.q_proj, self.out_proj
+        few = x.dim() == 3 and gemm_few(x) and gemm_takes(x, q_proj)
+        query = self._split_heads(gemm(x, q_proj) if few else q_proj(x))
         output = sdpa(query, key, value, mask, is_causal)  # (batch, length, heads, head_dim)
         output = output.reshape(x.shape[0], x.shape[1], -1)
-        return gemm(output, self.out_proj) if few and gemm_takes(output, self.out_proj) else self.out_proj(output)
+        return gemm(output, out_proj) if few and gemm_takes(output, out_proj) else out_proj(output)
 
     def forward(self, x: Tensor) -> Tensor:
         """Self-attention of ``x`` over itself, no mask (the encoder's)."""
@@ -225,7 +226,7 @@ class DecoderLayer(nn.Module):
                                   [self.self_attn_layer_norm, self.encoder_attn_layer_norm, self.final_layer_norm],
                                   [self.fc2])
             # What is added to x has its width.
-            and own.out_proj.out_features == cross.out_proj.out_features == self.fc2.out_features == x.shape[2]
+            and len(own.out_proj.weight) == len(cross.out_proj.weight) == len(self.fc2.weight) == x.shape[2]
         )
 
     def _row_step(self, x: Tensor, cache: tuple[Tensor, Tensor, Tensor, Tensor], positions: Tensor) -> Tensor:

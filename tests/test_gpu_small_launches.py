@@ -780,7 +780,7 @@ def test_layers_of_other_widths_are_refused(device):
         with pytest.raises(ValueError, match="residual"):
             layers.rows_linear(x, [linear], residual=x)
         half = nn.Linear(128, outputs, bias=False).to(device, torch.bfloat16).requires_grad_(False)
-        with pytest.raises(ValueError, match="added to"):
+        with pytest.raises(RuntimeError, match="added to"):
             layers.gemm(x.bfloat16(), half, into=torch.zeros(2, 1, 128, device=device, dtype=torch.bfloat16))
 
         config = {"d_model": 128, "decoder_attention_heads": 2, "decoder_ffn_dim": 256}
@@ -797,6 +797,17 @@ def test_layers_of_other_widths_are_refused(device):
         attention = attention.to(device, torch.bfloat16).requires_grad_(False)
         with pytest.raises(RuntimeError):
             attention(torch.randn(2, 70, 128, device=device, dtype=torch.bfloat16), None, None)
+
+    # The weight's own shape counts, as in F.linear, not what the module was built with.
+    linear = nn.Linear(128, 128).to(device).requires_grad_(False)
+    linear.weight = nn.Parameter(linear.weight[:64].clone(), requires_grad=False)
+    assert not layers.rows_linear_takes(x, [linear], [], [])  # a bias of another length
+    linear.bias = nn.Parameter(linear.bias[:64].clone(), requires_grad=False)
+    assert layers.rows_linear_takes(x, [linear], [], [])
+    (got,) = layers.rows_linear(x, [linear])
+    assert_close(got.cpu(), linear(x).cpu(), "f32")
+    half = linear.to(torch.bfloat16)
+    assert_close(layers.gemm(x.bfloat16(), half).float().cpu(), half(x.bfloat16()).float().cpu(), "bf16")
 
     class Wrapped(nn.Module):  # a layer that is no nn.Linear and has its weight alone
         def __init__(self, linear):
