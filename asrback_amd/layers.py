@@ -210,8 +210,8 @@ def rows_linear_takes(x: Tensor, linears: list[nn.Module], norms: list[nn.Module
                 return False
             if bias is not None and (bias.shape != weight.shape[:1] or not bias.is_contiguous()):
                 return False
-    return all(m.normalized_shape == weight.shape == (inputs,) and bias is not None and bias.shape == weight.shape and _vectors(weight) and _vectors(bias)
-               for m, (weight, bias) in zip(norms, held[last + len(wide):]))
+    return all(m.normalized_shape == weight.shape == (inputs,) and bias is not None and bias.shape == weight.shape
+               and _vectors(weight) and _vectors(bias) for m, (weight, bias) in zip(norms, held[last + len(wide):]))
 
 
 def rows_linear(x: Tensor, linears: list[nn.Linear], norm: nn.LayerNorm | None = None, *, gelu: bool = False,
